@@ -12,6 +12,7 @@ returns, for the whole call).
 """
 
 import math
+import sys
 
 import numpy as np
 import torch
@@ -213,6 +214,8 @@ class _Held:
         self.interp, self.prep = interp, prep
 
     def __del__(self):
+        if sys.is_finalizing():
+            return
         self.prep.arena.buf.free()
         self.interp._pool.free_all()
 
