@@ -349,9 +349,13 @@ int ktir_launch_row_rmw_noalloc(const ktir_rmw_t* d);
  *   acc' = acc * alpha + P @ V_j,  l' = l * alpha + rowsum P
  * with loop-carried f32 m, l (per row) and acc.  One lane = one query block
  * of M rows; lane l runs trips[l] iterations, the K tile of iteration j
- * starts at k_base[l] + j * k_step (V: v_base[l] + j * v_step).  M = N = D = 128, bf16 or f16
- * Q/K/V, MFMA with f32 accumulation; P enters the P @ V product as a
- * hi + lo pair of operand-type values (about 16 significant bits). */
+ * starts at k_base[l] + j * k_step (V: v_base[l] + j * v_step).  M, N and D
+ * are 64 or 128 (any combination), bf16 or f16 Q/K/V, MFMA with f32
+ * accumulation.  M = N = D = 128: P enters the P @ V product as a hi + lo
+ * pair of operand-type values (about 16 significant bits), or as v16_ptr
+ * says below; the other shapes carry P as two f16 or three bf16 terms (22 /
+ * 24 bits), use no f16 copy of V, and need K and V rows less than 2^23
+ * elements apart. */
 typedef struct ktir_attn {
   int64_t lanes, M, N, D;
   uint64_t q_ptr, k_ptr, v_ptr;        /* element 0 of each tensor */
@@ -395,7 +399,9 @@ typedef struct ktir_attn {
    * and kpos0; every lane appears once).  Used in the cases that run P @ V
    * in f16 with scale > 0 and (under a mask) neg = -inf: one group of four
    * wavefronts per lane, the two groups taking turns between MFMA work and
-   * softmax.  Other launches ignore the pairs and run one lane per workgroup. */
+   * softmax.  Launches with M = 64 run a pair per workgroup as well, two
+   * wavefronts per lane.  Other launches ignore the pairs and run one lane per
+   * workgroup. */
   uint64_t pairs;
   int64_t n_pairs;
 } ktir_attn_t;

@@ -1,0 +1,360 @@
+// Fused online-softmax attention loop for tiles of 64 or 128 rows and keys
+// and heads of 64 or 128 columns (other than 128 x 128 x 128, which
+// ktir_attn.hip runs): the KV loop of the reference's attention kernels
+// (notebooks/demo_gen_mlir.py:471-567, examples/triton-ktir/paged_attention.mlir:191-396)
+// as one launch.
+//
+// A workgroup is four wavefronts of 32 query rows each: one lane (simulated
+// core) of 128 rows, or two lanes of 64 rows that read one K/V stream (the
+// host pairs them).  Per KV tile of N keys, as in ktir_attn.hip:
+//   S^T = K Q^T     A = K rows from LDS, B = Q^T in registers, so a query row's
+//                   scores lie in lanes l and l ^ 32;
+//   softmax         row max and sum in the lane and one exchange, P, l and O kept
+//                   relative to a base mr <= m that moves when m passes it by 8;
+//   O^T += V^T P^T  V^T by transposing LDS reads, the keys in the order in which
+//                   a lane's own scores are its P fragment.
+// P stays as exact as the f32 P of the op-by-op loop: it enters P V as two f16
+// terms (22 bits) or three bf16 terms (24 bits) whose exact products the MFMA
+// adds in f32.
+//
+// K and V tiles are double-buffered in LDS: tile j + 1 streams in (buffer_load
+// ... lds, no registers) while tile j is computed, one barrier per tile.  A
+// 64 x 64 x 64 step stages 16 KB for 24 MFMAs and about 300 vector
+// instructions per wavefront and takes 32 KB of LDS, so several workgroups
+// share a CU and one's softmax runs under another's MFMAs.  The vector
+// instructions bound it (the exact split of P takes as many as the
+// exponentials).  Full attention of 16 heads, 2048 x 64, f16, 64 x 64 tiles:
+// 40 us (430 TFLOP/s) against 43.4 ms for the loop's about 450 launches.
+#include <type_traits>
+
+#include "ktir_attn_common.h"
+
+namespace ktir {
+
+// Slot permutation of a tile row's 16-byte chunks: 8 chunks for 128-byte rows
+// (64 columns), 16 for 256-byte rows (128 columns).  Both are XORs of row bits
+// chosen so that 8 rows' same chunk (ds_read_b128 of K) and 4 rows' 32-byte
+// pieces (ds_read_b64_tr_b16 of V) lie in distinct banks.
+template <int D>
+__device__ __forceinline__ int att_swz(int r) {
+  if constexpr (D == 64)
+    return ((r & 1) << 1) ^ ((r & 2) << 1) ^ ((r >> 2) & 1) ^ (((r >> 3) & 1) << 1);
+  else
+    return ((r & 1) ? 4 : 0) ^ ((r & 2) ? 10 : 0) ^ ((r & 4) ? 1 : 0) ^ ((r & 8) ? 8 : 0);
+}
+
+// Wavefront w (uniform, 0..3) copies rows N/4 w .. + N/4 of an N x D tile into
+// LDS in 1 KB blocks of 512 / D rows: lane l fills slot l % (D / 8) of its row.
+template <int N, int D>
+__device__ __forceinline__ void att_stage(const uint16_t* src, int64_t row_stride, uint16_t* lds, int w, int l) {
+  constexpr int CH = D / 8, RB = 512 / D, RW = N / 4;
+  const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(src + (int64_t)(RW * w) * row_stride), (short)0, (int)(((RW - 1) * row_stride + D) * 2), 0x00020000);
+  const int r = l / CH, c = l % CH;
+#pragma unroll
+  for (int i = 0; i < RW / RB; ++i) {
+    // a wavefront's rows start at a multiple of 16, so row % 16 is known here
+    const int x = c ^ att_swz<D>((RB * i + r) & 15);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void*)(lds + D * (RW * w + RB * i)),
+                                             16, (int)((r * row_stride + 8 * x) * 2), (int)(i * RB * row_stride * 2), 0, 0);
+  }
+}
+
+// four values as PARTS terms of the operand type, largest first: t[p] holds
+// (x0, x1) and (x2, x3) packed
+template <bool BF16, int PARTS>
+__device__ __forceinline__ void att_split(const float* x, uint32_t (&t)[PARTS][2]) {
+  float r[4] = {x[0], x[1], x[2], x[3]};
+#pragma unroll
+  for (int p = 0; p < PARTS; ++p) {
+    t[p][0] = cvt2<BF16>(r[0], r[1]);
+    t[p][1] = cvt2<BF16>(r[2], r[3]);
+    if (p + 1 < PARTS) {
+      const f32x2_t a = uncvt2<BF16>(t[p][0]), b = uncvt2<BF16>(t[p][1]);
+      r[0] = __fsub_rn(r[0], a.x);
+      r[1] = __fsub_rn(r[1], a.y);
+      r[2] = __fsub_rn(r[2], b.x);
+      r[3] = __fsub_rn(r[3], b.y);
+    }
+  }
+}
+
+// the packed values of w with 0 in the place of infinities and NaN
+template <bool BF16>
+__device__ __forceinline__ uint32_t att_finite(uint32_t w) {
+  constexpr uint32_t E = BF16 ? 0x7f80u : 0x7c00u;
+  const uint32_t lo = (w & E) == E ? 0u : w & 0xffffu, hi = ((w >> 16) & E) == E ? 0u : w & 0xffff0000u;
+  return lo | hi;
+}
+
+// the smallest f16 in the place of a leading term 0 whose value is positive
+__device__ __forceinline__ void att_lift(const float* p, uint32_t (&t)[2]) {
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    if (p[2 * k] > 0.f && !(t[k] & 0xffffu)) t[k] |= 1u;
+    if (p[2 * k + 1] > 0.f && !(t[k] >> 16)) t[k] |= 0x10000u;
+  }
+}
+
+// The position mask keeps score (row, key) iff ((lo <= kpos - qpos <= hi) != inv).
+template <bool BF16, int M, int N, int D>
+__global__ __launch_bounds__(256, N * D == 64 * 64 ? 3 : 2) void attn_tile(const ktir_attn_t d, int mlo, int mhi, int minv) {
+  constexpr int KT = N / 32, DS = D / 16, DT = D / 32, PARTS = BF16 ? 3 : 2;
+  __shared__ __align__(16) uint16_t K0s[N * D];     // K tiles of even / odd j
+  __shared__ __align__(16) uint16_t K1s[N * D];
+  __shared__ __align__(16) uint16_t V0s[N * D];     // V tiles of even / odd j
+  __shared__ __align__(16) uint16_t V1s[N * D];
+  const int tid = threadIdx.x, l = tid & 63, h = l >> 5, r32 = l & 31;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int32_t* trips = (const int32_t*)d.trips;
+  // the workgroup's lanes: wavefronts 0, 1 run la, wavefronts 2, 3 lb
+  int la, lb;
+  if (M == 64 && d.pairs) {
+    la = uni(((const int32_t*)d.pairs)[2 * blockIdx.x]);
+    lb = uni(((const int32_t*)d.pairs)[2 * blockIdx.x + 1]);
+  } else {
+    la = uni(d.order ? ((const int32_t*)d.order)[blockIdx.x] : (int)blockIdx.x);
+    lb = M == 64 ? -1 : la;
+  }
+  const int ta = la >= 0 ? uni(trips[la]) : 0, tb = lb >= 0 ? uni(trips[lb]) : 0;
+  const int lane = w >> 1 ? lb : la, T = w >> 1 ? tb : ta, Tmax = ta > tb ? ta : tb;
+  const int lk = la >= 0 ? la : lb;                 // whose K/V stream (both share it)
+  if (lk < 0) return;
+  const uint16_t* K = (const uint16_t*)d.k_ptr + uni(((const int64_t*)d.k_base)[lk]);
+  const uint16_t* V = (const uint16_t*)d.v_ptr + uni(((const int64_t*)d.v_base)[lk]);
+  const int row = (M == 64 ? (w & 1) : w) * 32 + r32;   // query row inside the lane's tile
+  uint4 qf[DS];                                     // Q^T fragments: Q[row][16 s + 8 h .. + 8]
+  int64_t qpos = 0;
+  if (T > 0) {
+    const uint16_t* qr = (const uint16_t*)d.q_ptr + uni(((const int64_t*)d.q_base)[lane]) + (int64_t)row * d.q_row + 8 * h;
+#pragma unroll
+    for (int s = 0; s < DS; ++s) qf[s] = *(const uint4*)(qr + 16 * s);
+    qpos = uni(((const int64_t*)d.qpos0)[lane]) + row;
+  }
+  const int64_t kpos00 = uni(((const int64_t*)d.kpos0)[lk]);
+  const bool pos_scale = d.scale > 0.f;
+  const float c1 = __fmul_rn(d.scale, LOG2E);
+  const f32x16_t z16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  f32x16_t o[DT];                                   // O^T tiles: d = 32 dt + 8 g + 4 h + t, row r32
+  float m, mr, lsum;
+  const int k_off = r32 * D, k_x = att_swz<D>(r32 & 15);
+  // V^T fragment: member tj of 16-lane group tg addresses key 4 (tg / 2) + tj / 4
+  // (+ 8) of the 16-key step, columns 16 (tg % 2) + 4 (tj % 4) of a 32-column tile
+  const int tg = l >> 4, tj = l & 15;
+  const int v_row0 = 4 * (tg >> 1) + (tj >> 2);
+  const int v_c = 2 * (tg & 1) + ((tj >> 1) & 1), v_in = 4 * (tj & 1);
+  const int v_b0 = v_row0 * D + v_in, v_x0 = v_c ^ att_swz<D>(v_row0), v_x1 = v_c ^ att_swz<D>(v_row0 + 8);
+
+  auto step = [&](auto inf_v, int j, const uint16_t* Kc, const uint16_t* Vc, uint16_t* Kn,
+                  uint16_t* Vn) __attribute__((always_inline)) {
+    constexpr bool INF_V = decltype(inf_v)::value;
+    if (j + 1 < Tmax) {
+      att_stage<N, D>(K + (int64_t)(j + 1) * d.k_step, d.k_row, Kn, w, l);
+      att_stage<N, D>(V + (int64_t)(j + 1) * d.v_step, d.v_row, Vn, w, l);
+    }
+    if (j < T) {
+      f32x16_t sc[KT];
+#pragma unroll
+      for (int kt = 0; kt < KT; ++kt) sc[kt] = z16;
+#pragma unroll
+      for (int s = 0; s < DS; ++s) {
+        const uint16_t* kp = &Kc[k_off + 8 * ((2 * s + h) ^ k_x)];
+#pragma unroll
+        for (int kt = 0; kt < KT; ++kt) sc[kt] = mfma_at<BF16>(*(const uint4*)(kp + kt * 32 * D), qf[s], sc[kt]);
+      }
+      // lane value (kt, i) is key kt * 32 + 8 (i / 4) + 4 h + i % 4 of row `row`
+      const int dbase = (int)(kpos00 + (int64_t)j * d.kpos_step - qpos);
+      const bool all_keep = !d.causal ||
+          (minv ? (dbase + N - 1 < mlo || dbase > mhi) : (dbase >= mlo && dbase + N - 1 <= mhi));
+      // no masked score in the wavefront and scale > 0: row max of S = scale *
+      // row max of Q K^T, and P = 2^(QK scale log2e - mr log2e)
+      const bool fast = pos_scale && __all(all_keep);
+      if (!fast) {
+#pragma unroll
+        for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) {
+            float s = __fmul_rn(d.scale, sc[kt][i]);
+            if (d.causal) {
+              const int df = dbase + kt * 32 + 8 * (i >> 2) + 4 * h + (i & 3);
+              if ((df >= mlo && df <= mhi) == (bool)minv) s = d.neg;
+            }
+            sc[kt][i] = s;
+          }
+      }
+      float x[KT];
+#pragma unroll
+      for (int kt = 0; kt < KT; ++kt) {
+        x[kt] = sc[kt][0];
+#pragma unroll
+        for (int i = 1; i < 15; i += 2) x[kt] = fmax3_nan(x[kt], sc[kt][i], sc[kt][i + 1]);
+        x[kt] = fmax_nan(x[kt], sc[kt][15]);
+      }
+      float xm = x[0];
+#pragma unroll
+      for (int kt = 1; kt < KT; ++kt) xm = fmax_nan(xm, x[kt]);
+      xm = pair_max(xm);
+      const float mn = fmax_nan(m, fast ? __fmul_rn(d.scale, xm) : xm);
+      const bool up = mn > __fadd_rn(mr, 8.0f);
+      if (__any(up)) {
+        const float al = up ? exp_f(__fsub_rn(mr, mn)) : 1.f;
+#pragma unroll
+        for (int t = 0; t < DT; ++t)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) o[t][i] = __fmul_rn(o[t][i], al);
+        lsum = __fmul_rn(lsum, al);
+        mr = up ? mn : mr;
+      }
+      if (fast) {
+        const float c0 = -__fmul_rn(mr, LOG2E);
+#pragma unroll
+        for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) sc[kt][i] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[kt][i], c1, c0));
+      } else {
+#pragma unroll
+        for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) sc[kt][i] = exp_f(__fsub_rn(sc[kt][i], mr));
+      }
+      float a0 = 0.f, a1 = 0.f, a2 = 0.f, a3 = 0.f;
+#pragma unroll
+      for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+        for (int i = 0; i < 16; i += 4) {
+          a0 = __fadd_rn(a0, sc[kt][i]);
+          a1 = __fadd_rn(a1, sc[kt][i + 1]);
+          a2 = __fadd_rn(a2, sc[kt][i + 2]);
+          a3 = __fadd_rn(a3, sc[kt][i + 3]);
+        }
+      lsum = __fadd_rn(lsum, pair_sum(__fadd_rn(__fadd_rn(a0, a1), __fadd_rn(a2, a3))));
+      m = mn;
+#pragma unroll
+      for (int ks = 0; ks < N / 16; ++ks) {
+        const int kt = ks >> 1, g0 = 2 * (ks & 1);
+        const uint16_t* vt = &Vc[16 * ks * D];
+        float p[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) p[i] = sc[kt][4 * g0 + i];
+        uint32_t t0[PARTS][2], t1[PARTS][2];
+        att_split<BF16, PARTS>(p, t0);
+        att_split<BF16, PARTS>(p + 4, t1);
+        if constexpr (INF_V && !BF16) {
+          // a positive P below f16's range still times an infinite V is infinite
+          att_lift(p, t0[0]);
+          att_lift(p + 4, t1[0]);
+        }
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) {
+          const uint2 lo = ds_tr16(vt + v_b0 + 8 * ((4 * dt) ^ v_x0));
+          const uint2 hi = ds_tr16(vt + v_b0 + 8 * D + 8 * ((4 * dt) ^ v_x1));
+          const uint4 a = make_uint4(lo.x, lo.y, hi.x, hi.y);
+          uint4 af = a;
+          if constexpr (INF_V)
+            af = make_uint4(att_finite<BF16>(a.x), att_finite<BF16>(a.y), att_finite<BF16>(a.z), att_finite<BF16>(a.w));
+#pragma unroll
+          for (int q = PARTS - 1; q >= 0; --q)
+            o[dt] = mfma_at<BF16>(q ? af : a, make_uint4(t0[q][0], t0[q][1], t1[q][0], t1[q][1]), o[dt]);
+        }
+      }
+    }
+    __builtin_amdgcn_s_waitcnt(0);                  // this wavefront's part of tile j + 1 has landed
+    __syncthreads();                                // every wavefront: done with tile j, tile j + 1 whole
+  };
+  auto loop = [&](auto inf_v) __attribute__((always_inline)) {
+#pragma unroll
+    for (int t = 0; t < DT; ++t) o[t] = z16;
+    m = mr = -__builtin_inff();
+    lsum = 0.f;
+    if (Tmax > 0) {
+      att_stage<N, D>(K, d.k_row, K0s, w, l);
+      att_stage<N, D>(V, d.v_row, V0s, w, l);
+    }
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    for (int j = 0; j < Tmax; j += 2) {
+      step(inf_v, j, K0s, V0s, K1s, V1s);
+      if (j + 1 < Tmax) step(inf_v, j + 1, K1s, V1s, K0s, V0s);
+    }
+  };
+  loop(std::false_type{});
+  // An infinite V times the terms of P after the first (0, or of the other
+  // sign) is NaN where P V is infinite.  So a NaN anywhere in the workgroup's
+  // result runs the loop again with only the first term meeting such values.
+  bool nan = false;
+#pragma unroll
+  for (int t = 0; t < DT; ++t)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) nan |= o[t][i] != o[t][i];
+  if (__syncthreads_or(nan)) loop(std::true_type{});
+  if (lane < 0) return;
+  if (T > 0) {
+    // bring P, l and O from mr to m
+    const float fin = exp_f(__fsub_rn(mr, m));
+    if (!__all(fin == 1.f)) {
+#pragma unroll
+      for (int t = 0; t < DT; ++t)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[t][i] = __fmul_rn(o[t][i], fin);
+      lsum = __fmul_rn(lsum, fin);
+    }
+  }
+  if (h == 0) {
+    ((float*)d.m_out)[(int64_t)lane * M + row] = m;
+    ((float*)d.l_out)[(int64_t)lane * M + row] = lsum;
+  }
+  if (d.acc_out) {
+    float* orow = (float*)d.acc_out + ((int64_t)lane * M + row) * D + 4 * h;
+#pragma unroll
+    for (int t = 0; t < DT; ++t)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        *(float4*)(orow + 32 * t + 8 * g) = make_float4(o[t][4 * g], o[t][4 * g + 1], o[t][4 * g + 2], o[t][4 * g + 3]);
+  }
+  if (d.o_ptr) {
+    // O = acc / l (f32, correctly rounded), then rounded to the output type
+    const int64_t ob = uni(((const int64_t*)d.o_base)[lane]) + (int64_t)row * d.o_row + 4 * h;
+#pragma unroll
+    for (int t = 0; t < DT; ++t)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const float q0 = __fdiv_rn(o[t][4 * g], lsum), q1 = __fdiv_rn(o[t][4 * g + 1], lsum);
+        const float q2 = __fdiv_rn(o[t][4 * g + 2], lsum), q3 = __fdiv_rn(o[t][4 * g + 3], lsum);
+        const int64_t e = ob + 32 * t + 8 * g;
+        if (d.o_dtype == KTIR_F32)
+          *(float4*)((float*)d.o_ptr + e) = make_float4(q0, q1, q2, q3);
+        else if (d.o_dtype == KTIR_BF16)
+          *(uint2*)((uint16_t*)d.o_ptr + e) = make_uint2(cvt2<true>(q0, q1), cvt2<true>(q2, q3));
+        else
+          *(uint2*)((uint16_t*)d.o_ptr + e) = make_uint2(cvt2<false>(q0, q1), cvt2<false>(q2, q3));
+      }
+  }
+}
+
+bool attn_tile_shape(int64_t M, int64_t N, int64_t D) {
+  return (M == 64 || M == 128) && (N == 64 || N == 128) && (D == 64 || D == 128) && !(M == 128 && N == 128 && D == 128);
+}
+
+// `lo`, `hi`, `inv`: the mask predicate as a range test on kpos - qpos
+void launch_attn_tile(const ktir_attn_t& d, int lo, int hi, int inv) {
+  const bool paired = d.M == 64 && d.pairs && d.n_pairs > 0;
+  const dim3 grid((unsigned)(paired ? d.n_pairs : d.lanes));
+  ktir_attn_t a = d;
+  if (!paired) a.pairs = 0;
+  auto go = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(256), 0, stream(), a, lo, hi, inv); };
+  auto by_type = [&](auto f16, auto bf16) {
+    if (d.dtype == KTIR_BF16) go(bf16);
+    else go(f16);
+  };
+  switch ((d.M == 128) * 4 + (d.N == 128) * 2 + (d.D == 128)) {
+    case 0: by_type(attn_tile<false, 64, 64, 64>, attn_tile<true, 64, 64, 64>); break;
+    case 1: by_type(attn_tile<false, 64, 64, 128>, attn_tile<true, 64, 64, 128>); break;
+    case 2: by_type(attn_tile<false, 64, 128, 64>, attn_tile<true, 64, 128, 64>); break;
+    case 3: by_type(attn_tile<false, 64, 128, 128>, attn_tile<true, 64, 128, 128>); break;
+    case 4: by_type(attn_tile<false, 128, 64, 64>, attn_tile<true, 128, 64, 64>); break;
+    case 5: by_type(attn_tile<false, 128, 64, 128>, attn_tile<true, 128, 64, 128>); break;
+    default: by_type(attn_tile<false, 128, 128, 64>, attn_tile<true, 128, 128, 64>); break;
+  }
+}
+
+}  // namespace ktir

@@ -813,10 +813,14 @@ def _attention_loop(ex, op, lb, st, trips, inits):
             and qe.args[0].attr.offsets is None):
         return None
     q_leaf = qe.args[0].attr
-    AT = 128
-    if tuple(q.shape) != (AT, AT) or len(q_leaf.strides) < 2 or q_leaf.strides[-1] != 1 \
-            or any(s != 0 for s in q_leaf.strides[:-2]):
+    # tiles of 64 or 128 rows, keys and columns: the MFMA kernels' shapes (a
+    # wavefront owns 32 rows).  Others, and operands that are not aligned,
+    # run op by op: 43 ms against 40 us for 16 heads of 2048 x 64, f16.
+    if len(q.shape) != 2 or any(s not in (64, 128) for s in q.shape) or len(q_leaf.strides) < 2 \
+            or q_leaf.strides[-1] != 1 or any(s != 0 for s in q_leaf.strides[:-2]):
         return None
+    M, D = (int(s) for s in q.shape)
+    N = None
     dtype = q_leaf.dtype
     # K and V tiles: base offsets at iteration 0, uniform step, in bounds for every iteration run
     tiles = {}
@@ -836,26 +840,31 @@ def _attention_loop(ex, op, lb, st, trips, inits):
             return None
         ext = tuple(a0.cs.extent)
         big = [i for i, e in enumerate(ext) if e != 1]
-        if len(big) != 2 or ext[big[0]] != AT or ext[big[1]] != AT or v.strides[big[1]] != 1:
+        if len(big) != 2 or ext[big[0]] not in (64, 128) or ext[big[0]] != (N or ext[big[0]]) or ext[big[1]] != D \
+                or v.strides[big[1]] != 1:
             return None
+        N = int(ext[big[0]])
         lo_off = sum(int(l) * int(s) for l, s in zip(a0.cs.lo, v.strides))
         spec, alloc, rel = ex._hbm_leaf(v, a0.origin + lo_off, ext, v.strides)
         row, step = int(v.strides[big[0]]), int(d.flat[0])
         run = trips > 0
         lo = rel + np.minimum(0, tm1 * step)
-        hi = rel + np.maximum(0, tm1 * step) + (AT - 1) * row + AT - 1
-        if np.any(run & ((lo < 0) | (hi >= alloc.n_elems) | (rel % 8 != 0))) or row % 8 or step % 8 or row < AT:
+        hi = rel + np.maximum(0, tm1 * step) + (N - 1) * row + D - 1
+        if np.any(run & ((lo < 0) | (hi >= alloc.n_elems) | (rel % 8 != 0))) or row % 8 or step % 8 or row < D \
+                or row >= 1 << 23:
             return None
         tiles[key] = (alloc, rel, row, step)
     q_off = q_leaf.lane.values(L)
     q_row = int(q_leaf.strides[-2])
     run = trips > 0
-    if np.any(run & ((q_off < q_leaf.lo) | (q_off + (AT - 1) * q_row + AT - 1 >= q_leaf.hi) | (q_off % 8 != 0))) \
-            or q_row % 8 or q_row < AT:
+    if np.any(run & ((q_off < q_leaf.lo) | (q_off + (M - 1) * q_row + D - 1 >= q_leaf.hi) | (q_off % 8 != 0))) \
+            or q_row % 8 or q_row < D:
         return None
+    # 128 x 128 x 128 tiles run the two-group kernel, whose P @ V is in f16
+    full = M == N == D == 128
     # launch
     d = rt.ATTN()
-    d.lanes, d.M, d.N, d.D = L, AT, AT, AT
+    d.lanes, d.M, d.N, d.D = L, M, N, D
     keep = []
 
     def up(arr):
@@ -870,17 +879,17 @@ def _attention_loop(ex, op, lb, st, trips, inits):
     d.q_row, d.k_row, d.v_row = q_row, tiles["k"][2], tiles["v"][2]
     d.k_step, d.v_step = tiles["k"][3], tiles["v"][3]
     d.trips = up(trips.astype(np.int32))
-    if dtype == "bf16":
+    if dtype == "bf16" and full:
         # f16 copy of the V elements the loop reads (the kernel runs P @ V in
         # f16 when every one converts exactly), when that range is no larger
         # than the reads themselves
         _, vrel, vrow, vstep = tiles["v"]
         run = trips > 0
         vlo = vrel + np.minimum(0, tm1 * vstep)
-        vhi = vrel + np.maximum(0, tm1 * vstep) + (AT - 1) * vrow + AT
+        vhi = vrel + np.maximum(0, tm1 * vstep) + (N - 1) * vrow + D
         if np.any(run):
             lo_, hi_ = int(vlo[run].min()), int(vhi[run].max())
-            if 0 < hi_ - lo_ <= int(trips[run].sum()) * AT * AT:
+            if 0 < hi_ - lo_ <= int(trips[run].sum()) * N * D:
                 v16 = ex.pool.temp((hi_ - lo_) * 2)
                 flag = ex.pool.temp(4)
                 keep += [v16, flag]
@@ -899,25 +908,25 @@ def _attention_loop(ex, op, lb, st, trips, inits):
     d.causal = 1 if mask_op is not None else 0
     d.pred = rt.K["KTIR_CMP_" + pred]
     d.dtype = rt.DTYPE_CODE[dtype]
-    m_buf = ex.pool.temp(L * AT * 4)
-    l_buf = ex.pool.temp(L * AT * 4)
-    a_buf = ex.pool.temp(L * AT * AT * 4)
+    m_buf = ex.pool.temp(L * M * 4)
+    l_buf = ex.pool.temp(L * M * 4)
+    a_buf = ex.pool.temp(L * M * D * 4)
     d.m_out, d.l_out, d.acc_out = m_buf.ptr, l_buf.ptr, a_buf.ptr
     keep += [m_buf, l_buf, a_buf, q_leaf]
     tmax = max(int(trips.max()), 1)
     for key in ("k", "v"):
         alloc, rel, row, step = tiles[key]
-        ex.log(alloc, False, rel, (tmax, AT, AT), (step, row, 1))
+        ex.log(alloc, False, rel, (tmax, N, D), (step, row, 1))
     ex.launch("attn", d, keep)
     ex.attn_pending = dict(desc=d, keep=keep, acc=a_buf, l=l_buf, lanes=L, level=len(ex.levels),
                            body_names=set(names),
                            reads={id(x) for x in (q_leaf.alloc, tiles["k"][0], tiles["v"][0]) if x is not None})
-    vec = lambda b: Tile(Expr("ld", "f32", (AT,), attr=LeafSpec(b.ptr, "f32", LaneOff(0, AT), (1,), 0, L * AT,
-                                                                  keep=(b,))))
+    vec = lambda b: Tile(Expr("ld", "f32", (M,), attr=LeafSpec(b.ptr, "f32", LaneOff(0, M), (1,), 0, L * M,
+                                                                 keep=(b,))))
     res = [None, None, None]
     res[im], res[il] = vec(m_buf), vec(l_buf)
-    res[ia] = Tile(Expr("ld", "f32", (AT, AT), attr=LeafSpec(a_buf.ptr, "f32", LaneOff(0, AT * AT), (AT, 1), 0,
-                                                               L * AT * AT, keep=(a_buf,))))
+    res[ia] = Tile(Expr("ld", "f32", (M, D), attr=LeafSpec(a_buf.ptr, "f32", LaneOff(0, M * D), (D, 1), 0,
+                                                             L * M * D, keep=(a_buf,))))
     return res
 
 
@@ -1041,13 +1050,14 @@ def _paged_attention(ex, trips, tm1, q, probes, peeled, l0, slots, mask):
     return res
 
 
-def _plain_ld(e, ptr, inner):
+def _plain_ld(e, ptr, shape, inner):
     """`e` reads a whole attention state buffer at `ptr`: lane stride = one
-    lane's block, the two inner strides `inner`, any leading dims of extent 1."""
+    lane's block, the two inner extents `shape` and strides `inner`, any
+    leading dims of extent 1."""
     if e.kind != "ld" or e.attr.ptr != ptr or e.attr.offsets is not None or e.attr.winner is not None:
         return False
     sh, stv = tuple(e.shape), tuple(e.attr.strides)
-    if len(sh) < 2 or any(x != 1 for x in sh[:-2]) or tuple(sh[-2:]) != (128, 128):
+    if len(sh) < 2 or any(x != 1 for x in sh[:-2]) or tuple(sh[-2:]) != shape:
         return False
     return stv[-2:] == inner and e.attr.lane.arr is None and e.attr.lane.base == 0
 
@@ -1067,10 +1077,10 @@ def attention_epilogue(ex, e, dest) -> bool:
         x = x.args[0]
     if x.kind != "bin" or x.attr != rt.op("DIVF") or x.dtype != "f32" or len(x.args) != 2:
         return False
-    acc_buf, l_buf = pend["acc"], pend["l"]
+    acc_buf, l_buf, M, D = pend["acc"], pend["l"], pend["desc"].M, pend["desc"].D
     a, b = x.args
-    if not (_plain_ld(a, acc_buf.ptr, (128, 1)) and a.attr.lane.stride == 128 * 128
-            and _plain_ld(b, l_buf.ptr, (1, 0)) and b.attr.lane.stride == 128):
+    if not (_plain_ld(a, acc_buf.ptr, (M, D), (D, 1)) and a.attr.lane.stride == M * D
+            and _plain_ld(b, l_buf.ptr, (M, D), (1, 0)) and b.attr.lane.stride == M):
         return False
     if dest.dtype not in ("f32", "bf16", "f16") or dest.offsets is not None or dest.winner is not None:
         return False
@@ -1084,8 +1094,8 @@ def attention_epilogue(ex, e, dest) -> bool:
     L = ex.L
     o_row = int(dst[-2])
     offs = dest.lane.values(L)
-    if np.any(offs < dest.lo) or np.any(offs + 127 * o_row + 127 >= dest.hi) or np.any(offs % 8) or o_row % 8 \
-            or o_row < 128:
+    if np.any(offs < dest.lo) or np.any(offs + (M - 1) * o_row + D - 1 >= dest.hi) or np.any(offs % 8) or o_row % 8 \
+            or o_row < D:
         return False
     d = pend["desc"]
     # acc stays needed if any live value other than this store still reads it

@@ -452,6 +452,62 @@ def test_flash_attention_fused(args):
         np.testing.assert_array_equal(out[k], ref[k])
 
 
+# (rows = keys, columns), causal, S: a pair of lanes, a lane without a partner
+# (three query blocks of a stream), one block
+_TILE_SHAPES = [(64, 64, True, 256), (64, 64, False, 192), (64, 64, True, 64), (128, 64, True, 384),
+                (128, 64, False, 256), (64, 128, True, 192), (64, 128, False, 128)]
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("blk,D,causal,S", _TILE_SHAPES)
+def test_flash_attention_tiles(blk, D, causal, S, dt):
+    """The loop's tiles of 64 or 128 rows, keys and columns in one launch:
+    P, l and acc are f32-exact, so a result is its f32 value (of sums in
+    another order) rounded once: one unit of the output type."""
+    ref, out, g = _run(_cases.flash_attention(B=1, H=2, S=S, D=D, blk=blk, dt=dt, causal=causal))
+    assert dict(g.last_plan.counts()) == {"attn": 1}
+    f = bf16_from_bits if dt == "bf16" else (lambda x: x.astype(np.float32))
+    np.testing.assert_allclose(f(out["o_ptr"]), f(ref["o_ptr"]), rtol=2.0 ** (-7 if dt == "bf16" else -10), atol=1e-5)
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("fill,sign", [("-1.0e4", 1), ("0xFF800000", -1)])
+def test_flash_attention_tiles_other_fill_or_scale(fill, sign, dt):
+    src, fn, kw = _cases.flash_attention(B=1, H=1, S=192, D=64, blk=64, dt=dt)
+    src = src.replace("%neg_inf = arith.constant 0xFF800000 : f32",
+                      f"%neg_inf = arith.constant 0xFF800000 : f32\n    %fill = arith.constant {fill} : f32")
+    src = src.replace("%r = arith.select %keep, %sv, %neg_inf : f32", "%r = arith.select %keep, %sv, %fill : f32")
+    kw["scale"] = sign * kw["scale"]
+    ref, out, g = _run((src, fn, kw))
+    assert g.last_plan.counts().get("attn") == 1
+    f = bf16_from_bits if dt == "bf16" else (lambda x: x.astype(np.float32))
+    np.testing.assert_allclose(f(out["o_ptr"]), f(ref["o_ptr"]), rtol=2.0 ** (-7 if dt == "bf16" else -10), atol=1e-5)
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("blk,D", [(64, 64), (128, 64), (64, 128)])
+def test_flash_attention_tiles_non_finite_inputs(blk, D, dt):
+    """NaN in a query row, infinities in a key and in V: NaN and the
+    infinities of P V exactly where the oracle has them."""
+    from oracle.interp import bf16_bits
+    src, fn, kw = _cases.flash_attention(B=1, H=2, S=256, D=D, blk=blk, dt=dt)
+    f = bf16_from_bits if dt == "bf16" else (lambda x: x.astype(np.float32))
+    back = (lambda x: bf16_bits(x.astype(np.float32))) if dt == "bf16" else (lambda x: x.astype(np.float16))
+    q, k, v = (f(kw[n]).copy() for n in ("q_ptr", "k_ptr", "v_ptr"))
+    q[0, 1, 70, 7] = np.nan
+    k[0, 0, 130, 3] = np.inf
+    v[0, 0, 20, 5] = np.inf
+    v[0, 1, 65, 9], v[0, 1, 66, 11] = -np.inf, np.nan
+    kw["q_ptr"], kw["k_ptr"], kw["v_ptr"] = back(q), back(k), back(v)
+    ref, out, g = _run((src, fn, kw))
+    assert g.last_plan.counts().get("attn") == 1
+    got, want = f(out["o_ptr"]), f(ref["o_ptr"])
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+    assert np.isnan(want).any() and np.isposinf(want).any() and np.isneginf(want).any()
+    ok = ~np.isnan(want)
+    np.testing.assert_allclose(got[ok], want[ok], rtol=2.0 ** (-7 if dt == "bf16" else -10), atol=1e-5)
+
+
 @pytest.mark.parametrize("dt", ["bf16", "f16"])
 def test_flash_attention_fused_without_pairs(dt, monkeypatch):
     """A launch that names no lane pairs (as a C-ABI caller may) runs one
