@@ -15,14 +15,12 @@
 // (LDS for s >= 64, wave shuffles below), the last pairs the two elements of
 // a pair.  Each combine is commutative, so both partners of a butterfly hold
 // the lower element's value and the result ends up in every thread.
-#include "ktir_program_impl.h"
+#include "ktir_rowform.h"
 
 namespace ktir {
 
 constexpr int RC_MAX_STEPS = 16;
 
-typedef float gf2 __attribute__((ext_vector_type(2)));
-typedef uint32_t gu4 __attribute__((ext_vector_type(4)));
 constexpr int RC_MAX_OPS = 8;
 
 struct RcOp {
@@ -102,8 +100,9 @@ struct RowRegs {
 
 // ---- host-side analysis ------------------------------------------------------
 
-static bool rows_leaf_ok(const ktir_leaf_t& L, int nd) {
-  return L.offsets == 0 && L.winner == 0 && L.strides[nd - 1] == 1 && (L.flags & KTIR_LEAF_VEC) &&
+// `vec`: the flag bits the row's accesses need (0: rows of any alignment)
+static bool rows_leaf_ok(const ktir_leaf_t& L, int nd, int vec) {
+  return L.offsets == 0 && L.winner == 0 && L.strides[nd - 1] == 1 && (L.flags & vec) == vec &&
          (L.dtype == KTIR_F16 || L.dtype == KTIR_BF16 || L.dtype == KTIR_F32);
 }
 
@@ -172,7 +171,7 @@ static bool plan_plain(const RcPlan& R) {
   return true;
 }
 
-static bool analyze_rows(const ktir_prog_t& P, RcPlan& R) {
+static bool analyze_rows(const ktir_prog_t& P, RcPlan& R, int vec) {
   enum { K_NONE = 0, K_ROW = 1, K_LEAF = 2, K_ACC = 3 };
   int kind[KTIR_NREG], slot_of[KTIR_NREG];
   for (int i = 0; i < KTIR_NREG; ++i) kind[i] = K_NONE, slot_of[i] = -1;
@@ -182,7 +181,7 @@ static bool analyze_rows(const ktir_prog_t& P, RcPlan& R) {
   auto slot_for = [&](int leaf) -> int {
     for (int s = 0; s < R.n_slots; ++s)
       if (R.slot_leaf[s] == leaf) return s;
-    if (R.n_slots == 2 || !rows_leaf_ok(P.leaves[leaf], nd)) return -1;
+    if (R.n_slots == 2 || !rows_leaf_ok(P.leaves[leaf], nd, vec)) return -1;
     R.slot_leaf[R.n_slots] = (int8_t)leaf;
     return R.n_slots++;
   };
@@ -305,7 +304,7 @@ static bool analyze_rows(const ktir_prog_t& P, RcPlan& R) {
         if (x.op == KTIR_OP_RED) {
           S.end = 0;
         } else {
-          if (!rows_leaf_ok(P.leaves[x.aux], nd)) return false;
+          if (!rows_leaf_ok(P.leaves[x.aux], nd, vec)) return false;
           S.end = 1;
           S.st_leaf = (int8_t)x.aux;
         }
@@ -461,16 +460,6 @@ __device__ __forceinline__ float minnan(float x, float y) {
 // e^x on the hardware exp2: 2^(x log2 e).  The rounding of x log2 e costs
 // about |x| * 6e-8 relative error (a few f32 ulps for softmax arguments).
 __device__ __forceinline__ float exp_hw(float x) { return __builtin_amdgcn_exp2f(x * 1.44269504088896341f); }
-
-// x / s for a row scalar s with r = 1/s correctly rounded: q = x r, then one
-// Markstein correction q + (x - s q) r (fused); within one ulp of x / s and
-// nearly always its correct rounding.  Operands near the ends of the
-// exponent range take __fdiv_rn.
-__device__ __forceinline__ float div_by(float x, float s, float r) {
-  const float q = x * r;
-  const float res = __builtin_fmaf(-s, q, x);
-  return __builtin_fmaf(res, r, q);
-}
 
 // one chain op over the E chain values; the opcode and operand kind are
 // uniform, so both are dispatched once outside the element loops.  Ops are
@@ -775,13 +764,6 @@ __global__ __launch_bounds__(256) void prog_rowchain(const ktir_prog_t P, const 
 // Self-contained plan of the row-wave kernel (copied to LDS by each
 // workgroup, so the kernel's control reads are LDS reads that never wait
 // behind the row loads in flight).
-struct RwLeaf {
-  uint64_t ptr, lane_base;
-  int64_t base, lane_stride, lo, hi;
-  int64_t strides[KTIR_MAX_DIMS - 1];   // outer dims
-  int32_t dtype, esize;
-};
-
 struct RwHead {
   int8_t kind, src, n_ops, end, fold_op, fold_dt, dst, out;   // out: store leaf (index into RwPlan.leaf)
   int8_t head, pad[3];
@@ -1056,42 +1038,6 @@ __device__ __forceinline__ float rw_pass(const RwHead& S, const RcOp* ops, const
   return FOLDX ? fold_any(fop, fdt, a, b) : fold_rt(fop, a, b);
 }
 
-// Position of row r: its lane (core) and its index in each outer dim.  Rows,
-// lanes and dims are below 2^31 (checked at launch): 32-bit division.
-struct RwPos {
-  int32_t lane;
-  int32_t idx[KTIR_MAX_DIMS - 1];
-};
-
-template <typename PL>
-__device__ __forceinline__ RwPos rw_pos(const PL& SP, int64_t r, int32_t rows_per_lane) {
-  RwPos p;
-  const uint32_t ru = (uint32_t)r, rpl = (uint32_t)rows_per_lane;
-  const uint32_t lane = ru / rpl;
-  uint32_t t = ru - lane * rpl;
-  p.lane = (int32_t)lane;
-  const int nd = __builtin_amdgcn_readfirstlane(SP.nd);
-#pragma unroll
-  for (int d = KTIR_MAX_DIMS - 2; d >= 0; --d) {
-    p.idx[d] = 0;
-    if (d < nd - 1) {
-      const uint32_t ext = (uint32_t)__builtin_amdgcn_readfirstlane((int)SP.shape[d]);
-      const uint32_t q = t / ext;
-      p.idx[d] = (int32_t)(t - q * ext);
-      t = q;
-    }
-  }
-  return p;
-}
-
-// element offset of column 0 of the row at p in leaf L
-__device__ __forceinline__ int64_t rw_row_base(const RwLeaf& L, const RwPos& p) {
-  int64_t e = L.lane_base ? uni(((const KTIR_G(int64_t)*)L.lane_base)[p.lane]) : L.base + (int64_t)p.lane * L.lane_stride;
-#pragma unroll
-  for (int d = 0; d < KTIR_MAX_DIMS - 1; ++d) e += (int64_t)p.idx[d] * L.strides[d];
-  return e;
-}
-
 // registers <- row r of the non-invariant slots; false (nothing read) when a
 // row is not wholly inside its allocation
 template <int NQ>
@@ -1146,37 +1092,6 @@ __device__ __forceinline__ void rw_stage_slow(const RwPlan& SP, int s, const RwP
     else if (L.dtype == KTIR_BF16) ((uint16_t*)dst)[i] = (uint16_t)(__float_as_uint(v) >> 16);
     else ((_Float16*)dst)[i] = (_Float16)v;
   }
-}
-
-template <typename PL, typename RR>
-__device__ __forceinline__ void rw_row_exec(const PL& SP, const ktir_instr_t in, RR& rr, int64_t lane) {
-  const int op = in.op;
-  const float a = rr.get(in.a), b = rr.get(in.b);
-  float v;
-  if (op >= KTIR_OP_NEGF && op < KTIR_OP_ADDF) {
-    v = unop_simple(op, in.dt, a);
-  } else if (op >= KTIR_OP_ADDI) {
-    v = __int_as_float(binop_i_simple(op, __float_as_int(a), __float_as_int(b)));
-  } else if (op >= KTIR_OP_ADDF) {
-    v = binop_f_simple(op, in.dt, a, b);
-  } else {
-    switch (op) {
-      case KTIR_OP_CONST: v = __int_as_float(in.imm); break;
-      case KTIR_OP_LANE: {
-        const double d = ((const KTIR_G(double)*)uni((int64_t)SP.lane_scalars))[lane * uni(SP.n_lane_scalars) + in.aux];
-        v = is_float_dt(in.dt) ? round_to((float)d, in.dt) : __int_as_float((int)(long long)d);
-        break;
-      }
-      case KTIR_OP_CAST: v = cast_val(a, in.aux, in.dt); break;
-      case KTIR_OP_BITCAST: v = a; break;
-      case KTIR_OP_SELECT: v = __float_as_int(a) ? b : rr.get(in.c); break;
-      case KTIR_OP_FMA: v = round_to(__fadd_rn(__fmul_rn(a, b), rr.get(in.c)), in.dt); break;
-      case KTIR_OP_CMPF: v = __int_as_float(cmp_f(in.aux, a, b)); break;
-      case KTIR_OP_CMPI: v = __int_as_float(cmp_i(in.aux, __float_as_int(a), __float_as_int(b))); break;
-      default: v = 0.f;
-    }
-  }
-  rr.set(in.dst, __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v))));
 }
 
 // Row staging: the next row's cached leaves are read into registers (NQ
@@ -1425,67 +1340,6 @@ static bool try_launch_rowwave(const ktir_prog_t& P, const RcPlan& R, int64_t ro
 // packed f16 instructions give the same bits; exp is the hardware exp2
 // rounded to f16 (within one f16 ulp of NumPy's, as the general kernels'
 // exp), and the division a quotient within one f32 ulp rounded to f16.
-constexpr int RF_MAX_ROW = 8;
-enum { RF_SOFTMAX = 1, RF_NORM = 2, RF_SOFTMAX16 = 3, RF_NORM16 = 4 };
-
-struct RfPlan {
-  int32_t nd, has_w, w_first, n_row0, n_row1, numf;   // numf: softmax16's max ignores NaN
-  int64_t shape[KTIR_MAX_DIMS];
-  uint64_t lane_scalars;
-  int64_t n_lane_scalars;
-  RwLeaf x, w, y;
-  int8_t fold0, fold1;        // registers the folds write
-  int8_t m, s;                // softmax: the subtracted register and the divisor; norm-scale: s the multiplier
-  int32_t pad1;
-  ktir_instr_t row0[RF_MAX_ROW], row1[RF_MAX_ROW];   // after the first and the second fold
-};
-
-template <int DT>
-__device__ __forceinline__ void rf_unpack(const gu4 c, float (&v)[8]) {
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const uint32_t u = c[k];
-    if (DT == KTIR_BF16) {
-      v[2 * k] = __uint_as_float(u << 16);
-      v[2 * k + 1] = __uint_as_float(u & 0xffff0000u);
-    } else {
-      v[2 * k] = (float)__builtin_bit_cast(_Float16, (uint16_t)(u & 0xffffu));
-      v[2 * k + 1] = (float)__builtin_bit_cast(_Float16, (uint16_t)(u >> 16));
-    }
-  }
-}
-
-// eight values rounded to nearest-even in DT, packed
-template <int DT>
-__device__ __forceinline__ gu4 rf_pack(const float (&v)[8]) {
-  gu4 c;
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    if (DT == KTIR_BF16)
-      c[k] = (__float_as_uint(round_bf16(v[2 * k])) >> 16) | (__float_as_uint(round_bf16(v[2 * k + 1])) & 0xffff0000u);
-    else
-      c[k] = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)v[2 * k]) |
-             ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)v[2 * k + 1]) << 16);
-  }
-  return c;
-}
-
-// as rf_pack, f16 pairs converted by one instruction (v_cvt_pk_f16_f32, round
-// to nearest even); the row kernels whose register count it does not raise
-template <int DT>
-__device__ __forceinline__ gu4 rf_pack2(const float (&v)[8]) {
-  if (DT == KTIR_BF16) return rf_pack<DT>(v);
-  typedef float f2 __attribute__((ext_vector_type(2)));
-  typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-  gu4 c;
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const f2 x = {v[2 * k], v[2 * k + 1]};
-    c[k] = __builtin_bit_cast(uint32_t, __builtin_convertvector(x, h2));
-  }
-  return c;
-}
-
 // the chunks of the 16-bit row at element e0 of L: 16-byte loads when the row
 // lies inside [lo, hi), else element by element (out-of-range elements read 0)
 template <int NQ>
@@ -1565,18 +1419,6 @@ __device__ __forceinline__ float rf_sum(G get) {
     for (int j = 0; j < h; ++j) a[j] = __fadd_rn(a[j], a[j + h]);
   return a[0];
 }
-
-// Row registers in lanes 0..7 of one vector register: a read is one lane
-// access and a write one lane select, with no selection over the register
-// number.
-struct RowLanes {
-  int v, lane;
-  __device__ __forceinline__ float get(int i) const { return __int_as_float(__builtin_amdgcn_readlane(v, i)); }
-  __device__ __forceinline__ void set(int i, float x) {
-    const int u = __builtin_amdgcn_readfirstlane(__float_as_int(x));
-    v = lane == i ? u : v;
-  }
-};
 
 // An empty statement that the compiler must assume rewrites the chunks: the
 // row is unpacked again in each pass from its 16-bit chunks instead of being
@@ -2037,8 +1879,8 @@ static void rowfix_dt(const RfPlan& F, int recipe, int dt, int64_t rows) {
   }
 }
 
-static bool rf_leaf_ok(const ktir_leaf_t& L, int nd, int dt) {
-  return rows_leaf_ok(L, nd) && L.dtype == dt && (L.flags & KTIR_LEAF_VEC8);
+static bool rf_leaf_ok(const ktir_leaf_t& L, int nd, int dt, int vec) {
+  return rows_leaf_ok(L, nd, vec) && L.dtype == dt;
 }
 
 static bool rf_invariant(const ktir_prog_t& P, const ktir_leaf_t& L) {
@@ -2051,10 +1893,9 @@ static bool rf_op(const RcOp& o, int op, int kind) {
   return o.op == op && o.dt == KTIR_F32 && o.kind == kind && (op != KTIR_OP_DIVF || o.aux == 0);
 }
 
-// Match the pass plan against the two fixed forms and launch; false leaves
-// the program to the general row kernels.
-static bool try_launch_rowfix(const ktir_prog_t& P, const RcPlan& R, int64_t rows, int64_t inner) {
-  if (inner != 512 && inner != 1024 && inner != 2048 && inner != 4096) return false;
+// Match the pass plan against the fixed forms (rows whose leaves carry the
+// flag bits `vec`): F, `recipe` and the rows' dtype `dt`, or false.
+static bool match_rowfix(const ktir_prog_t& P, const RcPlan& R, int64_t rows, int vec, RfPlan& F, int& recipe, int& dt) {
   if (rows > INT32_MAX) return false;
   for (int d = 0; d < P.ndim; ++d)
     if (P.shape[d] > INT32_MAX) return false;
@@ -2071,7 +1912,7 @@ static bool try_launch_rowfix(const ktir_prog_t& P, const RcPlan& R, int64_t row
       return false;
     }
   }
-  RfPlan F{};
+  F = RfPlan{};
   F.nd = P.ndim;
   for (int d = 0; d < KTIR_MAX_DIMS; ++d) F.shape[d] = d < P.ndim ? P.shape[d] : 1;
   F.lane_scalars = P.lane_scalars;
@@ -2087,11 +1928,11 @@ static bool try_launch_rowfix(const ktir_prog_t& P, const RcPlan& R, int64_t row
   if (A.end != 0 || (A.fold_dt != KTIR_F32 && !m16)) return false;
   const int sx = A.src;
   const ktir_leaf_t& X = P.leaves[R.slot_leaf[sx]];
-  const int dt = X.dtype;
-  if ((dt != KTIR_F16 && dt != KTIR_BF16) || (m16 && dt != KTIR_F16) || !rf_leaf_ok(X, P.ndim, dt)) return false;
+  dt = X.dtype;
+  if ((dt != KTIR_F16 && dt != KTIR_BF16) || (m16 && dt != KTIR_F16) || !rf_leaf_ok(X, P.ndim, dt, vec)) return false;
   F.x = rw_leaf(P, R.slot_leaf[sx]);
   const RcStep& Z = R.steps[pass[n_pass - 1]];   // the storing pass
-  if (Z.end != 1 || Z.src != sx || !rf_leaf_ok(P.leaves[Z.st_leaf], P.ndim, dt) || gap[n_pass - 1] != 0) return false;
+  if (Z.end != 1 || Z.src != sx || !rf_leaf_ok(P.leaves[Z.st_leaf], P.ndim, dt, vec) || gap[n_pass - 1] != 0) return false;
   F.y = rw_leaf(P, Z.st_leaf);
   // an optional last rounding to the stored dtype (the store rounds the same way)
   auto tail = [&](const RcStep& S, int n) {
@@ -2109,7 +1950,6 @@ static bool try_launch_rowfix(const ktir_prog_t& P, const RcPlan& R, int64_t row
     return (S.n_ops == i + 2 && nop(S, i, op, kind)) ||
            (S.n_ops == i + 1 && S.ops[i].op == op && S.ops[i].dt == KTIR_F32 && S.ops[i].kind == kind);
   };
-  int recipe;
   if (n_pass == 3 && m16) {
     const RcStep& B = R.steps[pass[1]];
     if (R.n_slots != 1 || A.n_ops != 0 || (A.fold_op != KTIR_OP_MAXNUMF && A.fold_op != KTIR_OP_MAXIMUMF)) return false;
@@ -2147,7 +1987,7 @@ static bool try_launch_rowfix(const ktir_prog_t& P, const RcPlan& R, int64_t row
     if (R.n_slots != 1 + F.has_w) return false;
     if (F.has_w) {
       const ktir_leaf_t& W = P.leaves[R.slot_leaf[1 - sx]];
-      if (!rf_leaf_ok(W, P.ndim, dt) || !rf_invariant(P, W)) return false;
+      if (!rf_leaf_ok(W, P.ndim, dt, vec) || !rf_invariant(P, W)) return false;
       F.w = rw_leaf(P, R.slot_leaf[1 - sx]);
     }
     recipe = RF_NORM16;
@@ -2189,7 +2029,7 @@ static bool try_launch_rowfix(const ktir_prog_t& P, const RcPlan& R, int64_t row
     if (R.n_slots != 1 + F.has_w) return false;
     if (F.has_w) {
       const ktir_leaf_t& W = P.leaves[R.slot_leaf[1 - sx]];
-      if (!rf_leaf_ok(W, P.ndim, dt) || !rf_invariant(P, W)) return false;
+      if (!rf_leaf_ok(W, P.ndim, dt, vec) || !rf_invariant(P, W)) return false;
       F.w = rw_leaf(P, R.slot_leaf[1 - sx]);
     }
     recipe = RF_NORM;
@@ -2198,28 +2038,43 @@ static bool try_launch_rowfix(const ktir_prog_t& P, const RcPlan& R, int64_t row
   }
   F.fold0 = A.dst;
   F.n_row0 = rows_of(0, F.row0);
-  switch (inner / 512) {
-    case 1: rowfix_dt<1>(F, recipe, dt, rows); break;
-    case 2: rowfix_dt<2>(F, recipe, dt, rows); break;
-    case 4: rowfix_dt<4>(F, recipe, dt, rows); break;
-    default: rowfix_dt<8>(F, recipe, dt, rows); break;
-  }
   return true;
 }
 
+// ktir_rowany.hip: softmax and norm-scale rows of any length
+bool launch_rowany(const RfPlan& F, int recipe, int dt, int64_t rows, int64_t n);
+
 // Launch `P` (mode 1) through the row-chain kernel if it has the supported form.
 bool try_launch_rows(const ktir_prog_t& P, int64_t rows, int64_t inner) {
-  if (P.mode != 1 || inner < 64 || inner > 8192 || (inner & (inner - 1))) return false;
+  if (P.mode != 1) return false;
   if (P.lanes > 0 && P.lane_scalars == 0) {
     for (int i = 0; i < P.n_instr; ++i)
       if (P.instr[i].op == KTIR_OP_LANE) return false;
   }
   RcPlan R;
-  if (!analyze_rows(P, R)) return false;
+  if (!analyze_rows(P, R, 0)) return false;
+  RfPlan F;
+  int recipe, dt;
+  const bool fixed = inner == 512 || inner == 1024 || inner == 2048 || inner == 4096;
+  // 512 .. 4096 elements, 16-byte aligned rows: a wavefront holds the row
+  if (fixed && match_rowfix(P, R, rows, KTIR_LEAF_VEC8, F, recipe, dt)) {
+    switch (inner / 512) {
+      case 1: rowfix_dt<1>(F, recipe, dt, rows); break;
+      case 2: rowfix_dt<2>(F, recipe, dt, rows); break;
+      case 4: rowfix_dt<4>(F, recipe, dt, rows); break;
+      default: rowfix_dt<8>(F, recipe, dt, rows); break;
+    }
+    return true;
+  }
+  // any other length or alignment of the f32-math forms, but norm rows of 64
+  // or 128 elements, whose sum the chain kernel folds without LDS (2^25
+  // elements: 432 and 225 us against 505 and 260; from 256 on 157 against 140)
+  const bool short_norm = inner == 64 || inner == 128;
+  if (match_rowfix(P, R, rows, 0, F, recipe, dt) && !(recipe == RF_NORM && short_norm && analyze_rows(P, R, KTIR_LEAF_VEC)) &&
+      launch_rowany(F, recipe, dt, rows, inner))
+    return true;
+  if (inner < 64 || inner > 8192 || (inner & (inner - 1)) || !analyze_rows(P, R, KTIR_LEAF_VEC)) return false;
   const bool plain = plan_plain(R);
-  // the fixed forms: the f32-math ones take plain plans, the f16-math ones
-  // f16 folds (try_launch_rowfix checks which)
-  if (try_launch_rowfix(P, R, rows, inner)) return true;
   if (try_launch_rowwave(P, R, rows, inner, !plain)) return true;
   // threads per row and elements per thread: n = tpr * E, E in {2..32}, tpr in {32..256}
   int tpr = (int)(inner / 16);

@@ -265,6 +265,34 @@ def test_rmsnorm_bit_exact_many_rows_per_workgroup(cols, dt, row_grid_limit):
     np.testing.assert_array_equal(out["y_ptr"], ref["y_ptr"])
 
 
+# one row per wavefront (up to 2048 elements) and per workgroup; whole chunks,
+# a cut last chunk, odd lengths (rows off every alignment), the longest rows
+_ANY_COLS = [5, 8, 64, 100, 513, 1000, 2047, 2056, 3000, 3001, 3072, 3080, 5120, 6144, 8192, 12287, 16383, 16384]
+
+
+@pytest.mark.parametrize("limit", [0, 3])
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("cols", _ANY_COLS)
+def test_softmax_any_length(cols, dt, limit, row_grid_limit):
+    """f32 exponentials and sums (the sum in another order than the oracle's),
+    one rounding: within one unit of the output type, subnormals included."""
+    row_grid_limit(limit)
+    ref, out, g = _run(_cases.softmax(rows=20, cols=cols, cores=4, rblk=1, dt=dt))
+    assert g.last_plan.counts() == {"prog": 1}
+    np.testing.assert_allclose(_half_f32(out["y_ptr"], dt), _half_f32(ref["y_ptr"], dt),
+                               rtol=2.0 ** (-10 if dt == "f16" else -7), atol=2.0 ** -24 if dt == "f16" else 1e-38)
+
+
+@pytest.mark.parametrize("limit", [0, 3])
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("cols", _ANY_COLS)
+def test_rmsnorm_any_length_bit_exact(cols, dt, limit, row_grid_limit):
+    row_grid_limit(limit)
+    ref, out, g = _run(_cases.rmsnorm(rows=20, cols=cols, cores=4, rblk=1, dt=dt, wide=True))
+    assert g.last_plan.counts() == {"prog": 1}
+    np.testing.assert_array_equal(out["y_ptr"], ref["y_ptr"])
+
+
 @pytest.mark.parametrize("limit", [0, 3])
 @pytest.mark.parametrize("cols", [64, 256, 1024, 4096, 8192, 96, 3000])
 @pytest.mark.parametrize("combiner", ["arith.addf", "arith.maximumf"])
