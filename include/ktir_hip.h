@@ -289,6 +289,13 @@ typedef struct ktir_mm {
    * 0 / 0: not grouped. */
   uint64_t quads;
   int64_t n_quads;
+  /* Optional (0: not known): the lanes as planes of plane_m x plane_n tiles
+   * (const int32_t* [planes * plane_m * plane_n], row by row, every lane
+   * once): the lane in row r and column c of a plane reads A r * M rows and B
+   * c * N columns after the plane's first lane, so a workgroup may compute
+   * any block of the plane's result. */
+  uint64_t plane;
+  int64_t plane_m, plane_n;
 } ktir_mm_t;
 int ktir_launch_matmul(const ktir_mm_t* d);
 

@@ -89,6 +89,9 @@ __global__ __launch_bounds__(256) void mm_generic(const ktir_mm_t d) {
 using namespace ktir;
 
 int ktir_launch_matmul_mfma(const ktir_mm_t* d, bool* handled);
+namespace ktir {
+bool launch_mm_plane(const ktir_mm_t* d);
+}
 
 extern "C" int ktir_launch_matmul(const ktir_mm_t* d) {
   if (!d || d->M < 0 || d->N < 0 || d->K < 0 || d->ksteps < 1) return set_error(KTIR_E_ARG, "ktir_launch_matmul: bad descriptor");
@@ -96,6 +99,10 @@ extern "C" int ktir_launch_matmul(const ktir_mm_t* d) {
   bool handled = false;
   int rc = ktir_launch_matmul_mfma(d, &handled);
   if (rc != KTIR_OK || handled) return rc;
+  if (launch_mm_plane(d)) {
+    KTIR_HIP_CHECK(hipGetLastError());
+    return KTIR_OK;
+  }
   int64_t work = d->lanes * ((d->M + GT - 1) / GT) * ((d->N + GT - 1) / GT);
   unsigned blocks = (unsigned)(work < 65536 ? work : 65536);
   hipLaunchKernelGGL(mm_generic, dim3(blocks), dim3(256), 0, stream(), *d);

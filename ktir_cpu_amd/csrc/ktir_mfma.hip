@@ -13,13 +13,9 @@
 //   A (32 x 16): lane l holds row l%32, k = 8*(l/32) .. +8
 //   B (16 x 32): lane l holds col l%32, k = 8*(l/32) .. +8
 //   D (32 x 32): lane l holds col l%32, rows 8*(i/4) + 4*(l/32) + i%4, i < 16
-#include "ktir_common.h"
+#include "ktir_mfma_common.h"
 
 namespace ktir {
-
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bfx8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int MT = 128, NT = 128, BK = 64, LDK = BK + 8;   // LDS row: 72 halfs (pad breaks bank conflicts)
 
@@ -27,26 +23,6 @@ constexpr int MT = 128, NT = 128, BK = 64, LDK = BK + 8;   // LDS row: 72 halfs 
 __device__ __forceinline__ uint32_t half_of(const uint4& v, int i) {
   const uint32_t w = i < 2 ? v.x : (i < 4 ? v.y : (i < 6 ? v.z : v.w));
   return (i & 1) ? (w >> 16) : (w & 0xffffu);
-}
-
-template <bool BF16>
-__device__ __forceinline__ f32x16 mfma32(const uint4& a, const uint4& b, f32x16 c) {
-  if constexpr (BF16) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bfx8, a), __builtin_bit_cast(bfx8, b), c, 0, 0, 0);
-  } else {
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, a), __builtin_bit_cast(half8, b), c, 0, 0, 0);
-  }
-}
-
-// one result element of dtype DT (f32, f16 or bf16, round to nearest even)
-template <int DT>
-__device__ __forceinline__ void mm_put(uint64_t ptr, int64_t off, float v) {
-  if constexpr (DT == KTIR_F32)
-    ((KTIR_G(float)*)ptr)[off] = v;
-  else if constexpr (DT == KTIR_F16)
-    ((KTIR_G(_Float16)*)ptr)[off] = (_Float16)v;
-  else
-    ((KTIR_G(uint16_t)*)ptr)[off] = (uint16_t)(__float_as_uint(round_bf16(v)) >> 16);
 }
 
 // a wavefront's 64 x 64 quadrant as 2 x 2 MFMA tiles, starting at element
@@ -196,29 +172,6 @@ __global__ __launch_bounds__(256) void mm_mfma(const ktir_mm_t d, int64_t tiles_
 //           8 (l / 32) .. + 8) are two ds_read_b64_tr_b16 transposing reads.
 // Both swizzles make every read phase touch distinct banks (with 32 or 64
 // LDS banks alike).
-typedef short mm_s16x4 __attribute__((ext_vector_type(4)));
-
-// slot permutation of the 16 chunks of a 256-byte LDS row r (an XOR of row
-// bits; conflict-free for ds_read_b64_tr_b16 column reads and ds_read_b128
-// row reads)
-__device__ __forceinline__ int swz16(int r) {
-  return ((r & 1) ? 4 : 0) ^ ((r & 2) ? 10 : 0) ^ ((r & 4) ? 1 : 0) ^ ((r & 8) ? 8 : 0);
-}
-
-__device__ __forceinline__ int swz_a(int r) { return (r & 7) ^ ((r >> 3) & 1); }
-
-__device__ __forceinline__ uint2 mm_tr16(const uint16_t* p) {
-  const mm_s16x4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) mm_s16x4*)p);
-  return __builtin_bit_cast(uint2, v);
-}
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t mm_rsrc(const uint16_t* base, int64_t hi_elems) {
-  int64_t bytes = hi_elems * 2;
-  if (bytes < 0) bytes = 0;
-  if (bytes > 0xffffffffll) bytes = 0xffffffffll;
-  return __builtin_amdgcn_make_buffer_rsrc((void*)base, (short)0, (int)(uint32_t)bytes, 0x00020000);
-}
-
 struct MmStage {
   __amdgpu_buffer_rsrc_t ra, rb;
   uint32_t ao0, ao1;            // lane byte offsets of A blocks (even / odd)
@@ -594,7 +547,16 @@ using namespace ktir;
 // 16-byte aligned rows, M and N multiples of 128, K a multiple of 64.  The
 // caller (the lockstep executor) has already checked that every lane's
 // operand range lies inside its allocation.
+// the fewest 256 x 256 blocks (one workgroup per CU) that beat smaller blocks
+// over the plane (ktir_mmplane.hip): 192 blocks (4096 x 3072 x 1024) 35 against
+// 39 us, 128 blocks (2048 x 4096 x 4096) 96 against 77 us
+constexpr int64_t Q_MIN = 160;
+
 static int64_t kt_steps(const ktir_mm_t* d) { return d->K / BK; }
+
+namespace ktir {
+bool launch_mm_plane(const ktir_mm_t* d);     // ktir_mmplane.hip
+}
 
 int ktir_launch_matmul_mfma(const ktir_mm_t* d, bool* handled) {
   *handled = false;
@@ -637,7 +599,8 @@ int ktir_launch_matmul_mfma(const ktir_mm_t* d, bool* handled) {
                     (d->c.dtype == KTIR_F32 || d->c.dtype == KTIR_F16 || d->c.dtype == KTIR_BF16) &&
                     d->round_dt == KTIR_F32 && d->accumulate != 1 && d->c.strides[1] == 1 &&
                     (127 * d->a.strides[0] + (d->ksteps - 1) * d->a_kstep + d->K) * 2 < (int64_t)0x7fffffff;
-  if (q256) {
+  if ((!q256 || d->n_quads < Q_MIN) && launch_mm_plane(d)) {
+  } else if (q256) {
     if (f16)
       hipLaunchKernelGGL((mm_mfma_256<false>), dim3((unsigned)d->n_quads), dim3(256), 0, stream(), *d);
     else

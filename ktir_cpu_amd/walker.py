@@ -331,6 +331,22 @@ def _mm_quads(la, lb, L: int, M: int, N: int) -> Optional[np.ndarray]:
     return _xcd_blocks(np.asarray(out, dtype=np.int32).reshape(-1, 4), ao, bo).ravel()
 
 
+def _mm_plane(la, lb, L: int, M: int, N: int) -> Optional[np.ndarray]:
+    """The lanes of a matmul as one plane of result tiles ([rows, columns] lane
+    numbers): the lane in row r, column c reads A r M rows and B c N columns
+    after the first.  None unless every (r, c) is one lane."""
+    if L < 1 or la.strides[-1] != 1 or lb.strides[-1] != 1 or la.offsets is not None or lb.offsets is not None:
+        return None
+    ao, bo = la.lane.values(L).astype(np.int64), lb.lane.values(L).astype(np.int64)
+    ua, r = np.unique(ao, return_inverse=True)
+    ub, c = np.unique(bo, return_inverse=True)
+    if len(ua) * len(ub) != L or np.any(np.diff(ua) != M * int(la.strides[-2])) or np.any(np.diff(ub) != N):
+        return None
+    table = np.full((len(ua), len(ub)), -1, np.int32)
+    table[r.reshape(-1), c.reshape(-1)] = np.arange(L)
+    return None if np.any(table < 0) else table
+
+
 # workgroups one XCD runs at once (MI355X: 256 CUs in 8 XCDs, one 256 x 256
 # matmul workgroup per CU)
 _XCD_SLOTS, _N_XCD = 32, 8
@@ -2314,6 +2330,11 @@ class Executor:
             qb = self.pool.upload(quads)
             keep.append(qb)
             d.quads, d.n_quads = qb.ptr, len(quads) // 4
+        plane = _mm_plane(la, lb, L, M, N) if M % 32 == 0 and N % 32 == 0 and dta == dtb and dta in ("f16", "bf16") else None
+        if plane is not None and L > 1:
+            pb = self.pool.upload(plane)
+            keep.append(pb)
+            d.plane, d.plane_m, d.plane_n = pb.ptr, *plane.shape
         keep.append(buf)
         self.launch("mm", d, keep)
         # the SSA value `name` holds this launch's result; a store of it may

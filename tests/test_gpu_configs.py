@@ -385,6 +385,45 @@ def test_gemm_bf16(shape):
     np.testing.assert_allclose(bf16_from_bits(out["c_ptr"]), bf16_from_bits(ref["c_ptr"]), rtol=1e-2, atol=1e-3)
 
 
+# (M, N, K, tile rows, tile columns, tile k, grid): lanes as one plane of
+# results.  64 x 64 blocks with a cut last k step; lanes of 32 x 96 and a
+# single cut step; 64 x 128 blocks, five steps and a cut sixth; 128 x 128 blocks
+# in four stages (seven steps) and in two (an odd number of block rows, a cut step)
+_PLANE_SHAPES = [(192, 320, 96, 64, 64, 32, 3, 5), (96, 192, 40, 32, 96, 40, 1, 2), (1408, 1024, 320, 64, 64, 32, 2, 2),
+                 (1408, 1024, 328, 64, 64, 8, 2, 2), (1536, 1536, 448, 128, 128, 64, 4, 4),
+                 (2240, 2176, 96, 64, 64, 32, 5, 2), (64, 64, 8, 64, 64, 8, 1, 1)]
+
+
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("shape", _PLANE_SHAPES)
+def test_gemm_plane_blocks(shape, dt):
+    """f32 sums of exact products in another order than the oracle's: off by at
+    most K 2^-24 of the sum of magnitudes (about 0.64 for these inputs), then
+    one rounding to the output type."""
+    ref, out, g = _run(_cases.gemm(*shape) if dt == "f16" else _cases.gemm_bf16(*shape))
+    assert set(g.last_plan.counts()) == {"mm"}
+    np.testing.assert_allclose(_half_f32(out["c_ptr"], dt), _half_f32(ref["c_ptr"], dt),
+                               rtol=2.0 ** (-10 if dt == "f16" else -7), atol=shape[2] * 2.0 ** -24)
+
+
+def test_gemm_plane_f32_result_and_separate_lanes():
+    """f32 results of 64 x 64 tiles; then the same launch without its plane
+    (lanes that share nothing): one plane per lane."""
+    from ktir_cpu_amd.interpreter import KTIRInterpreter
+    src, fn, kw = _cases.gemm(192, 320, 96, 64, 64, 32, 3, 5, out_dt="f32")
+    ref, out, g = _run((src, fn, kw))
+    np.testing.assert_allclose(out["c_ptr"], ref["c_ptr"], rtol=1e-5, atol=96 * 2.0 ** -24)
+    it = KTIRInterpreter()
+    it.load(src)
+    prep = it.prepare(fn, **kw)
+    d = prep.plan.launches[0][1]
+    assert (d.plane_m, d.plane_n) == (3, 5)
+    prep.reset_inputs()
+    d.plane = 0
+    prep.run()
+    np.testing.assert_allclose(prep.outputs()["c_ptr"], ref["c_ptr"], rtol=1e-5, atol=96 * 2.0 ** -24)
+
+
 @pytest.mark.parametrize("out_dt", ["f16", "bf16"])
 @pytest.mark.parametrize("pad", [3, 8])
 def test_gemm_256_block_into_wider_rows(out_dt, pad):
