@@ -453,11 +453,21 @@ typedef struct ktir_pattn {
   /* optional finalisation (out_ptr != 0), the division and cast that follow
    * the reference's loop: out[o(r, x)] = (out_dtype)(acc[r][x] / l[r]) with
    * o(r, x) = out_base[l] + (r / out_grp) * out_gstride + (r % out_grp) *
-   * out_row + x, elements outside [out_lo, out_hi) not written; m, l and acc
-   * are written as well */
+   * out_row + x, elements outside [out_lo, out_hi) not written; m, l and (unless
+   * acc_out is 0) acc are written as well */
   uint64_t out_ptr, out_base;          /* out_base: const int64_t* [lanes] */
   int64_t out_grp, out_gstride, out_row, out_lo, out_hi;
   int32_t out_dtype, out_pad;
+  /* optional (items 0: not used): the lanes as items, const int32_t* [2 *
+   * n_items] {first, count} into item_lanes (const int32_t* [lanes], every
+   * lane in one item).  An item's lanes have equal k_base, v_base, tbl_pos,
+   * trips and kpos0 and at most 32 rows together.  With pages of 16 keys, one
+   * 16-bit operand type and 64 or 128 columns, `splits` workgroups share an
+   * item's keys; for splits > 1 ws holds n_items * splits * (64 + 32 * D)
+   * floats.  Other launches ignore the items. */
+  uint64_t items, item_lanes, ws;
+  int64_t n_items;
+  int32_t splits, pad2;
 } ktir_pattn_t;
 int ktir_launch_paged_attention(const ktir_pattn_t* d);
 

@@ -353,7 +353,7 @@ __global__ __launch_bounds__(PA_THREADS) void pattn_kernel(const ktir_pattn_t d,
 #pragma unroll
   for (int k = 0; k < ACC / 4; ++k) {
     const int i = 4 * (tid + k * PA_THREADS);
-    if (i < M * D)
+    if (d.acc_out && i < M * D)
       *(float4*)((float*)d.acc_out + lane * M * D + i) = make_float4(acc[4 * k], acc[4 * k + 1], acc[4 * k + 2], acc[4 * k + 3]);
   }
   if (d.out_ptr) {
@@ -843,6 +843,7 @@ __global__ __launch_bounds__(64) void pattn_mfma(const ktir_pattn_t d, int vec, 
           if (e0 + t >= d.out_lo && e0 + t < d.out_hi) store_elem(d.out_ptr, e0 + t, d.out_dtype, v[t]);
       }
     }
+    if (!d.acc_out) return;
     float* ao = (float*)d.acc_out + (lane * M + n) * D;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -858,6 +859,8 @@ __global__ __launch_bounds__(64) void pattn_mfma(const ktir_pattn_t d, int vec, 
     }
   }
 }
+
+bool launch_pattn_split(const ktir_pattn_t* d);   // ktir_pattn_split.hip
 
 }  // namespace ktir
 
@@ -889,6 +892,10 @@ extern "C" int ktir_launch_paged_attention(const ktir_pattn_t* d) {
                      (long long)d->out_grp);
   if (d->lanes == 0) return KTIR_OK;
   if (d->lanes > INT_MAX) return set_error(KTIR_E_UNSUPPORTED, "ktir_launch_paged_attention: too many lanes");
+  if (launch_pattn_split(d)) {
+    KTIR_HIP_CHECK(hipGetLastError());
+    return KTIR_OK;
+  }
   // the matrix-core form: pages of 16 keys, at most 16 rows, D = 32, 64,
   // 128 or 256, one 16-bit operand type
   const bool same16 = d->q_dtype == d->kv_dtype && (d->kv_dtype == KTIR_F16 || d->kv_dtype == KTIR_BF16);

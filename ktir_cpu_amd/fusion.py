@@ -805,7 +805,7 @@ def _attention_loop(ex, op, lb, st, trips, inits):
         pred, ck0, cq0, neg, kpos_step, row_div = "EQ", np.zeros(L, np.int64), np.zeros(L, np.int64), 0.0, 0, 1
     if isinstance(p0["k"], IATile) and isinstance(p0["v"], IATile):
         return _paged_attention(ex, trips, tm1, q, (p0, p1, pl), (pk, pv), l0, (im, il, ia),
-                                (mask_op is not None, pred, ck0, cq0, neg, kpos_step, row_div))
+                                (mask_op is not None, pred, ck0, cq0, neg, kpos_step, row_div), names)
     if l0 != 0.0 or row_div != 1:
         return None
     qe = q.e
@@ -930,7 +930,7 @@ def _attention_loop(ex, op, lb, st, trips, inits):
     return res
 
 
-def _paged_attention(ex, trips, tm1, q, probes, peeled, l0, slots, mask):
+def _paged_attention(ex, trips, tm1, q, probes, peeled, l0, slots, mask, names):
     """Lower the online-softmax loop whose K and V tiles are pages of a
     cache read through a block table (indirect access tiles whose only
     indirect subscript is the page, as in the reference's
@@ -1037,10 +1037,19 @@ def _paged_attention(ex, trips, tm1, q, probes, peeled, l0, slots, mask):
     m_buf, l_buf, a_buf = ex.pool.temp(L * M * 4), ex.pool.temp(L * M * 4), ex.pool.temp(L * M * D * 4)
     d.m_out, d.l_out, d.acc_out = m_buf.ptr, l_buf.ptr, a_buf.ptr
     keep += [m_buf, l_buf, a_buf, ql]
+    if N == 16 and M <= 32 and D in (64, 128):
+        lanes, items = _pattn_items(trips, k[1], v[1], k[5], ck0.astype(np.int64), M)
+        d.item_lanes, d.items, d.n_items = up(lanes), up(items), len(items)
+        d.splits = _pattn_splits(len(items), int(trips.max()))
+        if d.splits > 1:
+            ws = ex.pool.temp(len(items) * d.splits * (64 + 32 * D) * 4)
+            keep.append(ws)
+            d.ws = ws.ptr
     zero = np.zeros(L, np.int64)
     for alloc in (k[0], v[0], k[4]):
         ex.log(alloc, False, zero, (1,), (1,), whole=True)
     ex.launch("pattn", d, keep)
+    ex.pattn_names = set(names)
     vec = lambda b: Tile(Expr("ld", "f32", (M,), attr=LeafSpec(b.ptr, "f32", LaneOff(0, M), (1,), 0, L * M,
                                                                  keep=(b,))))
     res = [None, None, None]
@@ -1048,6 +1057,38 @@ def _paged_attention(ex, trips, tm1, q, probes, peeled, l0, slots, mask):
     res[ia] = Tile(Expr("ld", "f32", (M, D), attr=LeafSpec(a_buf.ptr, "f32", LaneOff(0, M * D), (D, 1), 0,
                                                              L * M * D, keep=(a_buf,))))
     return res
+
+
+def _pattn_items(trips, k_base, v_base, tbl_pos, kpos0, M, rows=32):
+    """Lanes that read the same pages (equal K and V offsets, table position,
+    trip count and key positions) in items of at most `rows` query rows: (lane
+    numbers item by item, {first, count} of every item).  The items of one
+    stream of pages go to one XCD."""
+    _, grp = np.unique(np.stack([k_base, v_base, tbl_pos, kpos0, trips], 1), axis=0, return_inverse=True)
+    grp = grp.reshape(-1)
+    per = max(1, rows // M)
+    order = np.argsort(grp, kind="stable")
+    rank = np.arange(len(grp)) - np.concatenate([[0], np.cumsum(np.bincount(grp))])[grp[order]]
+    cut = np.flatnonzero(rank % per == 0)
+    count = np.diff(np.append(cut, len(grp)))
+    first = order[cut]
+    # the items in the order of workgroups, then the lanes in that of the items
+    seq = _xcd_order(trips[first], k_base[first], v_base[first])
+    lanes = np.concatenate([order[cut[i]:cut[i] + count[i]] for i in seq]) if len(seq) else np.zeros(0)
+    items = np.zeros((len(seq), 2), np.int32)
+    items[:, 1] = count[seq]
+    items[1:, 0] = np.cumsum(items[:-1, 1])
+    return lanes.astype(np.int32), items
+
+
+def _pattn_splits(n_items, trips, cus=256):
+    """Workgroups (of four wavefronts) that share an item's pages: one where the
+    items alone give most CUs a workgroup (the merge of several costs a launch
+    and a pass over their f32 states), else enough for one per CU, but at least
+    two pairs of pages for a wavefront."""
+    if 4 * n_items >= 3 * cus:
+        return 1
+    return max(1, min(-(-cus // n_items), trips // 16))
 
 
 def _plain_ld(e, ptr, shape, inner):

@@ -447,6 +447,7 @@ class Executor:
         self.sequential = sequential
         self.eager = sequential
         self.attn_pending = None     # last fused attention launch whose epilogue may still fold in
+        self.pattn_names = set()     # iter_args of the last paged attention loop
         self.mm_pending = None       # last matmul launch whose result store may still fold in
         self.allow_expand = allow_expand and not sequential
         self.plan = Plan(pool)
@@ -858,11 +859,16 @@ class Executor:
         if not shape or shape[-1] != D or _prod(shape[:-1]) != M or len(shape) > 3:
             return False
         rows = shape[:-1]
+
+        def spans(strides, want, ext):
+            # the stride of a dimension of one element does not matter
+            return len(strides) == len(want) and all(n == 1 or a == b for a, b, n in zip(strides, want, ext))
+
         if A.ptr != d.acc_out or A.dtype != "f32" or A.offsets is not None or A.lane.arr is not None \
-                or A.lane.base != 0 or A.lane.stride != M * D or A.strides != _cstrides(shape):
+                or A.lane.base != 0 or A.lane.stride != M * D or not spans(A.strides, _cstrides(shape), shape):
             return False
         if B.ptr != d.l_out or B.dtype != "f32" or B.offsets is not None or B.lane.arr is not None \
-                or B.lane.base != 0 or B.lane.stride != M or B.strides != _cstrides(rows) + (0,):
+                or B.lane.base != 0 or B.lane.stride != M or not spans(B.strides, _cstrides(rows) + (0,), shape):
             return False
         if dest.dtype != e.dtype or dest.offsets is not None or dest.winner or dest.strides[-1] != 1:
             return False
@@ -882,6 +888,12 @@ class Executor:
         d.out_ptr, d.out_base = dest.ptr, base.ptr
         d.out_grp, d.out_gstride, d.out_row, d.out_lo, d.out_hi = grp, gstride, row, dest.lo, dest.hi
         d.out_dtype = rt.DTYPE_CODE[dest.dtype]
+        # acc is written only where a live value other than this store reads it
+        # (the loop's own iter_args are not visible after the loop)
+        if not any(isinstance(v, Tile) and v.e is not e and name not in self.pattn_names
+                   and any(n.kind == "ld" and n.attr.ptr == d.acc_out for n in topo(v.e))
+                   for fr in self.frames for name, v in fr.vals.items()):
+            d.acc_out = 0
         return True
 
     def _split(self, e: Expr) -> Expr:

@@ -79,6 +79,60 @@ def test_paged_attention_shapes_within_tolerance(gen, inp, args):
     assert plan.counts().get("pattn") == 1
 
 
+# one token: the keys over two workgroups, an odd last pair of pages, one page;
+# 32 rows per lane; three lanes of 8 rows in the last item (7 lanes of a head)
+PA_SPLIT = [
+    ("decode", dict(tokens=1, block_q=1, blocks=128, max_pages=64), dict(num_tiles=33, context_len=520), 2),
+    ("decode_d64", dict(tokens=1, block_q=1, head=64, blocks=128, max_pages=64), dict(num_tiles=48, context_len=767), 3),
+    ("one_page", dict(tokens=1, block_q=1), dict(num_tiles=1, context_len=11), 1),
+    ("rows32", dict(tokens=16, block_q=8), dict(num_tiles=9, context_len=120), 1),
+    ("rows32_d64", dict(tokens=16, block_q=8, head=64), dict(num_tiles=4, context_len=45), 1),
+    ("part_item", dict(tokens=14, block_q=2), dict(num_tiles=6, context_len=77), 1),
+]
+
+
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("gen,args,splits", [c[1:] for c in PA_SPLIT], ids=[c[0] for c in PA_SPLIT])
+def test_paged_attention_split_keys_within_tolerance(gen, args, splits, dt):
+    from oracle.interp import bf16_bits
+    inp = {k: v for k, v in gen.items() if k != "block_q"}
+    kw = paged_inputs(seed=5, **inp)
+    if dt == "bf16":
+        kw = {k: (bf16_bits(v.astype(np.float32)) if k != "block_tables_ptr" else v) for k, v in kw.items()}
+    got, ref, plan = _both(configs.paged_attention(dt=dt, **gen), PA_FN, dict(kw, **dict(PA_ARGS, **args)), "output_ptr")
+    f = _bf16_f32 if dt == "bf16" else (lambda x: x.astype(np.float32))
+    np.testing.assert_allclose(f(got), f(ref), rtol=1e-2, atol=1e-3)
+    d = plan.launches[-1][1]
+    assert d.splits == splits and d.n_items > 0 and d.acc_out == 0
+
+
+def test_paged_attention_many_pages_per_wavefront(monkeypatch):
+    """More than 32 pairs of pages for a wavefront (the table is read 64
+    entries at a time), one page of them past the cache."""
+    from ktir_cpu_amd import fusion
+    monkeypatch.setattr(fusion, "_pattn_splits", lambda *a: 1)
+    gen = dict(tokens=1, q_heads=8, kv_heads=2, block_q=1, blocks=320, max_pages=300)
+    kw = paged_inputs(tokens=1, q_heads=8, kv_heads=2, blocks=320, max_pages=300, seed=9)
+    kw["block_tables_ptr"][0, 211] = 320 + 3
+    got, ref, plan = _both(configs.paged_attention(**gen), PA_FN,
+                           dict(kw, **dict(PA_ARGS, num_tiles=299, context_len=4770)), "output_ptr")
+    np.testing.assert_allclose(got.astype(np.float32), ref.astype(np.float32), rtol=1e-2, atol=1e-3)
+
+
+@pytest.mark.parametrize("num_tiles", [2, 5])
+def test_paged_attention_first_page_masked_is_nan(num_tiles):
+    """Keys from a row's position on: a row whose first page is masked whole is
+    NaN in the reference (exp(-inf - (-inf)) at its first step), also where
+    later pages hold kept keys; other rows, and pages masked whole later, are not."""
+    src = configs.paged_attention().replace("%keep = arith.cmpi ule", "%keep = arith.cmpi uge")
+    kw = dict(paged_inputs(seed=4), **dict(PA_ARGS, num_tiles=num_tiles, context_len=10))
+    got, ref, plan = _both(src, PA_FN, kw, "output_ptr")
+    assert np.isnan(ref).any() and np.isfinite(ref).any()
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(ref))
+    ok = np.isfinite(ref)
+    np.testing.assert_allclose(got[ok].astype(np.float32), ref[ok].astype(np.float32), rtol=1e-2, atol=1e-3)
+
+
 @pytest.mark.parametrize("n,d,rows", [(32, 64, 32), (256, 128, 64)])
 def test_sdpa_f16_within_tolerance(n, d, rows):
     kw = sdpa_inputs(n, d, seed=n)
