@@ -303,8 +303,8 @@ __global__ __launch_bounds__(256) void prog_map(const ktir_prog_t P, const FlatD
 }
 
 // Three or four inputs of one dtype DI, four registers (the host's register
-// allocation reuses an input's register once it is dead, so a RoPE half
-// (x1 cos - x2 sin) fits), one store: the form of prog_map with NIN inputs,
+// allocation reuses an input's register once it is dead), one store: the form
+// of prog_map with NIN inputs (sums of two products run on prog_rot instead),
 // every array indexed by constants only (named per-chunk values).
 struct MapOffs4 {
   int64_t in[4], o, lane;

@@ -244,6 +244,7 @@ using namespace ktir;
 
 namespace ktir {
 bool try_launch_map(const ktir_prog_t& Q, int64_t rows, int64_t inner);
+bool try_launch_rot(const ktir_prog_t& P, int64_t rows, int64_t inner);
 bool try_launch_tile(const ktir_prog_t& Q, int64_t lanes, int64_t per_lane, int64_t inner);
 bool try_launch_rows(const ktir_prog_t& P, int64_t rows, int64_t inner);
 int64_t row_grid_limit(int64_t blocks);
@@ -285,6 +286,10 @@ extern "C" int ktir_launch_program(const ktir_prog_t* P) {
     }
     dim3 b(256);
     uint32_t nv = (uint32_t)vecs;
+    if (!full && try_launch_rot(*P, rows, inner)) {   // a*b +- c*d, one or both sums of a rotation
+      KTIR_HIP_CHECK(hipGetLastError());
+      return KTIR_OK;
+    }
     if (!full && P->n_pf > 2 && try_launch_map(*P, rows, inner)) {   // three or four inputs in four registers
       KTIR_HIP_CHECK(hipGetLastError());
       return KTIR_OK;

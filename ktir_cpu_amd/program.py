@@ -478,6 +478,66 @@ def _compile_flat(root, nodes, lds, lanes, dest, space):
     return prog, keep
 
 
+def rotation_sum(e: Expr, dest: LeafSpec):
+    """(opcode, dtype, [a, b, c, d]) of an expression a*b +- c*d of four
+    different strided tiles, all of one float type that is also the stored
+    one, else None.  The flat program of such an expression holds the tiles in
+    leaves and registers 0..3 and the destination in leaf 4."""
+    if e.kind != "bin" or e.attr not in (rt.op("ADDF"), rt.op("SUBF")) or e.dtype not in ("f16", "bf16", "f32"):
+        return None
+    lds = []
+    for m in e.args:
+        if m.kind != "bin" or m.attr != rt.op("MULF") or m.dtype != e.dtype or m.shape != e.shape:
+            return None
+        lds += m.args
+    specs = [n.attr for n in lds if n.kind == "ld"]
+    if len({id(s) for s in specs}) != 4 or dest.dtype != e.dtype:
+        return None
+    if any(s.dtype != e.dtype or s.offsets is not None or s.winner is not None for s in specs + [dest]):
+        return None
+    return int(e.attr), e.dtype, specs
+
+
+def rotation_pair_program(first: rt.Prog, second: rt.Prog, op1: int, op2: int, at) -> rt.Prog:
+    """One flat program that stores the sums of `first` and `second` (both of
+    `rotation_sum`'s form); factor k of the second is input at[k] of the first."""
+    O = _ops()
+    p = rt.Prog.from_buffer_copy(first)
+    p.leaves[5] = second.leaves[4]
+    p.n_leaves = 6
+    mul, dt = rt.op("MULF"), int(first.leaves[4].dtype)
+    code = []
+    for op, f, leaf in ((op1, (0, 1, 2, 3), 4), (op2, at, 5)):
+        code += [(mul, 4, f[0], f[1], 0), (mul, 5, f[2], f[3], 0), (op, 6, 4, 5, 0), (O["ST"], 0, 6, 0, leaf)]
+    p.n_instr = len(code)
+    for i, (o, dst, a, b, leaf) in enumerate(code):
+        ins = p.instr[i]
+        ins.op, ins.dst, ins.a, ins.b, ins.c, ins.dt, ins.aux, ins.imm = o, dst, a, b, 0, dt, leaf, 0
+    return p
+
+
+def disjoint(a: LeafSpec, la: np.ndarray, b: LeafSpec, lb: np.ndarray, shape) -> bool:
+    """Whether two tiles of unit inner stride surely share no element: they
+    lie in allocations that do not overlap, or the same rows (equal strides,
+    lane offsets a constant apart) at column ranges that do not meet modulo
+    the common divisor of every row step."""
+    es = rt.ELEM_BYTES[a.dtype]
+    if a.ptr + a.hi * es <= b.ptr + b.lo * es or b.ptr + b.hi * es <= a.ptr + a.lo * es:
+        return True
+    if (a.ptr, a.dtype, a.strides) != (b.ptr, b.dtype, b.strides) or a.strides[-1] != 1:
+        return False
+    la, lb = np.asarray(la, np.int64), np.asarray(lb, np.int64)
+    delta = lb - la
+    if np.any(delta != delta[0]):
+        return False
+    step = int(np.gcd.reduce(np.concatenate([la - la[0], [s for s, n in zip(a.strides[:-1], shape) if n > 1]])
+                             .astype(np.int64)))
+    n, d = int(shape[-1]), int(delta[0])
+    if step == 0:
+        return abs(d) >= n
+    return d % step >= n and d % step + n <= step
+
+
 def topo_stop(root: Expr) -> List[Expr]:
     """Topological order of `root`'s DAG without descending into fold inputs."""
     seen, order = set(), []

@@ -19,7 +19,8 @@ from .affine import AffineMap, AffineSet, Box, evaluate
 from .executor import (Access, Alloc, Arena, ATile, DevScalar, DistATile, DistView, IATile, Instances, Lanes, NeedEager,
                        Plan, Pool, Tile, View, _launch, verify)
 from .ir import IRFunction, Operation, Region
-from .program import CompileError, Expr, LaneOff, LeafSpec, compile_program, is_float, round_host, topo
+from .program import (CompileError, Expr, LaneOff, LeafSpec, compile_program, disjoint, is_float,
+                      rotation_pair_program, rotation_sum, round_host, topo)
 
 # ---------------------------------------------------------------------------
 # op tables (semantics as the reference's: dialects/arith_ops.py:49-135,
@@ -447,6 +448,7 @@ class Executor:
         self.sequential = sequential
         self.eager = sequential
         self.attn_pending = None     # last fused attention launch whose epilogue may still fold in
+        self._last_sum = None            # the last launch, if it stores a sum of two products
         self.pattn_names = set()     # iter_args of the last paged attention loop
         self.mm_pending = None       # last matmul launch whose result store may still fold in
         self.allow_expand = allow_expand and not sequential
@@ -830,7 +832,59 @@ class Executor:
                 raise
             e2 = self._split(e)
             return self._emit_store(e2, dest, depth + 1)
+        sums = None if self.eager else rotation_sum(e, dest)
+        if sums is not None and self._rotation_pair(sums, dest, prog, keep):
+            return
         self.launch("prog", prog, keep + [dest])
+        if sums is not None:
+            self._last_sum = (prog, sums, dest)
+
+    def _rotation_pair(self, sums, dest: LeafSpec, prog, keep) -> bool:
+        """a*d +- c*b stored right after a*b +- c*d of the same tiles (the two
+        halves of a rotary embedding): one launch reads the four tiles once
+        and stores both.  40 heads x 4096 x 128 f16: see ktir_rot.hip for both
+        sides.  Only where neither result may touch what either sum reads and
+        the two results share no element, so that the order of the two stores
+        cannot be seen."""
+        last, launches = self._last_sum, self.plan.launches
+        if last is None or not launches or launches[-1][0] != "prog" or launches[-1][1] is not last[0]:
+            return False
+        first, (op1, dt, leaves1), dest1 = last
+        op2, dt2, leaves2 = sums
+        nd = int(prog.ndim)
+        if dt != dt2 or first.lanes != prog.lanes or first.ndim != nd \
+                or list(first.shape)[:nd] != list(prog.shape)[:nd] or int(prog.shape[nd - 1]) % 8:
+            return False
+        vec = rt.K["KTIR_LEAF_VEC8"]
+        if any(p.n_pf != 4 or list(p.pf_leaf) != [0, 1, 2, 3] or p.n_leaves != 5
+               or any(not p.leaves[i].flags & vec for i in range(5)) for p in (first, prog)):
+            return False
+        L = self.L
+        lanes1 = [x.lane.values(L) for x in leaves1 + [dest1]]
+        lanes2 = [x.lane.values(L) for x in leaves2 + [dest]]
+
+        def slot(k):
+            x = leaves2[k]
+            for i, y in enumerate(leaves1):
+                if (x.ptr, x.dtype, x.strides, x.lo, x.hi) == (y.ptr, y.dtype, y.strides, y.lo, y.hi) \
+                        and np.array_equal(lanes1[i], lanes2[k]):
+                    return i
+            return -1
+
+        at = [slot(k) for k in range(4)]
+        # each product of this sum has one factor from each product of the first
+        if sorted(at) != [0, 1, 2, 3] or {i // 2 for i in at[:2]} != {0, 1}:
+            return False
+        es = rt.ELEM_BYTES[dt]
+        for d in (dest1, dest):
+            if any(d.ptr + d.lo * es < x.ptr + x.hi * es and x.ptr + x.lo * es < d.ptr + d.hi * es for x in leaves1):
+                return False
+        if not disjoint(dest1, lanes1[4], dest, lanes2[4], tuple(int(n) for n in list(prog.shape)[:nd])):
+            return False
+        pair = rotation_pair_program(first, prog, op1, op2, at)
+        launches[-1] = ("prog", pair, tuple(launches[-1][2]) + tuple(keep) + (dest,))
+        self._last_sum = None
+        return True
 
     def _pattn_finalise(self, e: Expr, dest: LeafSpec) -> bool:
         """The store right after a paged attention launch of
