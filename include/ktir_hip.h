@@ -458,16 +458,17 @@ typedef struct ktir_pattn {
   uint64_t out_ptr, out_base;          /* out_base: const int64_t* [lanes] */
   int64_t out_grp, out_gstride, out_row, out_lo, out_hi;
   int32_t out_dtype, out_pad;
-  /* optional (items 0: not used): the lanes as items, const int32_t* [2 *
-   * n_items] {first, count} into item_lanes (const int32_t* [lanes], every
-   * lane in one item).  An item's lanes have equal k_base, v_base, tbl_pos,
-   * trips and kpos0 and at most 32 rows together.  With pages of 16 keys, one
-   * 16-bit operand type and 64 or 128 columns, `splits` workgroups share an
+  /* optional (items 0: not used): the lanes as items, int64_t [8 * n_items]
+   * {first | count << 32, trips, k_base, v_base, tbl_pos, kpos0, 0, 0} with
+   * first and count a range of item_lanes (const int32_t* [lanes], every lane
+   * in one item).  An item's lanes have these bases in common and at most 32
+   * rows together.  With pages of 16 keys, one 16-bit operand type and 64 or
+   * 128 columns, `splits` workgroups of `waves` (4 or 8) wavefronts share an
    * item's keys; for splits > 1 ws holds n_items * splits * (64 + 32 * D)
    * floats.  Other launches ignore the items. */
   uint64_t items, item_lanes, ws;
   int64_t n_items;
-  int32_t splits, pad2;
+  int32_t splits, waves;
 } ktir_pattn_t;
 int ktir_launch_paged_attention(const ktir_pattn_t* d);
 

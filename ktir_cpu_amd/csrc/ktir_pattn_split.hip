@@ -6,9 +6,9 @@
 // A lane has few rows (block_q tokens x the query heads of one KV head), and
 // every lane of a KV head reads the same pages.  The host groups lanes with
 // equal K and V offsets, table position, trip count and key positions into
-// items of at most 32 rows.  A workgroup is four wavefronts on one item, each
-// with the item's 32 rows and its own pages: pairs of pages (32 keys) k, k + 4 S,
-// k + 8 S, ... of the S workgroups that share the item.  So the wavefronts share
+// items of at most 32 rows.  A workgroup is W = 4 or 8 wavefronts on one item, each
+// with the item's 32 rows and its own pages: pairs of pages (32 keys) k, k + W S,
+// k + 2 W S, ... of the S workgroups that share the item.  So the wavefronts share
 // nothing until the end, run without barriers, and a single query row of a
 // decode step keeps the whole chip busy.  Per pair, as in ktir_attn_tile.hip:
 //   S^T = K Q^T (32 x 32 x 16 MFMA), masked and scaled in f32,
@@ -19,10 +19,15 @@
 // (whose f32 kernel holds P exactly).
 // Pages move HBM -> LDS (buffer_load ... lds) into the wavefront's own 16 KB
 // (128 columns): the next pair's K while this pair's softmax and P V run, its V
-// while the next scores are computed; two workgroups share a CU.
-// At the end the four states are merged through LDS; with S > 1 the merged
+// while the next scores are computed; two workgroups of four (or one of eight) share a CU.
+// At the end the W states are merged through LDS; with S > 1 the merged
 // state goes to a workspace and a second kernel merges the S of them.  A merge
 // weighs each state by exp(m_i - m), 0 for keys that were all masked.
+//
+// Bound: latency.  A token after 8191 with 8 KV heads of 128 f16 columns reads 34 MB
+// (6 us at a large copy's rate) in 11.6 us, of which about 4 are the chain item ->
+// table -> first page, and 5.4 us go to the merge: 18.0 us in all, 343 us on one
+// wavefront per lane; 256 tokens after 1024: 23.7 us with the copy of Q, 58.5 us.
 //
 // The loop's step is a page, so a row whose first page is masked whole is NaN
 // (exp(-inf - (-inf))) whatever follows; the wavefront that has page 0 makes it so.
@@ -33,7 +38,7 @@
 
 namespace ktir {
 
-constexpr int PS_ROWS = 32, PS_KEYS = 32, PS_WAVES = 4;
+constexpr int PS_ROWS = 32, PS_KEYS = 32;
 
 // slot permutation of a key row's 16-byte chunks (as att_swz in ktir_attn_tile.hip)
 template <int D>
@@ -76,14 +81,15 @@ __device__ __forceinline__ void ps_wait() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-// 16 keys x D columns of such a page into LDS rows row0 .. + 16
+// 16 keys x D columns of such a page into LDS rows row0 .. + 16; zeros (loads
+// past the end of a buffer of no bytes) if it is not `there`
 template <int D>
-__device__ __forceinline__ void ps_dma(uint64_t ptr, int64_t e0, int64_t row, uint32_t lds, int row0, int l) {
+__device__ __forceinline__ void ps_dma(uint64_t ptr, int64_t e0, int64_t row, bool there, uint32_t lds, int row0, int l) {
   constexpr int CH = D / 8, RB = 512 / D;      // chunks per row, rows per 1 KB
   const uint64_t a = ptr + 2 * (uint64_t)e0;
   const u32x4_t rs = {(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)a),
                       (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(a >> 32) & 0xffffu),
-                      (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)((15 * row + D) * 2)), 0x00020000u};
+                      (uint32_t)__builtin_amdgcn_readfirstlane(there ? (uint32_t)((15 * row + D) * 2) : 0u), 0x00020000u};
   const int r = l / CH, c = l % CH;
 #pragma unroll
   for (int i = 0; i < 16 / RB; ++i)
@@ -124,29 +130,46 @@ __device__ __forceinline__ void ps_split(const float* x, uint32_t (&t)[PARTS][2]
 // the weight of a state with maximum mi in one with maximum m >= mi
 __device__ __forceinline__ float ps_weight(float mi, float m) { return mi == -__builtin_inff() ? 0.f : exp_f(__fsub_rn(mi, m)); }
 
-// columns 16 q .. + 16 of row `row` of an item: acc (relative to m), l and m
+// where row `row` of an item goes (read before the work that ps_out waits for)
+struct PsDst {
+  int64_t lane, out;
+  int r, trips;
+  bool live;
+};
+
+__device__ __forceinline__ PsDst ps_dst(const ktir_pattn_t& d, const int32_t* lanes, int nl, int row) {
+  const int M = (int)d.M, li = row / M;
+  PsDst t;
+  t.r = row - li * M;
+  t.live = li < nl;
+  t.lane = lanes[t.live ? li : 0];
+  t.trips = ((const int32_t*)d.trips)[t.lane];
+  t.out = d.out_ptr ? ((const int64_t*)d.out_base)[t.lane] + (int64_t)(t.r / d.out_grp) * d.out_gstride +
+                          (int64_t)(t.r % d.out_grp) * d.out_row
+                    : 0;
+  return t;
+}
+
+// columns 16 q .. + 16 of such a row: acc (relative to m), l and m
 // into the launch's outputs, and acc / l into the fused store
 template <int D>
-__device__ __forceinline__ void ps_out(const ktir_pattn_t& d, const int32_t* lanes, int nl, int row, int q, const float (&acc)[16],
-                                       float l, float m) {
-  const int M = (int)d.M, li = row / M, r = row - li * M;
-  if (li >= nl) return;
-  const int64_t lane = lanes[li];
-  if (((const int32_t*)d.trips)[lane] > 0) l = __fadd_rn(l, __fmul_rn(d.l0, ps_weight(d.m0, m)));
+__device__ __forceinline__ void ps_out(const ktir_pattn_t& d, const PsDst& t, int q, const float (&acc)[16], float l, float m) {
+  if (!t.live) return;
+  const int64_t row = t.lane * d.M + t.r;
+  if (t.trips > 0) l = __fadd_rn(l, __fmul_rn(d.l0, ps_weight(d.m0, m)));
   else l = d.l0, m = d.m0;
   if (q == 0) {
-    ((float*)d.m_out)[lane * M + r] = m;
-    ((float*)d.l_out)[lane * M + r] = l;
+    ((float*)d.m_out)[row] = m;
+    ((float*)d.l_out)[row] = l;
   }
   if (d.acc_out) {
-    float4* a = (float4*)((float*)d.acc_out + (lane * M + r) * D + 16 * q);
+    float4* a = (float4*)((float*)d.acc_out + row * D + 16 * q);
 #pragma unroll
     for (int k = 0; k < 4; ++k) a[k] = make_float4(acc[4 * k], acc[4 * k + 1], acc[4 * k + 2], acc[4 * k + 3]);
   }
   if (!d.out_ptr) return;
   // the loop's finalisation: acc / l rounded to the output's dtype
-  const int64_t e0 = ((const int64_t*)d.out_base)[lane] + (int64_t)(r / d.out_grp) * d.out_gstride +
-                     (int64_t)(r % d.out_grp) * d.out_row + 16 * q;
+  const int64_t e0 = t.out + 16 * q;
   float v[16];
 #pragma unroll
   for (int k = 0; k < 16; ++k) v[k] = __fdiv_rn(acc[k], l);
@@ -167,23 +190,27 @@ __device__ __forceinline__ void ps_out(const ktir_pattn_t& d, const int32_t* lan
     if (e0 + k >= d.out_lo && e0 + k < d.out_hi) store_elem(d.out_ptr, e0 + k, d.out_dtype, v[k]);
 }
 
-template <bool BF16, int D, int PARTS>
-__global__ __launch_bounds__(64 * PS_WAVES, 2) void pattn_split(const ktir_pattn_t d, int vec, int* err) {
+// one item, as the host lays it out
+struct __attribute__((packed, aligned(64))) PsItem {
+  int32_t first, count;                        // its lanes: item_lanes[first ..]
+  int64_t trips, k_base, v_base, tbl_pos, kpos0;
+};
+
+template <bool BF16, int D, int PARTS, int W>
+__global__ __launch_bounds__(64 * W, 2) void pattn_split(const ktir_pattn_t d, int vec, int* err) {
   constexpr int DS = D / 16, DT = D / 32;
   // per wavefront K then V, 32 keys x D each; at the end its O^T
-  __shared__ __align__(16) uint16_t Ks[PS_WAVES][PS_KEYS * D];
-  __shared__ __align__(16) uint16_t Vs[PS_WAVES][PS_KEYS * D];
-  __shared__ float ms[PS_WAVES][PS_ROWS], ls[PS_WAVES][PS_ROWS];
+  __shared__ __align__(16) uint16_t Ks[W][PS_KEYS * D];
+  __shared__ __align__(16) uint16_t Vs[W][PS_KEYS * D];
+  __shared__ float ms[W][PS_ROWS], ls[W][PS_ROWS];
   const int tid = threadIdx.x, l = tid & 63, h = l >> 5, r32 = l & 31;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int S = d.splits;
   const int item = blockIdx.x / S, part = blockIdx.x - item * S;
-  const int first = uni(((const int32_t*)d.items)[2 * item]), nl = uni(((const int32_t*)d.items)[2 * item + 1]);
+  const PsItem* it = (const PsItem*)d.items + item;
+  const int first = uni(it->first), nl = uni(it->count), trips = uni((int)it->trips);
+  const int64_t kb = uni(it->k_base), vb = uni(it->v_base), tp = uni(it->tbl_pos), kp0 = uni(it->kpos0);
   const int32_t* lanes = (const int32_t*)d.item_lanes + first;
-  const int64_t lane0 = uni(lanes[0]);         // whose pages (every lane of the item reads them)
-  const int trips = uni(((const int32_t*)d.trips)[lane0]);
-  const int64_t kb = uni(((const int64_t*)d.k_base)[lane0]), vb = uni(((const int64_t*)d.v_base)[lane0]);
-  const int64_t tp = uni(((const int64_t*)d.tbl_pos)[lane0]), kp0 = uni(((const int64_t*)d.kpos0)[lane0]);
   uint16_t* K = Ks[w];
   uint16_t* V = Vs[w];
   const uint32_t k_lds = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint16_t*)K);
@@ -228,7 +255,7 @@ __global__ __launch_bounds__(64 * PS_WAVES, 2) void pattn_split(const ktir_pattn
   }
   // pairs of pages first_pair, first_pair + stride, ...; the table's entries of
   // 32 of them at a time, entry 2 k + p of pair k in lane 2 k + p
-  const int first_pair = part * PS_WAVES + w, stride = S * PS_WAVES, n_pairs = (trips + 1) >> 1;
+  const int first_pair = part * W + w, stride = S * W, n_pairs = (trips + 1) >> 1;
   bool bad = false;
   auto entries = [&](int k0) -> int64_t {
     const int j = 2 * (first_pair + (k0 + (l >> 1)) * stride) + (l & 1);
@@ -244,12 +271,14 @@ __global__ __launch_bounds__(64 * PS_WAVES, 2) void pattn_split(const ktir_pattn
     const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)table, src), hi = __builtin_amdgcn_readlane((uint32_t)(table >> 32), src);
     return (int64_t)(((uint64_t)hi << 32) | lo);
   };
-  // K or V of pair k, both pages by DMA (pages known to lie in their windows)
+  // K or V of pair k, both pages by DMA (pages known to lie in their windows;
+  // the second one of an odd loop's last pair is missing: zeros)
   auto dma = [&](int k, bool v) __attribute__((always_inline)) {
 #pragma unroll
     for (int p = 0; p < 2; ++p) {
-      if (!v) ps_dma<D>(d.k_ptr, kb + page_of(k, p) * d.k_page, d.k_row, k_lds, 16 * p, l);
-      else ps_dma<D>(d.v_ptr, vb + page_of(k, p) * d.v_page, d.v_row, v_lds, 16 * p, l);
+      const bool there = p == 0 || 2 * (first_pair + k * stride) + 1 < trips;
+      if (!v) ps_dma<D>(d.k_ptr, kb + page_of(k, p) * d.k_page, d.k_row, there, k_lds, 16 * p, l);
+      else ps_dma<D>(d.v_ptr, vb + page_of(k, p) * d.v_page, d.v_row, there, v_lds, 16 * p, l);
     }
   };
   // element by element, zeros outside the windows and for the missing second
@@ -388,11 +417,11 @@ __global__ __launch_bounds__(64 * PS_WAVES, 2) void pattn_split(const ktir_pattn
   for (int c0 = 0; c0 < mine; c0 += 32) {
     if (c0) table = entries(c0);
     const int c1 = c0 + 32 < mine ? c0 + 32 : mine;
-    // pages of these pairs that are there and wholly in their windows
+    // pages of these pairs that are wholly in their windows, or missing
     const int my_pair = c0 + (l >> 1);
     const int64_t ke = kb + table * d.k_page, ve = vb + table * d.v_page;
-    const bool ok = my_pair >= c1 || (vec && 2 * (first_pair + my_pair * stride) + (l & 1) < trips &&
-                                      ps_fast<D>(ke, d.k_row, d.k_lo, d.k_hi) && ps_fast<D>(ve, d.v_row, d.v_lo, d.v_hi));
+    const bool ok = my_pair >= c1 || (vec && (2 * (first_pair + my_pair * stride) + (l & 1) >= trips ||
+                                              (ps_fast<D>(ke, d.k_row, d.k_lo, d.k_hi) && ps_fast<D>(ve, d.v_row, d.v_lo, d.v_hi))));
     const uint64_t ballot = __builtin_amdgcn_ballot_w64(!ok);
     // the pairs before the first that is not
     const int nf = ballot ? __builtin_ctzll(ballot) >> 1 : c1 - c0;
@@ -433,25 +462,26 @@ __global__ __launch_bounds__(64 * PS_WAVES, 2) void pattn_split(const ktir_pattn
     ms[w][r32] = m;
     ls[w][r32] = lsum;
   }
-  __syncthreads();
   // row tid % 32, columns 16 q .. + 16
   const int row = tid & 31;
+  const PsDst dst = ps_dst(d, lanes, nl, row);
+  __syncthreads();
   float mm = ms[0][row];
 #pragma unroll
-  for (int v = 1; v < PS_WAVES; ++v) mm = fmax_nan(mm, ms[v][row]);
-  float wt[PS_WAVES], lm = 0.f;
+  for (int v = 1; v < W; ++v) mm = fmax_nan(mm, ms[v][row]);
+  float wt[W], lm = 0.f;
 #pragma unroll
-  for (int v = 0; v < PS_WAVES; ++v) {
+  for (int v = 0; v < W; ++v) {
     wt[v] = ps_weight(ms[v][row], mm);
     lm = __fadd_rn(lm, __fmul_rn(ls[v][row], wt[v]));
   }
-  for (int q = tid >> 5; q < D / 16; q += 8) {
+  for (int q = tid >> 5; q < D / 16; q += 2 * W) {
     float acc[16];
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
       float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
-      for (int v = 0; v < PS_WAVES; ++v) {
+      for (int v = 0; v < W; ++v) {
         const float4 x = grp(v, 4 * q + k)[row];
         a.x = __fadd_rn(a.x, __fmul_rn(x.x, wt[v]));
         a.y = __fadd_rn(a.y, __fmul_rn(x.y, wt[v]));
@@ -464,8 +494,8 @@ __global__ __launch_bounds__(64 * PS_WAVES, 2) void pattn_split(const ktir_pattn
       acc[4 * k + 3] = a.w;
     }
     if (S == 1) {
-      ps_out<D>(d, lanes, nl, row, q, acc, lm, mm);
-    } else if (row / M < nl) {
+      ps_out<D>(d, dst, q, acc, lm, mm);
+    } else if (dst.live) {
       // workspace: per workgroup m [32], l [32], then O as the LDS holds it
       float* ws = (float*)d.ws + (int64_t)blockIdx.x * (64 + PS_ROWS * D);
       if (q == 0) {
@@ -479,60 +509,107 @@ __global__ __launch_bounds__(64 * PS_WAVES, 2) void pattn_split(const ktir_pattn
   }
 }
 
-// the S states of an item, one workgroup per item and 16 columns (four threads a row)
+// The S states of an item, one workgroup per item and 16 columns.  Bound: a
+// chain of memory latencies, so as many states as there are threads for are
+// loaded at once: the item's live rows (to a power of two) side by side, G
+// threads with a state each on every row, PM_U states per thread before anything
+// waits for one.
+constexpr int PM_THREADS = 256, PM_U = 4;
+
 template <int D>
-__global__ __launch_bounds__(128) void pattn_merge(const ktir_pattn_t d) {
+__global__ __launch_bounds__(PM_THREADS) void pattn_merge(const ktir_pattn_t d) {
   constexpr int SZ = 64 + PS_ROWS * D;
   const int S = d.splits;
   const int item = blockIdx.x / (D / 16), q = blockIdx.x % (D / 16);
-  const int first = uni(((const int32_t*)d.items)[2 * item]), nl = uni(((const int32_t*)d.items)[2 * item + 1]);
+  const PsItem* it = (const PsItem*)d.items + item;
+  const int first = uni(it->first), nl = uni(it->count);
   const int32_t* lanes = (const int32_t*)d.item_lanes + first;
   const float* ws = (const float*)d.ws + (int64_t)item * S * SZ;
-  __shared__ float4 part[4][4][PS_ROWS];
-  __shared__ float lpart[4][PS_ROWS], mpart[4][PS_ROWS];
-  const int row = threadIdx.x & 31, t = threadIdx.x >> 5;   // states t, t + 4, ...
-  const bool live = row / (int)d.M < nl;
-  float m = -__builtin_inff();
+  __shared__ float4 part[4][PM_THREADS];
+  __shared__ float lpart[PM_THREADS], mpart[PM_THREADS];
+  const int tid = threadIdx.x, rows = nl * (int)d.M;        // 1 .. 32
+  const int lg = rows > 1 ? 32 - __builtin_clz(rows - 1) : 0;
+  const int row = tid & ((1 << lg) - 1), t = tid >> lg, G = PM_THREADS >> lg;   // states t, t + G, ...
+  const bool live = row < rows;
+  const float ninf = -__builtin_inff();
+  float mu[PM_U], lu[PM_U];
+  float4 x[PM_U][4];
+#pragma unroll
+  for (int u = 0; u < PM_U; ++u) {
+    const int s = t + u * G;
+    const bool on = live && s < S;
+    const float* p = ws + (int64_t)(on ? s : 0) * SZ;
+    mu[u] = on ? p[row] : ninf;
+    lu[u] = on ? p[32 + row] : 0.f;
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      x[u][k] = on ? *(const float4*)(p + 64 + ((4 * q + k) * 32 + row) * 4) : make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+  const PsDst dst = ps_dst(d, lanes, nl, row);
+  float m = mu[0];
+#pragma unroll
+  for (int u = 1; u < PM_U; ++u) m = fmax_nan(m, mu[u]);
   if (live)
-    for (int s = t; s < S; s += 4) m = fmax_nan(m, ws[(int64_t)s * SZ + row]);
-  mpart[t][row] = m;
+    for (int s = t + PM_U * G; s < S; s += G) m = fmax_nan(m, ws[(int64_t)s * SZ + row]);
+  mpart[tid] = m;
+  for (int off = G >> 1; off; off >>= 1) {
+    __syncthreads();
+    if (t < off) mpart[tid] = fmax_nan(mpart[tid], mpart[tid + (off << lg)]);
+  }
   __syncthreads();
-  m = fmax_nan(fmax_nan(mpart[0][row], mpart[1][row]), fmax_nan(mpart[2][row], mpart[3][row]));
+  m = mpart[row];
   float l = 0.f;
   float4 a[4];
 #pragma unroll
   for (int k = 0; k < 4; ++k) a[k] = make_float4(0.f, 0.f, 0.f, 0.f);
-  if (live) {
-    for (int s = t; s < S; s += 4) {
+  auto add = [&](float ms, float ls, const float4 (&v)[4]) __attribute__((always_inline)) {
+    const float w = ps_weight(ms, m);
+    l = __fadd_rn(l, __fmul_rn(ls, w));
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      a[k].x = __fadd_rn(a[k].x, __fmul_rn(v[k].x, w));
+      a[k].y = __fadd_rn(a[k].y, __fmul_rn(v[k].y, w));
+      a[k].z = __fadd_rn(a[k].z, __fmul_rn(v[k].z, w));
+      a[k].w = __fadd_rn(a[k].w, __fmul_rn(v[k].w, w));
+    }
+  };
+#pragma unroll
+  for (int u = 0; u < PM_U; ++u) add(mu[u], lu[u], x[u]);
+  if (live)
+    for (int s = t + PM_U * G; s < S; s += G) {
       const float* p = ws + (int64_t)s * SZ;
-      const float w = ps_weight(p[row], m);
-      l = __fadd_rn(l, __fmul_rn(p[32 + row], w));
+      float4 v[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) v[k] = *(const float4*)(p + 64 + ((4 * q + k) * 32 + row) * 4);
+      add(p[row], p[32 + row], v);
+    }
+  lpart[tid] = l;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) part[k][tid] = a[k];
+  for (int off = G >> 1; off; off >>= 1) {
+    __syncthreads();
+    if (t < off) {
+      const int o = tid + (off << lg);
+      l = __fadd_rn(l, lpart[o]);
+      lpart[tid] = l;
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
-        const float4 x = *(const float4*)(p + 64 + ((4 * q + k) * 32 + row) * 4);
-        a[k].x = __fadd_rn(a[k].x, __fmul_rn(x.x, w));
-        a[k].y = __fadd_rn(a[k].y, __fmul_rn(x.y, w));
-        a[k].z = __fadd_rn(a[k].z, __fmul_rn(x.z, w));
-        a[k].w = __fadd_rn(a[k].w, __fmul_rn(x.w, w));
+        const float4 y = part[k][o];
+        a[k] = make_float4(__fadd_rn(a[k].x, y.x), __fadd_rn(a[k].y, y.y), __fadd_rn(a[k].z, y.z), __fadd_rn(a[k].w, y.w));
+        part[k][tid] = a[k];
       }
     }
   }
-  lpart[t][row] = l;
-#pragma unroll
-  for (int k = 0; k < 4; ++k) part[t][k][row] = a[k];
-  __syncthreads();
-  if (t != 0 || !live) return;
-  l = __fadd_rn(__fadd_rn(lpart[0][row], lpart[1][row]), __fadd_rn(lpart[2][row], lpart[3][row]));
+  if (t != 0) return;
   float acc[16];
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
-    const float4 x = part[0][k][row], y = part[1][k][row], z = part[2][k][row], u = part[3][k][row];
-    acc[4 * k] = __fadd_rn(__fadd_rn(x.x, y.x), __fadd_rn(z.x, u.x));
-    acc[4 * k + 1] = __fadd_rn(__fadd_rn(x.y, y.y), __fadd_rn(z.y, u.y));
-    acc[4 * k + 2] = __fadd_rn(__fadd_rn(x.z, y.z), __fadd_rn(z.z, u.z));
-    acc[4 * k + 3] = __fadd_rn(__fadd_rn(x.w, y.w), __fadd_rn(z.w, u.w));
+    acc[4 * k] = a[k].x;
+    acc[4 * k + 1] = a[k].y;
+    acc[4 * k + 2] = a[k].z;
+    acc[4 * k + 3] = a[k].w;
   }
-  ps_out<D>(d, lanes, nl, row, q, acc, l, m);
+  ps_out<D>(d, dst, q, acc, l, m);
 }
 
 // True when launched: the caller gave items (at most 32 rows of lanes that read
@@ -540,6 +617,7 @@ __global__ __launch_bounds__(128) void pattn_merge(const ktir_pattn_t d) {
 // row maxima that start at -inf.
 bool launch_pattn_split(const ktir_pattn_t* d) {
   if (!d->items || !d->item_lanes || d->n_items < 1 || d->splits < 1 || (d->splits > 1 && !d->ws)) return false;
+  if (d->waves != 4 && d->waves != 8) return false;
   if (d->n_items * d->splits > INT_MAX || d->n_items * (d->D / 16) > INT_MAX) return false;
   if (d->q_dtype != d->kv_dtype || (d->kv_dtype != KTIR_F16 && d->kv_dtype != KTIR_BF16)) return false;
   if (d->N != 16 || d->M > PS_ROWS || (d->D != 64 && d->D != 128) || d->m0 != -__builtin_inff()) return false;
@@ -548,19 +626,24 @@ bool launch_pattn_split(const ktir_pattn_t* d) {
   const int vec = !((d->q_ptr | d->k_ptr | d->v_ptr) & 15) && !((d->q_row | d->k_row | d->v_row | d->k_page | d->v_page) & 7);
   const bool bf = d->kv_dtype == KTIR_BF16, more = d->M > 16;
   const dim3 grid((unsigned)(d->n_items * d->splits));
-  auto go = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(64 * PS_WAVES), 0, stream(), *d, vec, device_error_flag()); };
-  auto by = [&](auto f1, auto f2, auto b2, auto b3) {
-    if (bf) more ? go(b3) : go(b2);
-    else more ? go(f2) : go(f1);
+  auto go = [&](auto kern, int waves) {
+    hipLaunchKernelGGL(kern, grid, dim3(64 * waves), 0, stream(), *d, vec, device_error_flag());
   };
-  if (d->D == 64)
-    by(pattn_split<false, 64, 1>, pattn_split<false, 64, 2>, pattn_split<true, 64, 2>, pattn_split<true, 64, 3>);
-  else
-    by(pattn_split<false, 128, 1>, pattn_split<false, 128, 2>, pattn_split<true, 128, 2>, pattn_split<true, 128, 3>);
+  auto by = [&](auto dim, auto waves) {
+    constexpr int D = decltype(dim)::value, W = decltype(waves)::value;
+    if (bf) more ? go(pattn_split<true, D, 3, W>, W) : go(pattn_split<true, D, 2, W>, W);
+    else more ? go(pattn_split<false, D, 2, W>, W) : go(pattn_split<false, D, 1, W>, W);
+  };
+  const std::integral_constant<int, 64> d64;
+  const std::integral_constant<int, 128> d128;
+  const std::integral_constant<int, 4> w4;
+  const std::integral_constant<int, 8> w8;
+  if (d->D == 64) d->waves == 8 ? by(d64, w8) : by(d64, w4);
+  else d->waves == 8 ? by(d128, w8) : by(d128, w4);
   if (d->splits > 1) {
     const dim3 mg((unsigned)(d->n_items * (d->D / 16)));
-    if (d->D == 64) hipLaunchKernelGGL(pattn_merge<64>, mg, dim3(128), 0, stream(), *d);
-    else hipLaunchKernelGGL(pattn_merge<128>, mg, dim3(128), 0, stream(), *d);
+    if (d->D == 64) hipLaunchKernelGGL(pattn_merge<64>, mg, dim3(PM_THREADS), 0, stream(), *d);
+    else hipLaunchKernelGGL(pattn_merge<128>, mg, dim3(PM_THREADS), 0, stream(), *d);
   }
   return true;
 }

@@ -1041,6 +1041,7 @@ def _paged_attention(ex, trips, tm1, q, probes, peeled, l0, slots, mask, names):
         lanes, items = _pattn_items(trips, k[1], v[1], k[5], ck0.astype(np.int64), M)
         d.item_lanes, d.items, d.n_items = up(lanes), up(items), len(items)
         d.splits = _pattn_splits(len(items), int(trips.max()))
+        d.waves = _pattn_waves(len(items), d.splits, int(trips.max()))
         if d.splits > 1:
             ws = ex.pool.temp(len(items) * d.splits * (64 + 32 * D) * 4)
             keep.append(ws)
@@ -1062,8 +1063,9 @@ def _paged_attention(ex, trips, tm1, q, probes, peeled, l0, slots, mask, names):
 def _pattn_items(trips, k_base, v_base, tbl_pos, kpos0, M, rows=32):
     """Lanes that read the same pages (equal K and V offsets, table position,
     trip count and key positions) in items of at most `rows` query rows: (lane
-    numbers item by item, {first, count} of every item).  The items of one
-    stream of pages go to one XCD."""
+    numbers item by item, {first | count << 32, trips, K, V, table, key
+    position, 0, 0} of every item).  The items of one stream of pages go to one
+    XCD."""
     _, grp = np.unique(np.stack([k_base, v_base, tbl_pos, kpos0, trips], 1), axis=0, return_inverse=True)
     grp = grp.reshape(-1)
     per = max(1, rows // M)
@@ -1075,20 +1077,32 @@ def _pattn_items(trips, k_base, v_base, tbl_pos, kpos0, M, rows=32):
     # the items in the order of workgroups, then the lanes in that of the items
     seq = _xcd_order(trips[first], k_base[first], v_base[first])
     lanes = np.concatenate([order[cut[i]:cut[i] + count[i]] for i in seq]) if len(seq) else np.zeros(0)
-    items = np.zeros((len(seq), 2), np.int32)
-    items[:, 1] = count[seq]
-    items[1:, 0] = np.cumsum(items[:-1, 1])
+    items = np.zeros((len(seq), 8), np.int64)
+    n, lead = count[seq].astype(np.int64), first[seq]
+    items[:, 0] = (np.cumsum(n) - n) | n << 32
+    for i, a in enumerate((trips, k_base, v_base, tbl_pos, kpos0)):
+        items[:, 1 + i] = a[lead]
     return lanes.astype(np.int32), items
 
 
 def _pattn_splits(n_items, trips, cus=256):
-    """Workgroups (of four wavefronts) that share an item's pages: one where the
-    items alone give most CUs a workgroup (the merge of several costs a launch
-    and a pass over their f32 states), else enough for one per CU, but at least
-    two pairs of pages for a wavefront."""
-    if 4 * n_items >= 3 * cus:
-        return 1
-    return max(1, min(-(-cus // n_items), trips // 16))
+    """Workgroups of four wavefronts that share an item's pages: enough for one
+    per CU, with a pair of pages for every wavefront, where that saves at least
+    2.5 pairs' time over one workgroup of eight wavefronts, else one.  A pair
+    takes a wavefront about 1.4 us; the states of several workgroups cost a
+    launch, a pass over them and about 4 us.  8 KV heads, one token after 500 /
+    1000 / 4000: one workgroup 13.4 / 16.8 / 33 us, the most that have a pair
+    each 15.3 / 15.3 / 15.3 us."""
+    s = max(1, min(-(-cus // n_items), trips // 8))
+    return s if trips / 16 - trips / (8 * s) >= 2.5 else 1
+
+
+def _pattn_waves(n_items, splits, trips, cus=256):
+    """Wavefronts of a workgroup: eight where the only workgroup of a CU has
+    enough pages for them (256 tokens after 1024: 25.2 us, with four 27.2; after
+    8191: 72 us, with four 97), four where it has few (one token after 500: 13.4
+    us, with eight 13.8), shares an item with others or shares its CU."""
+    return 8 if splits == 1 and n_items <= cus and trips >= 48 else 4
 
 
 def _plain_ld(e, ptr, shape, inner):

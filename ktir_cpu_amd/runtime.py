@@ -135,7 +135,7 @@ class PATTN(C.Structure):
                 ("out_gstride", C.c_int64), ("out_row", C.c_int64), ("out_lo", C.c_int64), ("out_hi", C.c_int64),
                 ("out_dtype", C.c_int32), ("out_pad", C.c_int32),
                 ("items", C.c_uint64), ("item_lanes", C.c_uint64), ("ws", C.c_uint64), ("n_items", C.c_int64),
-                ("splits", C.c_int32), ("pad2", C.c_int32)]
+                ("splits", C.c_int32), ("waves", C.c_int32)]
 
 
 class KTIRDeviceError(RuntimeError):

@@ -91,10 +91,14 @@ PA_SPLIT = [
 ]
 
 
+@pytest.mark.parametrize("waves", [4, 8])
 @pytest.mark.parametrize("dt", ["f16", "bf16"])
 @pytest.mark.parametrize("gen,args,splits", [c[1:] for c in PA_SPLIT], ids=[c[0] for c in PA_SPLIT])
-def test_paged_attention_split_keys_within_tolerance(gen, args, splits, dt):
+def test_paged_attention_split_keys_within_tolerance(gen, args, splits, dt, waves, monkeypatch):
+    from ktir_cpu_amd import fusion
     from oracle.interp import bf16_bits
+    monkeypatch.setattr(fusion, "_pattn_splits", lambda *a: splits)
+    monkeypatch.setattr(fusion, "_pattn_waves", lambda *a: waves)
     inp = {k: v for k, v in gen.items() if k != "block_q"}
     kw = paged_inputs(seed=5, **inp)
     if dt == "bf16":
@@ -106,17 +110,35 @@ def test_paged_attention_split_keys_within_tolerance(gen, args, splits, dt):
     assert d.splits == splits and d.n_items > 0 and d.acc_out == 0
 
 
-def test_paged_attention_many_pages_per_wavefront(monkeypatch):
+@pytest.mark.parametrize("waves,pages", [(4, 299), (8, 547)])
+def test_paged_attention_many_pages_per_wavefront(waves, pages, monkeypatch):
     """More than 32 pairs of pages for a wavefront (the table is read 64
     entries at a time), one page of them past the cache."""
     from ktir_cpu_amd import fusion
     monkeypatch.setattr(fusion, "_pattn_splits", lambda *a: 1)
-    gen = dict(tokens=1, q_heads=8, kv_heads=2, block_q=1, blocks=320, max_pages=300)
-    kw = paged_inputs(tokens=1, q_heads=8, kv_heads=2, blocks=320, max_pages=300, seed=9)
-    kw["block_tables_ptr"][0, 211] = 320 + 3
+    monkeypatch.setattr(fusion, "_pattn_waves", lambda *a: waves)
+    size = dict(blocks=pages + 21, max_pages=pages + 1)
+    gen = dict(tokens=1, q_heads=8, kv_heads=2, block_q=1, **size)
+    kw = paged_inputs(tokens=1, q_heads=8, kv_heads=2, seed=9, **size)
+    kw["block_tables_ptr"][0, 211] = size["blocks"] + 3
     got, ref, plan = _both(configs.paged_attention(**gen), PA_FN,
-                           dict(kw, **dict(PA_ARGS, num_tiles=299, context_len=4770)), "output_ptr")
+                           dict(kw, **dict(PA_ARGS, num_tiles=pages, context_len=16 * pages - 14)), "output_ptr")
     np.testing.assert_allclose(got.astype(np.float32), ref.astype(np.float32), rtol=1e-2, atol=1e-3)
+
+
+@pytest.mark.parametrize("splits,rows", [(2, 4), (37, 4), (150, 4), (9, 32), (40, 32)])
+def test_paged_attention_many_states_merged(splits, rows, monkeypatch):
+    """States of 2 to 150 workgroups (some of them without a page), for 4 and
+    32 live rows: one, and several, per thread of the merge."""
+    from ktir_cpu_amd import fusion
+    monkeypatch.setattr(fusion, "_pattn_splits", lambda *a: splits)
+    tok = 1 if rows == 4 else 8
+    gen = dict(tokens=tok, block_q=tok, blocks=260, max_pages=256)
+    kw = paged_inputs(tokens=tok, blocks=260, max_pages=256, seed=10)
+    got, ref, plan = _both(configs.paged_attention(**gen), PA_FN,
+                           dict(kw, **dict(PA_ARGS, num_tiles=255, context_len=4071)), "output_ptr")
+    np.testing.assert_allclose(got.astype(np.float32), ref.astype(np.float32), rtol=1e-2, atol=1e-3)
+    assert plan.launches[-1][1].splits == splits
 
 
 @pytest.mark.parametrize("num_tiles", [2, 5])
