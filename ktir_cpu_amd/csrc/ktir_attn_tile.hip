@@ -23,8 +23,11 @@
 // instructions per wavefront and takes 32 KB of LDS, so several workgroups
 // share a CU and one's softmax runs under another's MFMAs.  The vector
 // instructions bound it (the exact split of P takes as many as the
-// exponentials).  Full attention of 16 heads, 2048 x 64, f16, 64 x 64 tiles:
-// 40 us (430 TFLOP/s) against 43.4 ms for the loop's about 450 launches.
+// exponentials).  Where no CU has a second workgroup, the key tiles go to two
+// groups of four wavefronts, whose states meet in LDS at the end.  Full attention
+// of 2048 x 64, f16, 64 x 64 tiles: 16 heads 33.9 us (510 TFLOP/s), 40 with one
+// group, and 43.4 ms for the loop's about 450 launches; 32 heads (two workgroups
+// per CU) 68.7 us.
 #include <type_traits>
 
 #include "ktir_attn_common.h"
@@ -97,15 +100,19 @@ __device__ __forceinline__ void att_lift(const float* p, uint32_t (&t)[2]) {
 }
 
 // The position mask keeps score (row, key) iff ((lo <= kpos - qpos <= hi) != inv).
-template <bool BF16, int M, int N, int D>
-__global__ __launch_bounds__(256, N * D == 64 * 64 ? 3 : 2) void attn_tile(const ktir_attn_t d, int mlo, int mhi, int minv) {
+// G groups of four wavefronts take every G-th key tile of the same lanes, each
+// with tile buffers of its own.
+template <bool BF16, int M, int N, int D, int G>
+__global__ __launch_bounds__(256 * G, G == 1 && N * D == 64 * 64 ? 3 : 2) void attn_tile(const ktir_attn_t d, int mlo, int mhi, int minv) {
   constexpr int KT = N / 32, DS = D / 16, DT = D / 32, PARTS = BF16 ? 3 : 2;
-  __shared__ __align__(16) uint16_t K0s[N * D];     // K tiles of even / odd j
-  __shared__ __align__(16) uint16_t K1s[N * D];
-  __shared__ __align__(16) uint16_t V0s[N * D];     // V tiles of even / odd j
-  __shared__ __align__(16) uint16_t V1s[N * D];
-  const int tid = threadIdx.x, l = tid & 63, h = l >> 5, r32 = l & 31;
+  __shared__ __align__(16) uint16_t K0a[G][N * D];  // K tiles of a group's even / odd steps
+  __shared__ __align__(16) uint16_t K1a[G][N * D];
+  __shared__ __align__(16) uint16_t V0a[G][N * D];  // V tiles of a group's even / odd steps
+  __shared__ __align__(16) uint16_t V1a[G][N * D];
+  const int tid = threadIdx.x & 255, l = tid & 63, h = l >> 5, r32 = l & 31;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int grp = G == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8);
+  uint16_t *K0s = K0a[grp], *K1s = K1a[grp], *V0s = V0a[grp], *V1s = V1a[grp];
   const int32_t* trips = (const int32_t*)d.trips;
   // the workgroup's lanes: wavefronts 0, 1 run la, wavefronts 2, 3 lb
   int la, lb;
@@ -148,9 +155,9 @@ __global__ __launch_bounds__(256, N * D == 64 * 64 ? 3 : 2) void attn_tile(const
   auto step = [&](auto inf_v, int j, const uint16_t* Kc, const uint16_t* Vc, uint16_t* Kn,
                   uint16_t* Vn) __attribute__((always_inline)) {
     constexpr bool INF_V = decltype(inf_v)::value;
-    if (j + 1 < Tmax) {
-      att_stage<N, D>(K + (int64_t)(j + 1) * d.k_step, d.k_row, Kn, w, l);
-      att_stage<N, D>(V + (int64_t)(j + 1) * d.v_step, d.v_row, Vn, w, l);
+    if (j + G < Tmax) {
+      att_stage<N, D>(K + (int64_t)(j + G) * d.k_step, d.k_row, Kn, w, l);
+      att_stage<N, D>(V + (int64_t)(j + G) * d.v_step, d.v_row, Vn, w, l);
     }
     if (j < T) {
       f32x16_t sc[KT];
@@ -205,8 +212,11 @@ __global__ __launch_bounds__(256, N * D == 64 * 64 ? 3 : 2) void attn_tile(const
         lsum = __fmul_rn(lsum, al);
         mr = up ? mn : mr;
       }
+      // a group without tile 0 whose scores have all been -inf: P is 0 against
+      // any base (with tile 0 it is the loop's exp(-inf - (-inf)), NaN)
+      const float mb = G > 1 && grp && mn == -__builtin_inff() ? 0.f : mr;
       if (fast) {
-        const float c0 = -__fmul_rn(mr, LOG2E);
+        const float c0 = -__fmul_rn(mb, LOG2E);
 #pragma unroll
         for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
@@ -215,7 +225,7 @@ __global__ __launch_bounds__(256, N * D == 64 * 64 ? 3 : 2) void attn_tile(const
 #pragma unroll
         for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
-          for (int i = 0; i < 16; ++i) sc[kt][i] = exp_f(__fsub_rn(sc[kt][i], mr));
+          for (int i = 0; i < 16; ++i) sc[kt][i] = exp_f(__fsub_rn(sc[kt][i], mb));
       }
       float a0 = 0.f, a1 = 0.f, a2 = 0.f, a3 = 0.f;
 #pragma unroll
@@ -258,23 +268,24 @@ __global__ __launch_bounds__(256, N * D == 64 * 64 ? 3 : 2) void attn_tile(const
         }
       }
     }
-    __builtin_amdgcn_s_waitcnt(0);                  // this wavefront's part of tile j + 1 has landed
-    __syncthreads();                                // every wavefront: done with tile j, tile j + 1 whole
+    __builtin_amdgcn_s_waitcnt(0);                  // this wavefront's part of the next tile has landed
+    __syncthreads();                                // every wavefront: done with tile j, the next one whole
   };
   auto loop = [&](auto inf_v) __attribute__((always_inline)) {
 #pragma unroll
     for (int t = 0; t < DT; ++t) o[t] = z16;
     m = mr = -__builtin_inff();
     lsum = 0.f;
-    if (Tmax > 0) {
-      att_stage<N, D>(K, d.k_row, K0s, w, l);
-      att_stage<N, D>(V, d.v_row, V0s, w, l);
+    if (grp < Tmax) {
+      att_stage<N, D>(K + (int64_t)grp * d.k_step, d.k_row, K0s, w, l);
+      att_stage<N, D>(V + (int64_t)grp * d.v_step, d.v_row, V0s, w, l);
     }
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
-    for (int j = 0; j < Tmax; j += 2) {
-      step(inf_v, j, K0s, V0s, K1s, V1s);
-      if (j + 1 < Tmax) step(inf_v, j + 1, K1s, V1s, K0s, V0s);
+    // as many steps in every group (one past the end computes nothing)
+    for (int j = 0; j < Tmax; j += 2 * G) {
+      step(inf_v, j + grp, K0s, V0s, K1s, V1s);
+      if (j + G < Tmax) step(inf_v, j + G + grp, K1s, V1s, K0s, V0s);
     }
   };
   loop(std::false_type{});
@@ -287,6 +298,42 @@ __global__ __launch_bounds__(256, N * D == 64 * 64 ? 3 : 2) void attn_tile(const
 #pragma unroll
     for (int i = 0; i < 16; ++i) nan |= o[t][i] != o[t][i];
   if (__syncthreads_or(nan)) loop(std::true_type{});
+  if constexpr (G == 2) {
+    // group 1's state, through the tiles (read by now: the barrier above), to
+    // the thread of group 0 with the same row and columns
+    constexpr int ROWS = G * N * D * 2 / 4096;      // 256 x 16 bytes
+    static_assert(4 * DT <= 2 * ROWS && ROWS >= 1, "state exchange");
+    auto ex = [&](int k) -> float4* { return (float4*)(k < ROWS ? K0a[0] : K1a[0]) + (k < ROWS ? k : k - ROWS) * 256 + tid; };
+    float* exs = (float*)V0a[0] + tid;
+    if (grp == 1) {
+#pragma unroll
+      for (int t = 0; t < DT; ++t)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+          *ex(4 * t + g) = make_float4(o[t][4 * g], o[t][4 * g + 1], o[t][4 * g + 2], o[t][4 * g + 3]);
+      exs[0] = m;
+      exs[256] = mr;
+      exs[512] = lsum;
+    }
+    __syncthreads();
+    if (grp == 1) return;
+    if (T > 0) {
+      const float m1 = exs[0], mm = fmax_nan(m, m1);
+      const float w0 = exp_f(__fsub_rn(mr, mm)), w1 = m1 == -__builtin_inff() ? 0.f : exp_f(__fsub_rn(exs[256], mm));
+#pragma unroll
+      for (int t = 0; t < DT; ++t)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const float4 x = *ex(4 * t + g);
+          o[t][4 * g] = __fadd_rn(__fmul_rn(o[t][4 * g], w0), __fmul_rn(x.x, w1));
+          o[t][4 * g + 1] = __fadd_rn(__fmul_rn(o[t][4 * g + 1], w0), __fmul_rn(x.y, w1));
+          o[t][4 * g + 2] = __fadd_rn(__fmul_rn(o[t][4 * g + 2], w0), __fmul_rn(x.z, w1));
+          o[t][4 * g + 3] = __fadd_rn(__fmul_rn(o[t][4 * g + 3], w0), __fmul_rn(x.w, w1));
+        }
+      lsum = __fadd_rn(__fmul_rn(lsum, w0), __fmul_rn(exs[512], w1));
+      m = mr = mm;
+    }
+  }
   if (lane < 0) return;
   if (T > 0) {
     // bring P, l and O from mr to m
@@ -341,19 +388,33 @@ void launch_attn_tile(const ktir_attn_t& d, int lo, int hi, int inv) {
   const dim3 grid((unsigned)(paired ? d.n_pairs : d.lanes));
   ktir_attn_t a = d;
   if (!paired) a.pairs = 0;
-  auto go = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(256), 0, stream(), a, lo, hi, inv); };
-  auto by_type = [&](auto f16, auto bf16) {
-    if (d.dtype == KTIR_BF16) go(bf16);
-    else go(f16);
+  const std::integral_constant<int, 64> c64;
+  const std::integral_constant<int, 128> c128;
+  // Two groups where every workgroup has a CU of its own (and the tiles fit): a
+  // second wavefront per SIMD runs its softmax under the first one's MFMAs.  With
+  // more workgroups those that share a CU do that, and the exchange costs.
+  int cus = 0, dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+    cus = 0;
+  const bool two = (int)grid.x <= cus;
+  auto go = [&](auto cm, auto cn, auto cd) {
+    constexpr int M = decltype(cm)::value, N = decltype(cn)::value, D = decltype(cd)::value;
+    auto run = [&](auto kern, int groups) {
+      hipLaunchKernelGGL(kern, grid, dim3(256 * groups), 0, stream(), a, lo, hi, inv);
+    };
+    const bool bf = d.dtype == KTIR_BF16;
+    if constexpr (N * D <= 64 * 128)
+      if (two) return bf ? run(attn_tile<true, M, N, D, 2>, 2) : run(attn_tile<false, M, N, D, 2>, 2);
+    bf ? run(attn_tile<true, M, N, D, 1>, 1) : run(attn_tile<false, M, N, D, 1>, 1);
   };
   switch ((d.M == 128) * 4 + (d.N == 128) * 2 + (d.D == 128)) {
-    case 0: by_type(attn_tile<false, 64, 64, 64>, attn_tile<true, 64, 64, 64>); break;
-    case 1: by_type(attn_tile<false, 64, 64, 128>, attn_tile<true, 64, 64, 128>); break;
-    case 2: by_type(attn_tile<false, 64, 128, 64>, attn_tile<true, 64, 128, 64>); break;
-    case 3: by_type(attn_tile<false, 64, 128, 128>, attn_tile<true, 64, 128, 128>); break;
-    case 4: by_type(attn_tile<false, 128, 64, 64>, attn_tile<true, 128, 64, 64>); break;
-    case 5: by_type(attn_tile<false, 128, 64, 128>, attn_tile<true, 128, 64, 128>); break;
-    default: by_type(attn_tile<false, 128, 128, 64>, attn_tile<true, 128, 128, 64>); break;
+    case 0: go(c64, c64, c64); break;
+    case 1: go(c64, c64, c128); break;
+    case 2: go(c64, c128, c64); break;
+    case 3: go(c64, c128, c128); break;
+    case 4: go(c128, c64, c64); break;
+    case 5: go(c128, c64, c128); break;
+    default: go(c128, c128, c64); break;
   }
 }
 

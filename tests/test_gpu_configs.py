@@ -538,6 +538,32 @@ def test_flash_attention_tiles(blk, D, causal, S, dt):
 
 
 @pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("blk,D,S", [(64, 64, 320), (128, 64, 384), (64, 128, 256)])
+def test_flash_attention_tiles_masked_whole(blk, D, S, dt):
+    """Tiles past the diagonal visited too, all their scores -inf: they add
+    nothing, also where one of two groups of wavefronts sees only such tiles."""
+    src, fn, kw = _cases.flash_attention(B=1, H=2, S=S, D=D, blk=blk, dt=dt)
+    old = "%n_kv = arith.addi %qb, %c1 : index"
+    assert old in src
+    src = src.replace(old, f"%n_kv = arith.constant {S // blk} : index")
+    ref, out, g = _run((src, fn, kw))
+    assert dict(g.last_plan.counts()) == {"attn": 1}
+    f = bf16_from_bits if dt == "bf16" else (lambda x: x.astype(np.float32))
+    assert np.isfinite(f(ref["o_ptr"])).all()
+    np.testing.assert_allclose(f(out["o_ptr"]), f(ref["o_ptr"]), rtol=2.0 ** (-7 if dt == "bf16" else -10), atol=1e-5)
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("blk,D,H", [(64, 64, 264), (128, 64, 150), (64, 128, 257)])
+def test_flash_attention_tiles_many_workgroups(blk, D, H, dt):
+    """More workgroups than CUs: one group of wavefronts each."""
+    ref, out, g = _run(_cases.flash_attention(B=1, H=H, S=2 * blk, D=D, blk=blk, dt=dt))
+    assert dict(g.last_plan.counts()) == {"attn": 1}
+    f = bf16_from_bits if dt == "bf16" else (lambda x: x.astype(np.float32))
+    np.testing.assert_allclose(f(out["o_ptr"]), f(ref["o_ptr"]), rtol=2.0 ** (-7 if dt == "bf16" else -10), atol=1e-5)
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
 @pytest.mark.parametrize("fill,sign", [("-1.0e4", 1), ("0xFF800000", -1)])
 def test_flash_attention_tiles_other_fill_or_scale(fill, sign, dt):
     src, fn, kw = _cases.flash_attention(B=1, H=1, S=192, D=64, blk=64, dt=dt)
