@@ -212,6 +212,11 @@ int ktir_malloc(uint64_t bytes, uint64_t* dptr);
 int ktir_free(uint64_t dptr);
 int ktir_memcpy_h2d(uint64_t dst, const void* src, uint64_t bytes);
 int ktir_memcpy_d2h(void* dst, uint64_t src, uint64_t bytes);
+/* The same for n pieces at once.  Uploads are in place for what the library
+ * launches next, without waiting (the host data may change at once; another
+ * stream's work needs ktir_sync in between); downloads share one wait. */
+int ktir_upload_list(int n, const uint64_t* dst, const void* const* src, const uint64_t* bytes);
+int ktir_download_list(int n, void* const* dst, const uint64_t* src, const uint64_t* bytes);
 int ktir_memcpy_d2d(uint64_t dst, uint64_t src, uint64_t bytes);
 int ktir_memset(uint64_t dst, int value, uint64_t bytes);
 int ktir_sync(void);

@@ -88,15 +88,15 @@ class Prepared:
 
     def outputs(self) -> Dict[str, np.ndarray]:
         """Every array argument read back (staged HBM seeds are not arguments)."""
-        rt.sync()
-        out = {}
+        out, parts = {}, []
         for a in self.arena.allocs:
             if a.name not in self.arrays:
                 continue
             src = self.arrays[a.name]
-            dst = np.empty(src.shape, dtype=src.dtype)
-            self.arena.buf.download_into(dst, a.off)
-            out[a.name] = dst
+            out[a.name] = np.empty(src.shape, dtype=src.dtype)
+            parts.append((out[a.name], a.off))
+        self.arena.buf.fetch(parts)
+        rt.sync()
         return out
 
 
@@ -146,8 +146,7 @@ class KTIRInterpreter:
 
     def execute_function(self, fn_name: str, **kwargs) -> Dict[str, np.ndarray]:
         """Run `fn_name` on the GPU; returns every ndarray argument (reference interpreter.py:122-194)."""
-        prep = self.prepare(fn_name, **kwargs)
-        return prep.outputs()
+        return self._prepare(fn_name, kwargs).outputs()     # which waits
 
     def _prepare_execution(self, grid_shape):
         """A fresh memory for one run (reference interpreter.py:95-120).
@@ -159,6 +158,11 @@ class KTIRInterpreter:
     def prepare(self, fn_name: str, **kwargs) -> Prepared:
         """Place the arguments on the device, walk the function once, launch
         it, and return a handle that can replay the device work."""
+        prep = self._prepare(fn_name, kwargs)
+        rt.sync()
+        return prep
+
+    def _prepare(self, fn_name: str, kwargs) -> Prepared:
         if not self.module:
             raise RuntimeError("No module loaded. Call load() first.")
         fn = self.module.get_function(fn_name)
@@ -198,9 +202,8 @@ class KTIRInterpreter:
         arena.layout(specs)
         self._arena = arena
         args: Dict[str, Any] = {}
+        arena.buf.put([(np.ascontiguousarray(initial[a.name]), a.off) for a in arena.allocs])
         for a in arena.allocs:
-            v = initial[a.name]
-            arena.buf.upload(np.ascontiguousarray(v).reshape(-1).view(np.uint8), a.off)
             if a.name in arrays:
                 args[a.name] = np.int64(a.addr // rt.ELEM_BYTES[a.dtype])
         hbm.attach(arena, {k: v.dtype for k, v in initial.items()})
@@ -236,6 +239,5 @@ class KTIRInterpreter:
                               lx=self._lx)
                 plan = ex.run()
                 plan.fallback_reason = str(why)
-        rt.sync()
         self.last_plan = plan
         return Prepared(self, fn_name, list(arrays), plan, arena, arrays, initial, self._lx)

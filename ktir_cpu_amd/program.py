@@ -579,7 +579,7 @@ def _finish(b: _Builder, lanes: int, space) -> Tuple[rt.Prog, list]:
     if b.lane_cols:
         tab = np.stack([np.asarray(c, dtype=np.float64) for c in b.lane_cols], axis=1)
         buf = rt.DeviceBuffer(tab.nbytes)
-        buf.upload(tab)
+        buf.put([(tab, 0)])
         keep.append(buf)
         p.lane_scalars = buf.ptr
         p.n_lane_scalars = tab.shape[1]
@@ -598,7 +598,7 @@ def _fill_leaf(dst: rt.Leaf, L: LeafSpec, lanes: int, ndim: int, keep: list):
         if arr.size < lanes:
             raise CompileError("lane offsets shorter than lane count")
         buf = rt.DeviceBuffer(arr.nbytes)
-        buf.upload(arr)
+        buf.put([(arr, 0)])
         keep.append(buf)
         dst.lane_base = buf.ptr
         dst.base, dst.lane_stride = 0, 0

@@ -163,12 +163,16 @@ def lib():
                      "ktir_launch_matmul", "ktir_event_create", "ktir_event_record",
                      "ktir_event_elapsed_ms", "ktir_event_destroy", "ktir_device_info",
                      "ktir_launch_row_rmw", "ktir_launch_attention", "ktir_rmw_variant", "ktir_shutdown", "ktir_set_row_grid_limit",
-                     "ktir_launch_row_rmw_noalloc", "ktir_launch_paged_attention"):
+                     "ktir_launch_row_rmw_noalloc", "ktir_launch_paged_attention",
+                     "ktir_upload_list", "ktir_download_list"):
             getattr(L, name).restype = C.c_int
         L.ktir_malloc.argtypes = [C.c_uint64, C.POINTER(C.c_uint64)]
         L.ktir_free.argtypes = [C.c_uint64]
         L.ktir_memcpy_h2d.argtypes = [C.c_uint64, C.c_void_p, C.c_uint64]
         L.ktir_memcpy_d2h.argtypes = [C.c_void_p, C.c_uint64, C.c_uint64]
+        u64s, ptrs = C.POINTER(C.c_uint64), C.POINTER(C.c_void_p)
+        L.ktir_upload_list.argtypes = [C.c_int, u64s, ptrs, u64s]
+        L.ktir_download_list.argtypes = [C.c_int, ptrs, u64s, u64s]
         L.ktir_memcpy_d2d.argtypes = [C.c_uint64, C.c_uint64, C.c_uint64]
         L.ktir_memset.argtypes = [C.c_uint64, C.c_int, C.c_uint64]
         L.ktir_launch_program.argtypes = [C.POINTER(Prog)]
@@ -247,6 +251,24 @@ class DeviceBuffer:
         self.host_writes += 1
         check(lib().ktir_memcpy_h2d(self.ptr + offset, a.ctypes.data, a.nbytes), "ktir_memcpy_h2d")
 
+    def put(self, parts):
+        """Upload C-contiguous arrays, (array, byte offset) each: in place for
+        the library's next launch (`upload` also waits)."""
+        n = len(parts)
+        assert all(a.flags.c_contiguous and o + a.nbytes <= self.nbytes for a, o in parts)
+        self.host_writes += n
+        check(lib().ktir_upload_list(n, (C.c_uint64 * n)(*[self.ptr + o for _, o in parts]),
+                                     (C.c_void_p * n)(*[a.ctypes.data for a, _ in parts]),
+                                     (C.c_uint64 * n)(*[a.nbytes for a, _ in parts])), "ktir_upload_list")
+
+    def fetch(self, parts):
+        """Download into C-contiguous arrays, (array, byte offset) each, behind one wait."""
+        n = len(parts)
+        assert all(a.flags.c_contiguous and o + a.nbytes <= self.nbytes for a, o in parts)
+        check(lib().ktir_download_list(n, (C.c_void_p * n)(*[a.ctypes.data for a, _ in parts]),
+                                       (C.c_uint64 * n)(*[self.ptr + o for _, o in parts]),
+                                       (C.c_uint64 * n)(*[a.nbytes for a, _ in parts])), "ktir_download_list")
+
     def download_into(self, dst: np.ndarray, offset: int = 0):
         """Copy dst.nbytes bytes from the buffer (at `offset`) into the
         C-contiguous host array `dst`."""
@@ -301,8 +323,7 @@ class BufferPool:
 
 
 def sync():
-    check(lib().ktir_sync(), "ktir_sync")
-    check(lib().ktir_check_error_flag(), "device")
+    check(lib().ktir_check_error_flag(), "device")     # waits for the stream
 
 
 class Event:
