@@ -2,10 +2,10 @@
 // math on f16 / bf16 rows: dialects/linalg_ops.py:86-246 folds with their
 // elementwise ops) for rows of any length up to KTIR_MAX_ROW and any alignment.
 //
-// W wavefronts own a row (one up to 3072 elements, then two and four) and
+// W wavefronts own a row (one up to 3072 elements, norm rows up to 4096, then
+// two and four) and
 // read it once, each thread C chunks of 8 elements; a workgroup runs a stream
-// of rows, the next row's loads in flight while the current one is computed.
-// Few wavefronts per row: what a row costs besides its elements (the
+// of rows.  Few wavefronts per row: what a row costs besides its elements (the
 // reductions, the row instructions between the folds) every one of them pays.
 // Rows that do not start on 16-byte boundaries are read with unaligned 16-byte
 // loads; the chunk that the row's end cuts is read from the last 8 elements
@@ -14,10 +14,10 @@
 // their allocations, so the kernel has no other bounds to check.
 // Memory bounds it from about 1000 elements on, the reductions below.
 // Against the interpreter's row kernel (prog_rows), f16 unless said:
-//   softmax  8192 x 3000 bf16 1191 -> 23 us (4.2 TB/s), 32768 x 1000 2148 -> 27 us,
-//            2048 x 16384 1298 -> 29 us;
-//   rmsnorm  8192 x 5120 1395 -> 49 us (3.4 TB/s), 32768 x 1000 1813 -> 49 us,
-//            2048 x 16384 979 -> 34 us.
+//   softmax  8192 x 3000 bf16 1191 -> 20 us (4.9 TB/s), 32768 x 1000 2148 -> 25 us,
+//            2048 x 16384 1298 -> 26 us;
+//   rmsnorm  8192 x 5120 1395 -> 43 us (3.9 TB/s), 32768 x 1000 1813 -> 47 us,
+//            2048 x 16384 979 -> 27 us.
 //   row max and the softmax sum: per thread, lane exchanges, then one exchange
 //     between the wavefronts through LDS;
 //   the norm's sum of squares: the reference's halving tree (element i with
@@ -110,6 +110,14 @@ struct RaMap {
   // elements of a part's last chunk (below 1: none, above 7: all eight)
   __device__ __forceinline__ int last() const { return part - 8 * (t + (Q - 1) * T); }
 };
+
+template <int C, int P>
+__device__ __forceinline__ gu4 ra_chunk(uint64_t row, const RaMap<C, P>& M, int i) {
+  const int end = M.part * P - 8;
+  int o = M.off(i);
+  if (i % M.Q == M.Q - 1) o = o < end ? o : end;
+  return *(const KTIR_G(ra_u4)*)((const KTIR_G(uint16_t)*)row + o);
+}
 
 template <int C, int P>
 __device__ __forceinline__ void ra_load(uint64_t row, const RaMap<C, P>& M, gu4 (&c)[C]) {
@@ -307,9 +315,9 @@ __device__ __forceinline__ void ra_softmax(const RaPlan& F, gu4 (&c)[C], const R
   }
 }
 
-template <int C, int DT, int P, int W>
-__device__ __forceinline__ void ra_norm(const RaPlan& F, gu4 (&c)[C], const gu4 (&w)[C], const RaMap<C, P>& M, uint64_t y_row,
-                                        int64_t lane, RowLanes& rr, float* lds) {
+template <int C, int DT, int P, int W, bool KEEP>
+__device__ __forceinline__ void ra_norm(const RaPlan& F, gu4 (&c)[C], const gu4 (&w)[KEEP ? C : 1], const RaMap<C, P>& M,
+                                        uint64_t y_row, int64_t lane, RowLanes& rr, float* lds) {
   // squares into LDS, the two halves of the row combined first (P = 2)
 #pragma unroll
   for (int i = 0; i < M.Q; ++i) {
@@ -338,13 +346,23 @@ __device__ __forceinline__ void ra_norm(const RaPlan& F, gu4 (&c)[C], const gu4 
   rr.set(F.fold0, ra_tree<W>(lds, M.part, M.t, M.T));
   for (int k = 0; k < F.n_row0; ++k) rw_row_exec(F, F.row0[k], rr, lane);
   const float s = rr.get(F.s);
+  gu4 wn = {0u, 0u, 0u, 0u};
+  if (!KEEP && F.has_w) wn = ra_chunk<C, P>(F.w, M, 0);
 #pragma unroll
   for (int i = 0; i < C; ++i) {
     float y[8];
+    gu4 wi = wn;
+    if (!KEEP && F.has_w && i + 1 < C) wn = ra_chunk<C, P>(F.w, M, i + 1);
     rf_unpack<DT>(c[i], y);
     if (F.has_w) {
       float wv[8];
-      rf_unpack<DT>(w[i], wv);
+      if constexpr (KEEP) {
+        wi = w[i];
+      } else if (P == 1 && i == C - 1) {
+        const int k = M.last();
+        if (k > 0 && k < 8) wi = ra_shift(wi, k);
+      }
+      rf_unpack<DT>(wi, wv);
       if (F.w_first) {
 #pragma unroll
         for (int j = 0; j < 8; ++j) y[j] = mul_keep(__fmul_rn(y[j], wv[j]), s);
@@ -361,36 +379,54 @@ __device__ __forceinline__ void ra_norm(const RaPlan& F, gu4 (&c)[C], const gu4 
   }
 }
 
+// Whether a workgroup holds the weights and has the next row's loads in flight
+// while it computes a row.  Those registers pay only where they cost no
+// wavefront: rows of one chunk per thread, and the longest norm rows that keep
+// all their squares in LDS (two workgroups per CU at most).  Elsewhere more
+// wavefronts hide the loads better: rmsnorm 8192 x 5120 40.6 -> 34.7 us, softmax
+// 10752 x 3072 21.4 -> 18.2 us (replayed on the same buffers).
+constexpr bool ra_keep(int recipe, int C, int P, int W) {
+  return C == 1 || (recipe == RF_NORM && W == 4 && P == 1 && C >= 7);
+}
+
 // wavefronts per SIMD to fit the registers to: the most that spills nothing
-constexpr int ra_waves(int recipe, int C) {
-  return C <= 3 ? 5 : (C <= (recipe == RF_NORM ? 4 : 5) ? 4 : (C <= 6 ? 3 : 2));
+constexpr int ra_waves(int recipe, int C, int P, int W) {
+  if (ra_keep(recipe, C, P, W)) return C == 1 ? 5 : 2;
+  return C <= 3 ? 6 : (C == 4 ? 5 : (C <= 6 || recipe == RF_NORM ? 4 : 3));
 }
 
 template <int RECIPE, int DT, int C, int P, int W>
-__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(ra_waves(RECIPE, C)))) void prog_rowany(const RaPlan F) {
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(ra_waves(RECIPE, C, P, W)))) void prog_rowany(const RaPlan F) {
   extern __shared__ __align__(16) float ra_lds[];
   const RaMap<C, P> M{(int)threadIdx.x, 64 * W, P == 1 ? F.n : F.n / P};
   constexpr uint32_t PAD = RECIPE == RF_SOFTMAX ? (DT == KTIR_BF16 ? 0xff80ff80u : 0xfc00fc00u) : 0u;   // -inf, or 0
   RowLanes rr{0, (int)(threadIdx.x & 63)};
   int r = blockIdx.x;
-  gu4 c[C], w[C];
-  if (RECIPE == RF_NORM && F.has_w) ra_load<C, P>(F.w, M, w);
+  constexpr bool KEEP = ra_keep(RECIPE, C, P, W);
+  gu4 c[C], w[RECIPE == RF_NORM && KEEP ? C : 1];
+  if constexpr (RECIPE == RF_NORM && KEEP)
+    if (F.has_w) ra_load<C, P>(F.w, M, w);
   ra_load<C, P>(F.x + 2 * (uint64_t)(r * F.x_step), M, c);
   while (true) {
     const int rn = r + (int)gridDim.x;
-    gu4 nx[C];
-    if (rn < F.rows) ra_load<C, P>(F.x + 2 * (uint64_t)(rn * F.x_step), M, nx);
+    gu4 nx[KEEP ? C : 1];
+    if constexpr (KEEP)
+      if (rn < F.rows) ra_load<C, P>(F.x + 2 * (uint64_t)(rn * F.x_step), M, nx);
     ra_trim<C, P>(M, c, PAD);
-    if constexpr (RECIPE == RF_NORM && P == 1) {
+    if constexpr (RECIPE == RF_NORM && P == 1 && KEEP) {
       if (r == (int)blockIdx.x && F.has_w) ra_trim<C, P>(M, w, 0u);
     }
     const uint64_t y_row = F.y + 2 * (uint64_t)(r * F.y_step);
     const int64_t lane = F.rows_per_lane == 1 ? r : r / F.rows_per_lane;
     if constexpr (RECIPE == RF_SOFTMAX) ra_softmax<C, DT, W>(F, c, M, y_row, lane, rr, ra_lds);
-    else ra_norm<C, DT, P, W>(F, c, w, M, y_row, lane, rr, ra_lds);
+    else ra_norm<C, DT, P, W, KEEP>(F, c, w, M, y_row, lane, rr, ra_lds);
     if (rn >= F.rows) break;
+    if constexpr (KEEP) {
 #pragma unroll
-    for (int i = 0; i < C; ++i) c[i] = nx[i];
+      for (int i = 0; i < C; ++i) c[i] = nx[i];
+    } else {
+      ra_load<C, P>(F.x + 2 * (uint64_t)(rn * F.x_step), M, c);
+    }
     r = rn;
     ra_sync<W>();                              // the next row's folds reuse the LDS
   }
@@ -424,7 +460,8 @@ static void rowany_p(const RaPlan& F) {
 }
 
 // C = the chunks per thread that the row fills to the last: up to six on one
-// wavefront, then two, then four (up to eight each)
+// wavefront (norm rows, which hold no exponentials, up to eight: 8192 x 4000 26
+// us, on two wavefronts 31), then two, then four (up to eight each)
 template <int RECIPE, int DT>
 static void rowany_c(const RaPlan& F) {
   const int q = (F.n + 7) / 8;
@@ -435,6 +472,12 @@ static void rowany_c(const RaPlan& F) {
     case 4: return rowany_p<RECIPE, DT, 4, 1>(F);
     case 5: return rowany_p<RECIPE, DT, 5, 1>(F);
     case 6: return rowany_p<RECIPE, DT, 6, 1>(F);
+  }
+  if constexpr (RECIPE == RF_NORM) {
+    switch ((q + 63) / 64) {
+      case 7: return rowany_p<RECIPE, DT, 7, 1>(F);
+      case 8: return rowany_p<RECIPE, DT, 8, 1>(F);
+    }
   }
   if (q <= 6 * 128) {
     switch ((q + 127) / 128) {

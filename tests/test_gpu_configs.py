@@ -267,7 +267,8 @@ def test_rmsnorm_bit_exact_many_rows_per_workgroup(cols, dt, row_grid_limit):
 
 # one row per wavefront (up to 2048 elements) and per workgroup; whole chunks,
 # a cut last chunk, odd lengths (rows off every alignment), the longest rows
-_ANY_COLS = [5, 8, 64, 100, 513, 1000, 2047, 2056, 3000, 3001, 3072, 3080, 5120, 6144, 8192, 12287, 16383, 16384]
+_ANY_COLS = [5, 8, 64, 100, 513, 1000, 2047, 2056, 3000, 3001, 3072, 3080, 3584, 3585, 4088, 4095, 4104, 5120, 6144, 8192,
+             12287, 14000, 16383, 16384]
 
 
 @pytest.mark.parametrize("limit", [0, 3])
