@@ -604,7 +604,7 @@ def collect_traffic(root):
                     name = row.get("Kernel_Name", "")
                     # set-up work outside the timed launch: the runtime's copies and
                     # fills, and the library's one-time fill of its own scratch array
-                    if name.startswith("__amd_rocclr") or name.startswith("rmw_fill"):
+                    if name.startswith("__amd_rocclr") or name.startswith("rmw_fill") or "copy_parts" in name:
                         continue
                     if row.get("Counter_Name") == counter:
                         vals.setdefault(name, []).append(float(row["Counter_Value"]))
