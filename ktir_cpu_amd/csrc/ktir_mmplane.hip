@@ -15,8 +15,8 @@
 // workgroup has a CU to itself three stages stay in flight (512 x 4096 x 4096,
 // f16: 49 us with two stages, 29 with four).  Then the LDS reads bound it: a
 // 64 x 64 quarter reads 16 KB for 16 MFMAs.
-// 512 x 4096 x 4096 in 64 x 64 tiles: 1009 us (mm_generic, f32 FMA) -> 29 us
-// (600 TFLOP/s); 2048^3 in 128 x 128 tiles: 47 us (mm_mfma_256) -> 27 us.
+// 512 x 4096 x 4096 in 64 x 64 tiles: 1009 us (mm_generic, f32 FMA) -> 26 us
+// (660 TFLOP/s); 2048^3 in 128 x 128 tiles: 47 us (mm_mfma_256) -> 26 us.
 // Layouts: A as 128-byte rows (16-byte chunk c of row
 // r at slot c ^ swz_a(r), read by ds_read_b128), B row-major as in HBM (chunk c
 // at c ^ mp_swz(r), read by ds_read_b64_tr_b16); both layouts are free of bank
