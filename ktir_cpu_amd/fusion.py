@@ -20,7 +20,7 @@ from typing import List, Optional
 import numpy as np
 
 from .affine import Box
-from .executor import ATile, IATile, NeedEager, Tile, V16Copy
+from .executor import ATile, DevScalar, IATile, NeedEager, Tile, V16Copy
 
 _SCALAR_OPS_PREFIX = ("arith.",)
 _SKIP = {"ktdp.load", "arith.extf", "linalg.matmul", "scf.yield"}
@@ -1115,6 +1115,35 @@ def _plain_ld(e, ptr, shape, inner):
     if len(sh) < 2 or any(x != 1 for x in sh[:-2]) or tuple(sh[-2:]) != shape:
         return False
     return stv[-2:] == inner and e.attr.lane.arr is None and e.attr.lane.base == 0
+
+
+def _read_outside(ops, names):
+    """Those of `names` that an op reads outside the loops that carry a value
+    of that name."""
+    out = set()
+    for o in ops:
+        out |= names.intersection(o.operands)
+        for r in o.regions:
+            inner = names.difference(o.attributes.get("iter_args", []), [n for n, _ in r.args])
+            if inner:
+                out |= _read_outside(r.ops, inner)
+    return out
+
+
+def acc_read_later(ex, ptr, names) -> bool:
+    """Whether a live value reads the accumulator at `ptr` of the attention
+    loop with iter_args `names`.  A value that is used for the last time has
+    left the frames by then, so a stored one that is still there is used again.
+    The loop's iter_args keep their last values in the frame, which nothing
+    reads unless their names occur outside such a loop."""
+    from .program import walk
+    gone = set(names) - _read_outside(ex.fn.operations, set(names))
+    for fr in ex.frames:
+        for name, v in fr.vals.items():
+            v = v.t if isinstance(v, DevScalar) else v
+            if name not in gone and isinstance(v, Tile) and any(n.kind == "ld" and n.attr.ptr == ptr for n in walk(v.e)):
+                return True
+    return False
 
 
 def attention_epilogue(ex, e, dest) -> bool:

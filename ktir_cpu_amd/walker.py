@@ -942,11 +942,8 @@ class Executor:
         d.out_ptr, d.out_base = dest.ptr, base.ptr
         d.out_grp, d.out_gstride, d.out_row, d.out_lo, d.out_hi = grp, gstride, row, dest.lo, dest.hi
         d.out_dtype = rt.DTYPE_CODE[dest.dtype]
-        # acc is written only where a live value other than this store reads it
-        # (the loop's own iter_args are not visible after the loop)
-        if not any(isinstance(v, Tile) and v.e is not e and name not in self.pattn_names
-                   and any(n.kind == "ld" and n.attr.ptr == d.acc_out for n in topo(v.e))
-                   for fr in self.frames for name, v in fr.vals.items()):
+        from .fusion import acc_read_later
+        if not acc_read_later(self, d.acc_out, self.pattn_names):
             d.acc_out = 0
         return True
 
