@@ -1182,28 +1182,14 @@ def attention_epilogue(ex, e, dest) -> bool:
             or o_row < D:
         return False
     d = pend["desc"]
-    # acc stays needed if any live value other than this store still reads it
-    # (the loop's own iter_args are not visible after the loop)
-    acc_live = False
-    for fr in ex.frames:
-        for name, v in fr.vals.items():
-            if name in pend["body_names"] or not isinstance(v, Tile) or v.e is e:
-                continue
-            if any(n.attr.ptr == acc_buf.ptr for n in _walk_ld(v.e)):
-                acc_live = True
     ob = ex.pool.upload(np.ascontiguousarray(offs.astype(np.int64)))
     pend["keep"].extend([ob, dest])
     d.o_ptr, d.o_base, d.o_row = dest.ptr, ob.ptr, o_row
     d.o_dtype = rt.DTYPE_CODE[dest.dtype]
-    if not acc_live:
+    if not acc_read_later(ex, acc_buf.ptr, pend["body_names"]):
         d.acc_out = 0
     ex.attn_pending = None
     return True
-
-
-def _walk_ld(e):
-    from .program import walk
-    return [n for n in walk(e) if n.kind == "ld"]
 
 
 # ---------------------------------------------------------------------------

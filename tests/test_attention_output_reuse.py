@@ -12,6 +12,7 @@ from ktir_cpu_amd import configs
 from ktir_cpu_amd import runtime as rt
 from ktir_cpu_amd.interpreter import KTIRInterpreter
 from oracle.interp import OracleInterpreter, bf16_from_bits
+from tests import _cases
 from tests.test_oracle_example_pins import PA_ARGS, PA_FN, paged_inputs
 
 
@@ -83,9 +84,27 @@ def _paged(how, dt="f16", **gen):
     return src, PA_FN, kw
 
 
+def _flash(how, blk, D, dt="f16", S=None):
+    src, fn, args = _cases.flash_attention(B=1, H=2, S=S or 2 * blk, D=D, blk=blk, dt=dt)
+    if how is None:
+        return src, fn, args
+    src = _again(src, how, "o_ptr", "o_view", "o_acc", "%o4", f"tensor<1x1x{blk}x{D}x{dt}>",
+                 f"!ktdp.access_tile<1x1x{blk}x{D}xindex>", "%ob", f"tensor<{blk}x{D}x{dt}>")
+    kw = {}
+    for k, v in args.items():
+        kw[k] = v
+        if k == "o_ptr":
+            kw["again_ptr"] = np.zeros_like(v)
+    return src, fn, kw
+
+
 CASES = {
     "paged_8_rows": lambda how, dt: _paged(how, dt),
     "paged_32_rows": lambda how, dt: _paged(how, dt, tokens=16, block_q=8),
+    "tiles_64": lambda how, dt: _flash(how, 64, 64, dt),
+    "tiles_128_by_64": lambda how, dt: _flash(how, 128, 64, dt),
+    "tiles_64_by_128": lambda how, dt: _flash(how, 64, 128, dt),
+    "tiles_128": lambda how, dt: _flash(how, 128, 128, dt),
 }
 
 
