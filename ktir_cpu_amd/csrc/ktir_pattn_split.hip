@@ -65,13 +65,36 @@ __device__ __forceinline__ bool ps_fast(int64_t e0, int64_t row, int64_t lo, int
   return !(e0 & 7) && e0 >= lo && e0 + 15 * row + D <= hi;
 }
 
-// The loads go through one asm statement each (no result registers; M0 holds
-// the LDS address) and are waited for by ps_wait alone: the compiler, which
-// does not tell the two buffers of a wavefront apart in a loop, would wait for
-// both wherever one is read.
-__device__ __forceinline__ void ps_load16(u32x4_t rsrc, uint32_t off, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(off), "s"(rsrc), "s"(lds)
-               : "memory", "m0");
+// N loads of 1 KB into successive KB of LDS in one asm statement (no result
+// registers) that ps_wait alone waits for: the compiler, which does not tell the
+// two buffers of a wavefront apart in a loop, would wait for both wherever one is
+// read.  The hazards inside are not the compiler's either: a vector instruction
+// (readfirstlane, a reload of a spilled register) may have written the
+// descriptor just before, which a load may read five wait states later (M0 to
+// the first load: move and s_nop 4), and M0, which holds the LDS address, is
+// what it was afterwards.
+template <int N>
+__device__ __forceinline__ void ps_load(u32x4_t rsrc, const uint32_t (&off)[N], uint32_t lds) {
+  static_assert(N == 2 || N == 4, "16 rows of 64 or 128 columns");
+  uint32_t m0;
+  if constexpr (N == 4)
+    asm volatile(
+        "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %6\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %5, 0 offen lds\n\t"
+        "s_add_u32 m0, m0, 0x400\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %5, 0 offen lds\n\t"
+        "s_add_u32 m0, m0, 0x400\n\ts_nop 0\n\tbuffer_load_dwordx4 %3, %5, 0 offen lds\n\t"
+        "s_add_u32 m0, m0, 0x400\n\ts_nop 0\n\tbuffer_load_dwordx4 %4, %5, 0 offen lds\n\t"
+        "s_mov_b32 m0, %0\n\ts_nop 0"
+        : "=&s"(m0)
+        : "v"(off[0]), "v"(off[1]), "v"(off[2]), "v"(off[3]), "s"(rsrc), "s"(lds)
+        : "memory", "scc");
+  else
+    asm volatile(
+        "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %4\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %3, 0 offen lds\n\t"
+        "s_add_u32 m0, m0, 0x400\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %3, 0 offen lds\n\t"
+        "s_mov_b32 m0, %0\n\ts_nop 0"
+        : "=&s"(m0)
+        : "v"(off[0]), "v"(off[1]), "s"(rsrc), "s"(lds)
+        : "memory", "scc");
 }
 
 // until at most N of this wavefront's loads are in flight; no memory access
@@ -91,10 +114,10 @@ __device__ __forceinline__ void ps_dma(uint64_t ptr, int64_t e0, int64_t row, bo
                       (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(a >> 32) & 0xffffu),
                       (uint32_t)__builtin_amdgcn_readfirstlane(there ? (uint32_t)((15 * row + D) * 2) : 0u), 0x00020000u};
   const int r = l / CH, c = l % CH;
+  uint32_t off[16 / RB];
 #pragma unroll
-  for (int i = 0; i < 16 / RB; ++i)
-    ps_load16(rs, (uint32_t)(((RB * i + r) * row + 8 * (c ^ ps_swz<D>((RB * i + r) & 15))) * 2),
-              lds + 2 * D * (row0 + RB * i));
+  for (int i = 0; i < 16 / RB; ++i) off[i] = (uint32_t)(((RB * i + r) * row + 8 * (c ^ ps_swz<D>((RB * i + r) & 15))) * 2);
+  ps_load<16 / RB>(rs, off, lds + 2 * D * row0);
 }
 
 // the same of any page: zeros outside [lo, hi)
