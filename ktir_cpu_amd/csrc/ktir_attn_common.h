@@ -52,6 +52,23 @@ __device__ __forceinline__ void split4(const float* p, uint32_t& h0, uint32_t& h
   l1 = cvt2<BF16>(__fsub_rn(p[2], b.x), __fsub_rn(p[3], b.y));
 }
 
+// the packed values of w with 0 in the place of infinities and NaN
+template <bool BF16>
+__device__ __forceinline__ uint32_t finite2(uint32_t w) {
+  constexpr uint32_t E = BF16 ? 0x7f80u : 0x7c00u;
+  const uint32_t lo = (w & E) == E ? 0u : w & 0xffffu, hi = ((w >> 16) & E) == E ? 0u : w & 0xffff0000u;
+  return lo | hi;
+}
+
+// the smallest f16 in the place of a leading term 0 whose value is positive
+__device__ __forceinline__ void lift4(const float* p, uint32_t (&t)[2]) {
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    if (p[2 * k] > 0.f && !(t[k] & 0xffffu)) t[k] |= 1u;
+    if (p[2 * k + 1] > 0.f && !(t[k] >> 16)) t[k] |= 0x10000u;
+  }
+}
+
 // v_permlane32_swap: lanes 32-63 of a trade places with lanes 0-31 of b, so
 // afterwards lanes 0-31 hold a of both half-waves (own in a, the other
 // half's in b) and lanes 32-63 hold b of both (the other half's in a)

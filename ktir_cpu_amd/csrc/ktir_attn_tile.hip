@@ -82,23 +82,6 @@ __device__ __forceinline__ void att_split(const float* x, uint32_t (&t)[PARTS][2
   }
 }
 
-// the packed values of w with 0 in the place of infinities and NaN
-template <bool BF16>
-__device__ __forceinline__ uint32_t att_finite(uint32_t w) {
-  constexpr uint32_t E = BF16 ? 0x7f80u : 0x7c00u;
-  const uint32_t lo = (w & E) == E ? 0u : w & 0xffffu, hi = ((w >> 16) & E) == E ? 0u : w & 0xffff0000u;
-  return lo | hi;
-}
-
-// the smallest f16 in the place of a leading term 0 whose value is positive
-__device__ __forceinline__ void att_lift(const float* p, uint32_t (&t)[2]) {
-#pragma unroll
-  for (int k = 0; k < 2; ++k) {
-    if (p[2 * k] > 0.f && !(t[k] & 0xffffu)) t[k] |= 1u;
-    if (p[2 * k + 1] > 0.f && !(t[k] >> 16)) t[k] |= 0x10000u;
-  }
-}
-
 // The position mask keeps score (row, key) iff ((lo <= kpos - qpos <= hi) != inv).
 // G groups of four wavefronts take every G-th key tile of the same lanes, each
 // with tile buffers of its own.
@@ -251,8 +234,8 @@ __global__ __launch_bounds__(256 * G, G == 1 && N * D == 64 * 64 ? 3 : 2) void a
         att_split<BF16, PARTS>(p + 4, t1);
         if constexpr (INF_V && !BF16) {
           // a positive P below f16's range still times an infinite V is infinite
-          att_lift(p, t0[0]);
-          att_lift(p + 4, t1[0]);
+          lift4(p, t0[0]);
+          lift4(p + 4, t1[0]);
         }
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) {
@@ -261,7 +244,7 @@ __global__ __launch_bounds__(256 * G, G == 1 && N * D == 64 * 64 ? 3 : 2) void a
           const uint4 a = make_uint4(lo.x, lo.y, hi.x, hi.y);
           uint4 af = a;
           if constexpr (INF_V)
-            af = make_uint4(att_finite<BF16>(a.x), att_finite<BF16>(a.y), att_finite<BF16>(a.z), att_finite<BF16>(a.w));
+            af = make_uint4(finite2<BF16>(a.x), finite2<BF16>(a.y), finite2<BF16>(a.z), finite2<BF16>(a.w));
 #pragma unroll
           for (int q = PARTS - 1; q >= 0; --q)
             o[dt] = mfma_at<BF16>(q ? af : a, make_uint4(t0[q][0], t0[q][1], t1[q][0], t1[q][1]), o[dt]);

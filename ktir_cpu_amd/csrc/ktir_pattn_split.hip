@@ -315,9 +315,7 @@ __global__ __launch_bounds__(64 * W, 2) void pattn_split(const ktir_pattn_t d, i
   };
   const f32x16_t z16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   f32x16_t o[DT];                              // O^T tiles: column 32 dt + 8 g + 4 h + t of row r32
-#pragma unroll
-  for (int t = 0; t < DT; ++t) o[t] = z16;
-  float m = -__builtin_inff(), mr = -__builtin_inff(), lsum = 0.f;
+  float m, mr, lsum;
   const int k_off = r32 * D, k_x = ps_swz<D>(r32 & 15);
   const int tg = l >> 4, tj = l & 15;
   const int v_row0 = 4 * (tg >> 1) + (tj >> 2);
@@ -327,9 +325,9 @@ __global__ __launch_bounds__(64 * W, 2) void pattn_split(const ktir_pattn_t d, i
   constexpr int LOADS = 32 * D / 512;          // a pair's K (or V) loads
   // One pair.  FAST: its K and V are in flight, K first; those of pair `next`
   // (the last pair again at the end, so that the count in flight is the same)
-  // follow as each buffer falls free.
-  auto step = [&](auto fast, int k, int next) __attribute__((always_inline)) {
-    constexpr bool FAST = decltype(fast)::value;
+  // follow as each buffer falls free.  INF_V: V may hold infinities.
+  auto step = [&](auto fast, auto inf_v, int k, int next) __attribute__((always_inline)) {
+    constexpr bool FAST = decltype(fast)::value, INF_V = decltype(inf_v)::value;
     const int j0 = 2 * (first_pair + k * stride);
     if constexpr (FAST) ps_wait<LOADS>();
     f32x16_t sc = z16;
@@ -404,14 +402,21 @@ __global__ __launch_bounds__(64 * W, 2) void pattn_split(const ktir_pattn_t d, i
       uint32_t t0[PARTS][2], t1[PARTS][2];
       ps_split<BF16, PARTS>(x + 8 * ks, t0);
       ps_split<BF16, PARTS>(x + 8 * ks + 4, t1);
+      if constexpr (INF_V && !BF16) {
+        // a positive P below f16's range still times an infinite V is infinite
+        lift4(x + 8 * ks, t0[0]);
+        lift4(x + 8 * ks + 4, t1[0]);
+      }
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) {
         const uint2 lo = ds_tr16(vt + v_b0 + 8 * ((4 * dt) ^ v_x0));
         const uint2 hi = ds_tr16(vt + v_b0 + 8 * D + 8 * ((4 * dt) ^ v_x1));
         const uint4 a = make_uint4(lo.x, lo.y, hi.x, hi.y);
+        uint4 af = a;
+        if constexpr (INF_V) af = make_uint4(finite2<BF16>(a.x), finite2<BF16>(a.y), finite2<BF16>(a.z), finite2<BF16>(a.w));
 #pragma unroll
         for (int q = PARTS - 1; q >= 0; --q)
-          o[dt] = mfma_at<BF16>(a, make_uint4(t0[q][0], t0[q][1], t1[q][0], t1[q][1]), o[dt]);
+          o[dt] = mfma_at<BF16>(q ? af : a, make_uint4(t0[q][0], t0[q][1], t1[q][0], t1[q][1]), o[dt]);
       }
     }
     if constexpr (FAST) {
@@ -437,28 +442,49 @@ __global__ __launch_bounds__(64 * W, 2) void pattn_split(const ktir_pattn_t d, i
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (FAST) dma(next, true);
   };
-  for (int c0 = 0; c0 < mine; c0 += 32) {
-    if (c0) table = entries(c0);
-    const int c1 = c0 + 32 < mine ? c0 + 32 : mine;
-    // pages of these pairs that are wholly in their windows, or missing
-    const int my_pair = c0 + (l >> 1);
-    const int64_t ke = kb + table * d.k_page, ve = vb + table * d.v_page;
-    const bool ok = my_pair >= c1 || (vec && (2 * (first_pair + my_pair * stride) + (l & 1) >= trips ||
-                                              (ps_fast<D>(ke, d.k_row, d.k_lo, d.k_hi) && ps_fast<D>(ve, d.v_row, d.v_lo, d.v_hi))));
-    const uint64_t ballot = __builtin_amdgcn_ballot_w64(!ok);
-    // the pairs before the first that is not
-    const int nf = ballot ? __builtin_ctzll(ballot) >> 1 : c1 - c0;
-    int k = c0;
-    if (nf > 0) {
-      dma(c0, false);
-      dma(c0, true);
-      for (; k < c0 + nf; ++k) step(std::true_type{}, k, k + 1 < c0 + nf ? k + 1 : k);
-      ps_wait<0>();
+  auto pages = [&](auto inf_v) __attribute__((always_inline)) {
+    constexpr bool INF_V = decltype(inf_v)::value;
+#pragma unroll
+    for (int t = 0; t < DT; ++t) o[t] = z16;
+    m = mr = -__builtin_inff();
+    lsum = 0.f;
+    for (int c0 = 0; c0 < mine; c0 += 32) {
+      if (INF_V || c0) table = entries(c0);
+      const int c1 = c0 + 32 < mine ? c0 + 32 : mine;
+      int k = c0;
+      if constexpr (!INF_V) {
+        // pages of these pairs that are wholly in their windows, or missing
+        const int my_pair = c0 + (l >> 1);
+        const int64_t ke = kb + table * d.k_page, ve = vb + table * d.v_page;
+        const bool ok = my_pair >= c1 || (vec && (2 * (first_pair + my_pair * stride) + (l & 1) >= trips ||
+                                                  (ps_fast<D>(ke, d.k_row, d.k_lo, d.k_hi) && ps_fast<D>(ve, d.v_row, d.v_lo, d.v_hi))));
+        const uint64_t ballot = __builtin_amdgcn_ballot_w64(!ok);
+        // the pairs before the first that is not
+        const int nf = ballot ? __builtin_ctzll(ballot) >> 1 : c1 - c0;
+        if (nf > 0) {
+          dma(c0, false);
+          dma(c0, true);
+          for (; k < c0 + nf; ++k) step(std::true_type{}, inf_v, k, k + 1 < c0 + nf ? k + 1 : k);
+          ps_wait<0>();
+        }
+      }
+      for (; k < c1; ++k) {
+        copy(k);
+        step(std::false_type{}, inf_v, k, k);
+      }
     }
-    for (; k < c1; ++k) {
-      copy(k);
-      step(std::false_type{}, k, k);
-    }
+  };
+  pages(std::false_type{});
+  // An infinite V times the terms of P after the first (0, or of the other
+  // sign) is NaN where P V is infinite.  So a NaN anywhere in the wavefront's
+  // result runs its pages again with only the first term meeting such values.
+  if constexpr (PARTS > 1) {
+    bool nan = false;
+#pragma unroll
+    for (int t = 0; t < DT; ++t)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) nan |= o[t][i] != o[t][i];
+    if (__any(nan)) pages(std::true_type{});
   }
   if (bad) *err = 1;
   // bring l and O from mr to m
