@@ -365,8 +365,9 @@ int ktir_launch_row_rmw_noalloc(const ktir_rmw_t* d);
  * are 64 or 128 (any combination), bf16 or f16 Q/K/V, MFMA with f32
  * accumulation.  M = N = D = 128: P enters the P @ V product as a hi + lo
  * pair of operand-type values (about 16 significant bits), or as v16_ptr
- * says below; the other shapes carry P as two f16 or three bf16 terms (22 /
- * 24 bits), use no f16 copy of V, and need K and V rows less than 2^23
+ * says below; the other shapes carry P as two f16 or three bf16 terms (23 /
+ * 24 bits; a step with a P below 2^-15 of its row's largest adds what two f16
+ * terms leave), use no f16 copy of V, and need K and V rows less than 2^23
  * elements apart. */
 typedef struct ktir_attn {
   int64_t lanes, M, N, D;

@@ -524,27 +524,38 @@ _FA_MASK = """      %sm_init = tensor.empty() : {Sf}
 
 
 def flash_attention(B: int = 4, H: int = 32, S: int = 8192, D: int = 128, blk: int = 128, dt: str = "bf16",
-                    causal: bool = True) -> str:
+                    causal: bool = True, kblk: int = 0) -> str:
     """O = softmax(Q K^T * scale, causal) V with online softmax over KV tiles.
 
     Grid [S/blk, H, B]; core (qb, h, b) owns query rows [qb*blk, (qb+1)*blk)
     of head (b, h) and visits KV tiles 0..qb (the causal prefix), or all
-    S/blk tiles when `causal` is False.
+    S/blk tiles when `causal` is False.  `kblk`: keys per tile (default blk).
     """
     nq = S // blk
+    kb = kblk or blk
     shp = [B, H, S, D]
     strides = [H * S * D, S * D, D, 1]
     T4 = _t([1, 1, blk, D], dt)
     Tb, Tf = _t([blk, D], dt), _t([blk, D], "f32")
-    Sf = _t([blk, blk], "f32")
-    Vf = _t([blk], "f32")
+    K4, Kb, Kf = _t([1, 1, kb, D], dt), _t([kb, D], dt), _t([kb, D], "f32")
+    Sf = _t([blk, kb], "f32")
+    KTf, Vf = _t([D, kb], "f32"), _t([blk], "f32")
     at = f"!ktdp.access_tile<1x1x{blk}x{D}xindex>"
-    n_kv = "arith.addi %qb, %c1 : index" if causal else f"arith.constant {nq} : index"
+    atk = f"!ktdp.access_tile<1x1x{kb}x{D}xindex>"
+    n_kv = "arith.addi %qb, %c1 : index" if causal else f"arith.constant {S // kb} : index"
+    if causal and kb != blk:
+        n_kv = "arith.divui %q_end, %KBLK : index"
     sm = "%sm" if causal else "%s"
     mask = _FA_MASK.format(Sf=Sf) if causal else ""
 
     def tile(name, view, row):
-        return _tile(name, view, ["%b", "%h", row, "%c0"], [1, 1, blk, D], shp, dt, "      ")
+        return _tile(name, view, ["%b", "%h", row, "%c0"], [1, 1, kb, D], shp, dt, "      ")
+
+    # the tiles that hold keys up to the last row's position
+    bounds = f"""
+    %KBLK = arith.constant {kb} : index
+    %last_k = arith.constant {blk + kb - 1} : index
+    %q_end = arith.addi %q0, %last_k : index""" if kb != blk else ""
 
     return f"""module {{
   func.func @flash_attention(%q_ptr: index, %k_ptr: index, %v_ptr: index, %o_ptr: index, %scale: f32)
@@ -568,22 +579,22 @@ def flash_attention(B: int = 4, H: int = 32, S: int = 8192, D: int = 128, blk: i
     %m_init = tensor.splat %neg_inf : {Vf}
     %l_init = tensor.splat %zero : {Vf}
     %acc_init = tensor.splat %zero : {Tf}
-    %n_kv = {n_kv}
+{bounds[1:]}{bounds and chr(10)}    %n_kv = {n_kv}
     %m_f, %l_f, %acc_f = scf.for %j = %c0 to %n_kv step %c1
         iter_args(%m = %m_init, %l = %l_init, %acc = %acc_init) -> ({Vf}, {Vf}, {Tf}) {{
-      %k0 = arith.muli %j, %BLK : index
+      %k0 = arith.muli %j, {'%BLK' if kb == blk else '%KBLK'} : index
 {tile("k_acc", "k_view", "%k0")}
 {tile("v_acc", "v_view", "%k0")}
-      %k4 = ktdp.load %k_acc : {at} -> {T4}
-      %v4 = ktdp.load %v_acc : {at} -> {T4}
-      %k2 = tensor.collapse_shape %k4 [[0, 1, 2], [3]] : {T4} into {Tb}
-      %v2 = tensor.collapse_shape %v4 [[0, 1, 2], [3]] : {T4} into {Tb}
-      %kf = arith.extf %k2 : {Tb} to {Tf}
-      %vf = arith.extf %v2 : {Tb} to {Tf}
-      %kt_init = tensor.empty() : {_t([D, blk], "f32")}
-      %kt = linalg.transpose ins(%kf : {Tf}) outs(%kt_init : {_t([D, blk], "f32")}) permutation = [1, 0]
+      %k4 = ktdp.load %k_acc : {atk} -> {K4}
+      %v4 = ktdp.load %v_acc : {atk} -> {K4}
+      %k2 = tensor.collapse_shape %k4 [[0, 1, 2], [3]] : {K4} into {Kb}
+      %v2 = tensor.collapse_shape %v4 [[0, 1, 2], [3]] : {K4} into {Kb}
+      %kf = arith.extf %k2 : {Kb} to {Kf}
+      %vf = arith.extf %v2 : {Kb} to {Kf}
+      %kt_init = tensor.empty() : {KTf}
+      %kt = linalg.transpose ins(%kf : {Kf}) outs(%kt_init : {KTf}) permutation = [1, 0]
       %s_init = tensor.splat %zero : {Sf}
-      %qk = linalg.matmul ins(%q, %kt : {Tf}, {_t([D, blk], "f32")}) outs(%s_init : {Sf}) -> {Sf}
+      %qk = linalg.matmul ins(%q, %kt : {Tf}, {KTf}) outs(%s_init : {Sf}) -> {Sf}
       %s = arith.mulf %scale_t, %qk : {Sf}
 {mask}      %rm_init = tensor.splat %neg_inf : {Vf}
       %rm = linalg.reduce {{ arith.maximumf }} ins({sm} : {Sf}) outs(%rm_init : {Vf}) dimensions = [1]
@@ -611,7 +622,7 @@ def flash_attention(B: int = 4, H: int = 32, S: int = 8192, D: int = 128, blk: i
           %sc = arith.mulf %av, %al : f32
           linalg.yield %sc : f32
       }} -> {Tf}
-      %acc_n = linalg.matmul ins(%p, %vf : {Sf}, {Tf}) outs(%accs : {Tf}) -> {Tf}
+      %acc_n = linalg.matmul ins(%p, %vf : {Sf}, {Kf}) outs(%accs : {Tf}) -> {Tf}
       %la = arith.mulf %l, %alpha : {Vf}
       %l_n = arith.addf %la, %ls : {Vf}
       scf.yield %m_new, %l_n, %acc_n : {Vf}, {Vf}, {Tf}

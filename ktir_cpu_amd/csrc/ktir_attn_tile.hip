@@ -10,21 +10,23 @@
 //   S^T = K Q^T     A = K rows from LDS, B = Q^T in registers, so a query row's
 //                   scores lie in lanes l and l ^ 32;
 //   softmax         row max and sum in the lane and one exchange, P, l and O kept
-//                   relative to a base mr <= m that moves when m passes it by 8;
+//                   relative to a base 2^b that moves when e^m passes it by P_LAG;
 //   O^T += V^T P^T  V^T by transposing LDS reads, the keys in the order in which
 //                   a lane's own scores are its P fragment.
-// P stays as exact as the f32 P of the op-by-op loop: it enters P V as two f16
-// terms (22 bits) or three bf16 terms (24 bits) whose exact products the MFMA
-// adds in f32.
+// P, f32 in the op-by-op loop, enters P V as three bf16 terms (24 bits) or, in
+// f16, as two terms (23 bits) and, in a step with a P below 2^-15, the rest
+// of them too (ktir_attn_common.h): results from float64 by no more than one
+// rounding of their type and f32's of the exponentials, as the loop's are.
 //
 // K and V tiles are double-buffered in LDS: tile j + 1 streams in (buffer_load
 // ... lds, no registers) while tile j is computed, one barrier per tile.  A
 // 64 x 64 x 64 step stages 16 KB for 24 MFMAs and about 300 vector
 // instructions per wavefront and takes 32 KB of LDS, so several workgroups
 // share a CU and one's softmax runs under another's MFMAs.  The vector
-// instructions bound it (the exact split of P takes as many as the
-// exponentials).  Where no CU has a second workgroup, the key tiles go to two
-// groups of four wavefronts, whose states meet in LDS at the end.  Full attention
+// instructions bound it (the split of P takes as many as the exponentials, the
+// test for small P 3 to 4 % of the time).  Where no CU has a second workgroup,
+// the key tiles go to two groups of four wavefronts, whose states meet in LDS at
+// the end.  Full attention
 // of 2048 x 64, f16, 64 x 64 tiles: 16 heads 33.9 us (510 TFLOP/s), 40 with one
 // group, and 43.4 ms for the loop's about 450 launches; 32 heads (two workgroups
 // per CU) 68.7 us.
@@ -33,18 +35,6 @@
 #include "ktir_attn_common.h"
 
 namespace ktir {
-
-// Slot permutation of a tile row's 16-byte chunks: 8 chunks for 128-byte rows
-// (64 columns), 16 for 256-byte rows (128 columns).  Both are XORs of row bits
-// chosen so that 8 rows' same chunk (ds_read_b128 of K) and 4 rows' 32-byte
-// pieces (ds_read_b64_tr_b16 of V) lie in distinct banks.
-template <int D>
-__device__ __forceinline__ int att_swz(int r) {
-  if constexpr (D == 64)
-    return ((r & 1) << 1) ^ ((r & 2) << 1) ^ ((r >> 2) & 1) ^ (((r >> 3) & 1) << 1);
-  else
-    return ((r & 1) ? 4 : 0) ^ ((r & 2) ? 10 : 0) ^ ((r & 4) ? 1 : 0) ^ ((r & 8) ? 8 : 0);
-}
 
 // Wavefront w (uniform, 0..3) copies rows N/4 w .. + N/4 of an N x D tile into
 // LDS in 1 KB blocks of 512 / D rows: lane l fills slot l % (D / 8) of its row.
@@ -57,28 +47,9 @@ __device__ __forceinline__ void att_stage(const uint16_t* src, int64_t row_strid
 #pragma unroll
   for (int i = 0; i < RW / RB; ++i) {
     // a wavefront's rows start at a multiple of 16, so row % 16 is known here
-    const int x = c ^ att_swz<D>((RB * i + r) & 15);
+    const int x = c ^ kv_swz<D>((RB * i + r) & 15);
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void*)(lds + D * (RW * w + RB * i)),
                                              16, (int)((r * row_stride + 8 * x) * 2), (int)(i * RB * row_stride * 2), 0, 0);
-  }
-}
-
-// four values as PARTS terms of the operand type, largest first: t[p] holds
-// (x0, x1) and (x2, x3) packed
-template <bool BF16, int PARTS>
-__device__ __forceinline__ void att_split(const float* x, uint32_t (&t)[PARTS][2]) {
-  float r[4] = {x[0], x[1], x[2], x[3]};
-#pragma unroll
-  for (int p = 0; p < PARTS; ++p) {
-    t[p][0] = cvt2<BF16>(r[0], r[1]);
-    t[p][1] = cvt2<BF16>(r[2], r[3]);
-    if (p + 1 < PARTS) {
-      const f32x2_t a = uncvt2<BF16>(t[p][0]), b = uncvt2<BF16>(t[p][1]);
-      r[0] = __fsub_rn(r[0], a.x);
-      r[1] = __fsub_rn(r[1], a.y);
-      r[2] = __fsub_rn(r[2], b.x);
-      r[3] = __fsub_rn(r[3], b.y);
-    }
   }
 }
 
@@ -126,14 +97,14 @@ __global__ __launch_bounds__(256 * G, G == 1 && N * D == 64 * 64 ? 3 : 2) void a
   const float c1 = __fmul_rn(d.scale, LOG2E);
   const f32x16_t z16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   f32x16_t o[DT];                                   // O^T tiles: d = 32 dt + 8 g + 4 h + t, row r32
-  float m, mr, lsum;
-  const int k_off = r32 * D, k_x = att_swz<D>(r32 & 15);
+  float m, b, lsum;                                 // b: the base 2^b of P, l and O (at most 2^P_LAG below e^m)
+  const int k_off = r32 * D, k_x = kv_swz<D>(r32 & 15);
   // V^T fragment: member tj of 16-lane group tg addresses key 4 (tg / 2) + tj / 4
   // (+ 8) of the 16-key step, columns 16 (tg % 2) + 4 (tj % 4) of a 32-column tile
   const int tg = l >> 4, tj = l & 15;
   const int v_row0 = 4 * (tg >> 1) + (tj >> 2);
   const int v_c = 2 * (tg & 1) + ((tj >> 1) & 1), v_in = 4 * (tj & 1);
-  const int v_b0 = v_row0 * D + v_in, v_x0 = v_c ^ att_swz<D>(v_row0), v_x1 = v_c ^ att_swz<D>(v_row0 + 8);
+  const int v_b0 = v_row0 * D + v_in, v_x0 = v_c ^ kv_swz<D>(v_row0), v_x1 = v_c ^ kv_swz<D>(v_row0 + 8);
 
   auto step = [&](auto inf_v, int j, const uint16_t* Kc, const uint16_t* Vc, uint16_t* Kn,
                   uint16_t* Vn) __attribute__((always_inline)) {
@@ -157,7 +128,7 @@ __global__ __launch_bounds__(256 * G, G == 1 && N * D == 64 * 64 ? 3 : 2) void a
       const bool all_keep = !d.causal ||
           (minv ? (dbase + N - 1 < mlo || dbase > mhi) : (dbase >= mlo && dbase + N - 1 <= mhi));
       // no masked score in the wavefront and scale > 0: row max of S = scale *
-      // row max of Q K^T, and P = 2^(QK scale log2e - mr log2e)
+      // row max of Q K^T, and P = 2^(QK scale log2e - b)
       const bool fast = pos_scale && __all(all_keep);
       if (!fast) {
 #pragma unroll
@@ -185,30 +156,51 @@ __global__ __launch_bounds__(256 * G, G == 1 && N * D == 64 * 64 ? 3 : 2) void a
       for (int kt = 1; kt < KT; ++kt) xm = fmax_nan(xm, x[kt]);
       xm = pair_max(xm);
       const float mn = fmax_nan(m, fast ? __fmul_rn(d.scale, xm) : xm);
-      const bool up = mn > __fadd_rn(mr, 8.0f);
+      const float bn = __fmul_rn(mn, LOG2E);
+      const bool up = bn > __fadd_rn(b, P_LAG<BF16>);
       if (__any(up)) {
-        const float al = up ? exp_f(__fsub_rn(mr, mn)) : 1.f;
+        const float al = up ? exp2_f(__fsub_rn(b, bn)) : 1.f;
 #pragma unroll
         for (int t = 0; t < DT; ++t)
 #pragma unroll
           for (int i = 0; i < 16; ++i) o[t][i] = __fmul_rn(o[t][i], al);
         lsum = __fmul_rn(lsum, al);
-        mr = up ? mn : mr;
+        b = up ? bn : b;
       }
       // a group without tile 0 whose scores have all been -inf: P is 0 against
       // any base (with tile 0 it is the loop's exp(-inf - (-inf)), NaN)
-      const float mb = G > 1 && grp && mn == -__builtin_inff() ? 0.f : mr;
+      const float pb = G > 1 && grp && mn == -__builtin_inff() ? 0.f : b;
       if (fast) {
-        const float c0 = -__fmul_rn(mb, LOG2E);
 #pragma unroll
         for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
-          for (int i = 0; i < 16; ++i) sc[kt][i] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[kt][i], c1, c0));
+          for (int i = 0; i < 16; ++i) sc[kt][i] = exp2_f(__builtin_fmaf(sc[kt][i], c1, -pb));
       } else {
 #pragma unroll
         for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
-          for (int i = 0; i < 16; ++i) sc[kt][i] = exp_f(__fsub_rn(sc[kt][i], mb));
+          for (int i = 0; i < 16; ++i) sc[kt][i] = exp2_f(__builtin_fmaf(sc[kt][i], LOG2E, -pb));
+      }
+      // whether a P of this tile is too small for two f16 terms
+      bool small = false;
+      if constexpr (!BF16 && !INF_V) {
+        float least = 1.f;
+        if (fast) {
+#pragma unroll
+          for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+            for (int i = 0; i < 16; i += 2)
+              least = fmin3_nan(least, sc[kt][i], sc[kt][i + 1]);
+        } else {
+#pragma unroll
+          for (int kt = 0; kt < KT; ++kt) {
+            float p[16];
+#pragma unroll
+            for (int i = 0; i < 16; ++i) p[i] = sc[kt][i];
+            least = fminf(least, least_positive<16>(p));
+          }
+        }
+        small = __any(least < P_SMALL);
       }
       float a0 = 0.f, a1 = 0.f, a2 = 0.f, a3 = 0.f;
 #pragma unroll
@@ -222,33 +214,48 @@ __global__ __launch_bounds__(256 * G, G == 1 && N * D == 64 * 64 ? 3 : 2) void a
         }
       lsum = __fadd_rn(lsum, pair_sum(__fadd_rn(__fadd_rn(a0, a1), __fadd_rn(a2, a3))));
       m = mn;
+      // P V: by the terms of the operand type, by the rest they leave (f16) or by
+      // bf16 terms of the whole P (f16, infinities in V)
+      enum { TERMS, REST, WHOLE };
+      auto pv = [&](auto how) __attribute__((always_inline)) {
+        constexpr int HOW = decltype(how)::value;
 #pragma unroll
-      for (int ks = 0; ks < N / 16; ++ks) {
-        const int kt = ks >> 1, g0 = 2 * (ks & 1);
-        const uint16_t* vt = &Vc[16 * ks * D];
-        float p[8];
+        for (int ks = 0; ks < N / 16; ++ks) {
+          const int kt = ks >> 1, g0 = 2 * (ks & 1);
+          const uint16_t* vt = &Vc[16 * ks * D];
+          float p[8];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) p[i] = sc[kt][4 * g0 + i];
-        uint32_t t0[PARTS][2], t1[PARTS][2];
-        att_split<BF16, PARTS>(p, t0);
-        att_split<BF16, PARTS>(p + 4, t1);
-        if constexpr (INF_V && !BF16) {
-          // a positive P below f16's range still times an infinite V is infinite
-          lift4(p, t0[0]);
-          lift4(p + 4, t1[0]);
+          for (int i = 0; i < 8; ++i) {
+            p[i] = sc[kt][4 * g0 + i];
+            if constexpr (HOW == REST) asm volatile("" : "+v"(p[i]));   // nothing kept for it from the terms
+            if constexpr (HOW == WHOLE) p[i] = __fmul_rn(p[i], P_SCALE<BF16>);
+          }
+          uint32_t t0[PARTS][2], t1[PARTS][2];
+          uint4 tb[3];
+          if constexpr (HOW != WHOLE) {
+            p_split<BF16, PARTS, HOW == REST>(p, t0);
+            p_split<BF16, PARTS, HOW == REST>(p + 4, t1);
+          }
+          if constexpr (HOW != TERMS) p_split_bf(p, tb);
+#pragma unroll
+          for (int dt = 0; dt < DT; ++dt) {
+            const uint2 lo = ds_tr16(vt + v_b0 + 8 * ((4 * dt) ^ v_x0));
+            const uint2 hi = ds_tr16(vt + v_b0 + 8 * D + 8 * ((4 * dt) ^ v_x1));
+            const uint4 a = make_uint4(lo.x, lo.y, hi.x, hi.y);
+            if constexpr (HOW == TERMS) {
+              o[dt] = pv_mfma<BF16, PARTS, INF_V>(a, t0, t1, o[dt]);
+            } else {
+              o[dt] = pv_mfma_bf<INF_V>(a, tb, o[dt]);
+              __builtin_amdgcn_sched_barrier(0);   // rare: must not set the register count
+            }
+          }
         }
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) {
-          const uint2 lo = ds_tr16(vt + v_b0 + 8 * ((4 * dt) ^ v_x0));
-          const uint2 hi = ds_tr16(vt + v_b0 + 8 * D + 8 * ((4 * dt) ^ v_x1));
-          const uint4 a = make_uint4(lo.x, lo.y, hi.x, hi.y);
-          uint4 af = a;
-          if constexpr (INF_V)
-            af = make_uint4(finite2<BF16>(a.x), finite2<BF16>(a.y), finite2<BF16>(a.z), finite2<BF16>(a.w));
-#pragma unroll
-          for (int q = PARTS - 1; q >= 0; --q)
-            o[dt] = mfma_at<BF16>(q ? af : a, make_uint4(t0[q][0], t0[q][1], t1[q][0], t1[q][1]), o[dt]);
-        }
+      };
+      if constexpr (!BF16 && INF_V) {
+        pv(std::integral_constant<int, WHOLE>{});
+      } else {
+        pv(std::integral_constant<int, TERMS>{});
+        if (small) pv(std::integral_constant<int, REST>{});
       }
     }
     __builtin_amdgcn_s_waitcnt(0);                  // this wavefront's part of the next tile has landed
@@ -257,7 +264,7 @@ __global__ __launch_bounds__(256 * G, G == 1 && N * D == 64 * 64 ? 3 : 2) void a
   auto loop = [&](auto inf_v) __attribute__((always_inline)) {
 #pragma unroll
     for (int t = 0; t < DT; ++t) o[t] = z16;
-    m = mr = -__builtin_inff();
+    m = b = -__builtin_inff();
     lsum = 0.f;
     if (grp < Tmax) {
       att_stage<N, D>(K + (int64_t)grp * d.k_step, d.k_row, K0s, w, l);
@@ -295,14 +302,14 @@ __global__ __launch_bounds__(256 * G, G == 1 && N * D == 64 * 64 ? 3 : 2) void a
         for (int g = 0; g < 4; ++g)
           *ex(4 * t + g) = make_float4(o[t][4 * g], o[t][4 * g + 1], o[t][4 * g + 2], o[t][4 * g + 3]);
       exs[0] = m;
-      exs[256] = mr;
+      exs[256] = b;
       exs[512] = lsum;
     }
     __syncthreads();
     if (grp == 1) return;
     if (T > 0) {
-      const float m1 = exs[0], mm = fmax_nan(m, m1);
-      const float w0 = exp_f(__fsub_rn(mr, mm)), w1 = m1 == -__builtin_inff() ? 0.f : exp_f(__fsub_rn(exs[256], mm));
+      const float m1 = exs[0], mm = fmax_nan(m, m1), bm = __fmul_rn(mm, LOG2E);
+      const float w0 = exp2_f(__fsub_rn(b, bm)), w1 = m1 == -__builtin_inff() ? 0.f : exp2_f(__fsub_rn(exs[256], bm));
 #pragma unroll
       for (int t = 0; t < DT; ++t)
 #pragma unroll
@@ -314,18 +321,20 @@ __global__ __launch_bounds__(256 * G, G == 1 && N * D == 64 * 64 ? 3 : 2) void a
           o[t][4 * g + 3] = __fadd_rn(__fmul_rn(o[t][4 * g + 3], w0), __fmul_rn(x.w, w1));
         }
       lsum = __fadd_rn(__fmul_rn(lsum, w0), __fmul_rn(exs[512], w1));
-      m = mr = mm;
+      m = mm;
+      b = bm;
     }
   }
   if (lane < 0) return;
   if (T > 0) {
-    // bring P, l and O from mr to m
-    const float fin = exp_f(__fsub_rn(mr, m));
-    if (!__all(fin == 1.f)) {
+    // bring l and O from 2^b to e^m, and O from P's scale
+    const float fin = exp2_f(__builtin_fmaf(-m, LOG2E, b));
+    if (!BF16 || !__all(fin == 1.f)) {
+      const float f = __fmul_rn(fin, 1.f / P_SCALE<BF16>);
 #pragma unroll
       for (int t = 0; t < DT; ++t)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) o[t][i] = __fmul_rn(o[t][i], fin);
+        for (int i = 0; i < 16; ++i) o[t][i] = __fmul_rn(o[t][i], f);
       lsum = __fmul_rn(lsum, fin);
     }
   }

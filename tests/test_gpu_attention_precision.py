@@ -1,0 +1,158 @@
+"""The fused attention launches against float64 where fewer bits of P, or of
+its exponent, would show: a heavy key without a value, scores far from zero,
+and every accepted tile shape with a tolerance of the output's rounding."""
+import numpy as np
+import pytest
+
+from ktir_cpu_amd import configs
+from ktir_cpu_amd import runtime as rt
+from oracle.interp import bf16_bits, bf16_from_bits
+
+pytestmark = pytest.mark.gpu
+
+# rows, keys, columns of the dense kernel's tiles of 64 or 128
+SHAPES = [(m, n, d) for m in (64, 128) for n in (64, 128) for d in (64, 128) if (m, n, d) != (128, 128, 128)]
+# half a unit of the output type, relative; half the spacing of its smallest values
+HALF = {"f16": (2.0 ** -11, 2.0 ** -25), "bf16": (2.0 ** -8, 0.0), "f32": (2.0 ** -24, 0.0)}
+
+
+def _bits(x, dt):
+    return bf16_bits(np.asarray(x, np.float32)) if dt == "bf16" else np.asarray(x, np.float16)
+
+
+def _f64(x):
+    return (bf16_from_bits(x) if x.dtype == np.uint16 else x).astype(np.float64)
+
+
+def _prepare(src, fn, kw):
+    from ktir_cpu_amd.interpreter import KTIRInterpreter
+    it = KTIRInterpreter()
+    it.load(src)
+    prep = it.prepare(fn, **kw)
+    (d,) = [x[1] for x in prep.plan.launches if x[0] in ("attn", "pattn")]
+    return prep, d
+
+
+def _device(ptr, n):
+    out = np.empty(n, np.float32)
+    rt.check(rt.lib().ktir_memcpy_d2h(out.ctypes.data, ptr, out.nbytes), "ktir_memcpy_d2h")
+    return out.astype(np.float64)
+
+
+def _dense(q, k, v, scale, causal):
+    """float64 attention, and the sum of P |V| that a relative error of P acts on."""
+    s = np.einsum("bhid,bhjd->bhij", q, k) * scale
+    if causal:
+        s = np.where(np.tril(np.ones(s.shape[-2:])) > 0, s, -np.inf)
+    p = np.exp(s - s.max(-1, keepdims=True))
+    p /= p.sum(-1, keepdims=True)
+    return p @ v, p @ np.abs(v)
+
+
+def _near(got, want, dt, spread, p_err=2.0 ** -21):
+    """One rounding to `dt`, after errors of `p_err` of every P (f32
+    exponentials and sums of them: a few units each)."""
+    half, tiny = HALF[dt]
+    assert (np.abs(got - want) <= half * np.abs(want) * 1.001 + tiny + p_err * spread).all(), \
+        (np.abs(got - want) / (half * np.abs(want) + tiny + p_err * spread)).max()
+
+
+def _exp_err(gap):
+    """Of an f32 exponential of -gap: its argument times log2 e is off by up to
+    2^-24 of itself, the hardware's exp2 by a unit; the same again for l."""
+    return gap * 2.0 ** -23 + 2.0 ** -21
+
+
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("causal,S", [(True, 384), (False, 256), (True, 128)])
+@pytest.mark.parametrize("M,N,D", SHAPES)
+def test_tiles_of_every_shape(M, N, D, causal, S, dt):
+    rng = np.random.default_rng(M + N + D)
+    q, k, v = (_bits(rng.standard_normal((1, 3, S, D)), dt) for _ in range(3))
+    prep, d = _prepare(configs.flash_attention(1, 3, S, D, M, dt, causal, N), "flash_attention",
+                       dict(q_ptr=q, k_ptr=k, v_ptr=v, o_ptr=np.zeros_like(q), scale=D ** -0.5))
+    assert (d.M, d.N, d.D) == (M, N, D) and dict(prep.plan.counts()) == {"attn": 1}
+    want, spread = _dense(_f64(q), _f64(k), _f64(v), D ** -0.5, causal)
+    _near(_f64(prep.outputs()["o_ptr"]), want, dt, spread)
+
+
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("M,N,D", [(64, 128, 64), (128, 64, 128)])
+def test_tiles_of_wider_rows(M, N, D, dt):
+    """Q, K, V and O as columns of wider arrays: rows 8 elements further apart."""
+    rng = np.random.default_rng(5)
+    S, W = 2 * max(M, N), D + 8
+    wide = [_bits(rng.standard_normal((1, 2, S, W)), dt) for _ in range(3)]
+    src = configs.flash_attention(1, 2, S, D, M, dt, False, N)
+    old, new = f"sizes: [1, 2, {S}, {D}], strides: [{2 * S * D}, {S * D}, {D}, 1]", \
+        f"sizes: [1, 2, {S}, {D}], strides: [{2 * S * W}, {S * W}, {W}, 1]"
+    assert src.count(old) == 4
+    prep, d = _prepare(src.replace(old, new), "flash_attention",
+                       dict(zip(("q_ptr", "k_ptr", "v_ptr"), wide), o_ptr=np.zeros_like(wide[0]), scale=D ** -0.5))
+    assert (d.q_row, d.k_row, d.v_row, d.o_row) == (W,) * 4
+    got = _f64(prep.outputs()["o_ptr"])
+    want, spread = _dense(*(_f64(x)[..., :D] for x in wide), D ** -0.5, False)
+    _near(got[..., :D], want, dt, spread)
+    assert (got[..., D:] == 0).all()
+
+
+def _sink(S, D, at, gap, value):
+    """q, k, v of one head: key `at` scores `gap` more than the others and has V = 0."""
+    q, k = np.zeros((S, D)), np.zeros((S, D))
+    q[:, 0] = 8.0
+    k[at, 0] = gap / 8.0
+    v = np.broadcast_to(value * (1.0 + np.arange(D) / 128.0), (S, D)).copy()
+    v[at] = 0.0
+    return q, k, v
+
+
+@pytest.mark.parametrize("out_dt", ["own", "f32"])
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("gap", [9.0, 14.0, 16.5, 24.0])
+@pytest.mark.parametrize("at", [3, 500])
+@pytest.mark.parametrize("M,N,D", [(64, 64, 64), (128, 128, 64), (64, 64, 128)])
+def test_tiles_heavy_key_without_value(M, N, D, at, gap, dt, out_dt):
+    """Every result is made of keys that weigh e^-gap: their P has to hold its
+    bits there, not only next to 1."""
+    S = 512
+    q, k, v = (_bits(x[None, None], dt) for x in _sink(S, D, at, gap, 250.0))
+    src = configs.flash_attention(1, 1, S, D, M, dt, False, N)
+    o = np.zeros_like(q)
+    if out_dt == "f32":
+        tail = src[src.index("%o_init"):]
+        f32 = tail.replace("    %ob = arith.truncf", "    %unused = arith.truncf").replace("%ob [[", "%of [[") \
+            .replace(f"tensor<{M}x{D}x{dt}> into", f"tensor<{M}x{D}xf32> into").replace(f"1x1x{M}x{D}x{dt}>", f"1x1x{M}x{D}xf32>") \
+            .replace(f"{S}x{D}x{dt}>", f"{S}x{D}xf32>")
+        head = src[:src.index("%o_init")]
+        i = head.index("%o_view =")
+        head = head[:i] + head[i:].replace(f"x{dt}>", "xf32>", 1)
+        src, o = head + f32, np.zeros(q.shape, np.float32)
+    prep, d = _prepare(src, "flash_attention", dict(q_ptr=q, k_ptr=k, v_ptr=v, o_ptr=o, scale=1.0))
+    assert (d.M, d.N, d.D) == (M, N, D)
+    want, spread = _dense(_f64(q), _f64(k), _f64(v), 1.0, False)
+    _near(_f64(prep.outputs()["o_ptr"]), want, dt if out_dt == "own" else "f32", spread, _exp_err(gap))
+
+
+def _far_scores(S, D, steps):
+    """q and k of exact scores near 7600 that rise by 3/4 from step to step of `steps` keys."""
+    q, k = np.zeros((S, D)), np.zeros((S, D))
+    q[:, 0], q[:, 1] = 4.0, 1.0
+    k[:, 0] = 1900.0
+    j = np.arange(S)
+    k[:, 1] = (j // steps) * 0.75 - (j * 7 % 13) / 8.0
+    return q, k
+
+
+@pytest.mark.parametrize("M,N,D", [(64, 64, 64), (128, 64, 128), (128, 128, 64)])
+def test_tiles_row_sum_of_far_scores(M, N, D):
+    """exp(S - m) of scores near 7600: the row sum as exact as of scores near 0,
+    also across the rows' moves of the base."""
+    S = 512
+    q, k = _far_scores(S, D, N)
+    rng = np.random.default_rng(1)
+    q, k, v = (_bits(x[None, None], "f16") for x in (q, k, rng.standard_normal((S, D))))
+    prep, d = _prepare(configs.flash_attention(1, 1, S, D, M, "f16", False, N), "flash_attention",
+                       dict(q_ptr=q, k_ptr=k, v_ptr=v, o_ptr=np.zeros_like(q), scale=1.0))
+    s = (_f64(q)[0, 0] @ _f64(k)[0, 0].T)[0]
+    np.testing.assert_array_equal(_device(d.m_out, S), np.full(S, s.max()))
+    np.testing.assert_allclose(_device(d.l_out, S), np.full(S, np.exp(s - s.max()).sum()), rtol=4e-6)
