@@ -60,16 +60,7 @@ __device__ __forceinline__ uint32_t finite2(uint32_t w) {
   return lo | hi;
 }
 
-// the smallest f16 in the place of a leading term 0 whose value is positive
-__device__ __forceinline__ void lift4(const float* p, uint32_t (&t)[2]) {
-#pragma unroll
-  for (int k = 0; k < 2; ++k) {
-    if (p[2 * k] > 0.f && !(t[k] & 0xffffu)) t[k] |= 1u;
-    if (p[2 * k + 1] > 0.f && !(t[k] >> 16)) t[k] |= 0x10000u;
-  }
-}
-
-// P in the P V products of ktir_attn_tile.hip.  The
+// P in the P V products of ktir_attn_tile.hip and ktir_pattn_split.hip.  The
 // loop holds P in f32; here it enters as terms of a 16-bit type whose products
 // are exact and are summed in f32.
 //   bf16: the terms have f32's exponents; three of them hold P's 24 bits.

@@ -12,11 +12,13 @@
 // nothing until the end, run without barriers, and a single query row of a
 // decode step keeps the whole chip busy.  Per pair, as in ktir_attn_tile.hip:
 //   S^T = K Q^T (32 x 32 x 16 MFMA), masked and scaled in f32,
-//   m, l and O of the wavefront's keys (online softmax, O relative to mr <= m),
+//   m, l and O of the wavefront's keys (online softmax, O relative to a base 2^b),
 //   O^T += V^T P^T.
 // P enters P V as PARTS terms of the operand type: one f16 / two bf16 terms for
-// lanes of at most 16 rows (as the one-wavefront kernel), one more for others
-// (whose f32 kernel holds P exactly).
+// lanes of at most 16 rows (as the one-wavefront kernel), one more for others,
+// whose f32 kernel holds P exactly: 24 bits in bf16, 23 in f16, and the rest of
+// them too in a step with a P below 2^-15 (ktir_attn_common.h; the test for it
+// takes 2 % of 256 tokens of 32 rows a lane after 1024, 40 us).
 // Pages move HBM -> LDS (buffer_load ... lds) into the wavefront's own 16 KB
 // (128 columns): the next pair's K while this pair's softmax and P V run, its V
 // while the next scores are computed; two workgroups of four (or one of eight) share a CU.
@@ -39,15 +41,6 @@
 namespace ktir {
 
 constexpr int PS_ROWS = 32, PS_KEYS = 32;
-
-// slot permutation of a key row's 16-byte chunks (as att_swz in ktir_attn_tile.hip)
-template <int D>
-__device__ __forceinline__ int ps_swz(int r) {
-  if constexpr (D == 64)
-    return ((r & 1) << 1) ^ ((r & 2) << 1) ^ ((r >> 2) & 1) ^ (((r >> 3) & 1) << 1);
-  else
-    return ((r & 1) ? 4 : 0) ^ ((r & 2) ? 10 : 0) ^ ((r & 4) ? 1 : 0) ^ ((r & 8) ? 8 : 0);
-}
 
 __device__ __forceinline__ int64_t ps_index(uint64_t ptr, int64_t e, int dt) {
   switch (dt) {
@@ -116,7 +109,7 @@ __device__ __forceinline__ void ps_dma(uint64_t ptr, int64_t e0, int64_t row, bo
   const int r = l / CH, c = l % CH;
   uint32_t off[16 / RB];
 #pragma unroll
-  for (int i = 0; i < 16 / RB; ++i) off[i] = (uint32_t)(((RB * i + r) * row + 8 * (c ^ ps_swz<D>((RB * i + r) & 15))) * 2);
+  for (int i = 0; i < 16 / RB; ++i) off[i] = (uint32_t)(((RB * i + r) * row + 8 * (c ^ kv_swz<D>((RB * i + r) & 15))) * 2);
   ps_load<16 / RB>(rs, off, lds + 2 * D * row0);
 }
 
@@ -128,25 +121,7 @@ __device__ __forceinline__ void ps_copy(uint64_t ptr, int64_t e0, int64_t row, i
   for (int i = l; i < 16 * D; i += 64) {
     const int r = i / D, c = i % D;
     const int64_t e = e0 + r * row + c;
-    lds[D * (row0 + r) + 8 * ((c >> 3) ^ ps_swz<D>(r)) + (c & 7)] = (e >= lo && e < hi) ? p[e] : (uint16_t)0;
-  }
-}
-
-// four values as PARTS terms of the operand type, largest first
-template <bool BF16, int PARTS>
-__device__ __forceinline__ void ps_split(const float* x, uint32_t (&t)[PARTS][2]) {
-  float r[4] = {x[0], x[1], x[2], x[3]};
-#pragma unroll
-  for (int p = 0; p < PARTS; ++p) {
-    t[p][0] = cvt2<BF16>(r[0], r[1]);
-    t[p][1] = cvt2<BF16>(r[2], r[3]);
-    if (p + 1 < PARTS) {
-      const f32x2_t a = uncvt2<BF16>(t[p][0]), b = uncvt2<BF16>(t[p][1]);
-      r[0] = __fsub_rn(r[0], a.x);
-      r[1] = __fsub_rn(r[1], a.y);
-      r[2] = __fsub_rn(r[2], b.x);
-      r[3] = __fsub_rn(r[3], b.y);
-    }
+    lds[D * (row0 + r) + 8 * ((c >> 3) ^ kv_swz<D>(r)) + (c & 7)] = (e >= lo && e < hi) ? p[e] : (uint16_t)0;
   }
 }
 
@@ -315,12 +290,12 @@ __global__ __launch_bounds__(64 * W, 2) void pattn_split(const ktir_pattn_t d, i
   };
   const f32x16_t z16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   f32x16_t o[DT];                              // O^T tiles: column 32 dt + 8 g + 4 h + t of row r32
-  float m, mr, lsum;
-  const int k_off = r32 * D, k_x = ps_swz<D>(r32 & 15);
+  float m, b, lsum;                            // b: the base 2^b of P, l and O (at most 2^P_LAG below e^m)
+  const int k_off = r32 * D, k_x = kv_swz<D>(r32 & 15);
   const int tg = l >> 4, tj = l & 15;
   const int v_row0 = 4 * (tg >> 1) + (tj >> 2);
   const int v_c = 2 * (tg & 1) + ((tj >> 1) & 1), v_in = 4 * (tj & 1);
-  const int v_b0 = v_row0 * D + v_in, v_x0 = v_c ^ ps_swz<D>(v_row0), v_x1 = v_c ^ ps_swz<D>(v_row0 + 8);
+  const int v_b0 = v_row0 * D + v_in, v_x0 = v_c ^ kv_swz<D>(v_row0), v_x1 = v_c ^ kv_swz<D>(v_row0 + 8);
   const int mine = first_pair < n_pairs ? (n_pairs - first_pair + stride - 1) / stride : 0;
   constexpr int LOADS = 32 * D / 512;          // a pair's K (or V) loads
   // One pair.  FAST: its K and V are in flight, K first; those of pair `next`
@@ -370,21 +345,25 @@ __global__ __launch_bounds__(64 * W, 2) void pattn_split(const ktir_pattn_t d, i
     bool poison = false;
     if (j0 == 0) poison = pair_max(x0) == -__builtin_inff();
     const float mn = fmax_nan(m, pair_max(fmax_nan(x0, x1)));
-    const bool up = mn > __fadd_rn(mr, 8.0f);
+    const float bn = __fmul_rn(mn, LOG2E);
+    const bool up = bn > __fadd_rn(b, P_LAG<BF16>);
     if (__any(up)) {
-      const float al = up ? exp_f(__fsub_rn(mr, mn)) : 1.f;
+      const float al = up ? exp2_f(__fsub_rn(b, bn)) : 1.f;
 #pragma unroll
       for (int t = 0; t < DT; ++t)
 #pragma unroll
         for (int i = 0; i < 16; ++i) o[t][i] = __fmul_rn(o[t][i], al);
       lsum = __fmul_rn(lsum, al);
-      mr = up ? mn : mr;
+      b = up ? bn : b;
     }
     m = mn;
     // all keys so far masked: P = 0 against any base
-    const float c0 = -__fmul_rn(mn == -__builtin_inff() ? 0.f : (mn != mn ? mn : mr), LOG2E);
+    const float pb = mn == -__builtin_inff() ? 0.f : (mn != mn ? mn : b);
 #pragma unroll
-    for (int i = 0; i < 16; ++i) x[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(x[i], LOG2E, c0));
+    for (int i = 0; i < 16; ++i) x[i] = exp2_f(__builtin_fmaf(x[i], LOG2E, -pb));
+    // whether a P is too small for two f16 terms
+    bool small = false;
+    if constexpr (!BF16 && PARTS == 2 && !INF_V) small = __any(least_positive<16>(x) < P_SMALL);
     float a0 = 0.f, a1 = 0.f, a2 = 0.f, a3 = 0.f;
 #pragma unroll
     for (int i = 0; i < 16; i += 4) {
@@ -396,38 +375,57 @@ __global__ __launch_bounds__(64 * W, 2) void pattn_split(const ktir_pattn_t d, i
     lsum = __fadd_rn(lsum, pair_sum(__fadd_rn(__fadd_rn(a0, a1), __fadd_rn(a2, a3))));
     // V of this pair has landed: only the next pair's K is in flight
     if constexpr (FAST) ps_wait<LOADS>();
+    // P V: by the terms of the operand type, by the rest they leave (two f16
+    // terms) or by bf16 terms of the whole P (the same with infinities in V)
+    enum { TERMS, REST, WHOLE };
+    auto pv = [&](auto how) __attribute__((always_inline)) {
+      constexpr int HOW = decltype(how)::value;
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      const uint16_t* vt = &V[16 * ks * D];
-      uint32_t t0[PARTS][2], t1[PARTS][2];
-      ps_split<BF16, PARTS>(x + 8 * ks, t0);
-      ps_split<BF16, PARTS>(x + 8 * ks + 4, t1);
-      if constexpr (INF_V && !BF16) {
-        // a positive P below f16's range still times an infinite V is infinite
-        lift4(x + 8 * ks, t0[0]);
-        lift4(x + 8 * ks + 4, t1[0]);
+      for (int ks = 0; ks < 2; ++ks) {
+        const uint16_t* vt = &V[16 * ks * D];
+        float p[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          p[i] = x[8 * ks + i];
+          if constexpr (HOW == REST) asm volatile("" : "+v"(p[i]));   // nothing kept for it from the terms
+          if constexpr (HOW == WHOLE) p[i] = __fmul_rn(p[i], P_SCALE<BF16>);
+        }
+        uint32_t t0[PARTS][2], t1[PARTS][2];
+        uint4 tb[3];
+        if constexpr (HOW != WHOLE) {
+          p_split<BF16, PARTS, HOW == REST>(p, t0);
+          p_split<BF16, PARTS, HOW == REST>(p + 4, t1);
+        }
+        if constexpr (HOW != TERMS) p_split_bf(p, tb);
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) {
+          const uint2 lo = ds_tr16(vt + v_b0 + 8 * ((4 * dt) ^ v_x0));
+          const uint2 hi = ds_tr16(vt + v_b0 + 8 * D + 8 * ((4 * dt) ^ v_x1));
+          const uint4 a = make_uint4(lo.x, lo.y, hi.x, hi.y);
+          if constexpr (HOW == TERMS) {
+            o[dt] = pv_mfma<BF16, PARTS, INF_V>(a, t0, t1, o[dt]);
+          } else {
+            o[dt] = pv_mfma_bf<INF_V>(a, tb, o[dt]);
+            __builtin_amdgcn_sched_barrier(0);     // rare: must not set the register count
+          }
+        }
       }
+      if constexpr (FAST && HOW == TERMS) {
+        // the V reads of the second 16 keys between the MFMAs of the first
+        __builtin_amdgcn_sched_group_barrier(0x100, 2 * DT, 0);
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt) {
-        const uint2 lo = ds_tr16(vt + v_b0 + 8 * ((4 * dt) ^ v_x0));
-        const uint2 hi = ds_tr16(vt + v_b0 + 8 * D + 8 * ((4 * dt) ^ v_x1));
-        const uint4 a = make_uint4(lo.x, lo.y, hi.x, hi.y);
-        uint4 af = a;
-        if constexpr (INF_V) af = make_uint4(finite2<BF16>(a.x), finite2<BF16>(a.y), finite2<BF16>(a.z), finite2<BF16>(a.w));
-#pragma unroll
-        for (int q = PARTS - 1; q >= 0; --q)
-          o[dt] = mfma_at<BF16>(q ? af : a, make_uint4(t0[q][0], t0[q][1], t1[q][0], t1[q][1]), o[dt]);
+        for (int q = 0; q < DT; ++q) {
+          __builtin_amdgcn_sched_group_barrier(0x008, PARTS, 0);
+          __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+        }
+        __builtin_amdgcn_sched_group_barrier(0x008, DT * PARTS, 0);
       }
-    }
-    if constexpr (FAST) {
-      // the V reads of the second 16 keys between the MFMAs of the first
-      __builtin_amdgcn_sched_group_barrier(0x100, 2 * DT, 0);
-#pragma unroll
-      for (int q = 0; q < DT; ++q) {
-        __builtin_amdgcn_sched_group_barrier(0x008, PARTS, 0);
-        __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-      }
-      __builtin_amdgcn_sched_group_barrier(0x008, DT * PARTS, 0);
+    };
+    if constexpr (!BF16 && PARTS == 2 && INF_V) {
+      pv(std::integral_constant<int, WHOLE>{});
+    } else {
+      pv(std::integral_constant<int, TERMS>{});
+      if (small) pv(std::integral_constant<int, REST>{});
     }
     if (j0 == 0 && __any(poison)) {
       const float nan = __builtin_nanf("");
@@ -446,7 +444,7 @@ __global__ __launch_bounds__(64 * W, 2) void pattn_split(const ktir_pattn_t d, i
     constexpr bool INF_V = decltype(inf_v)::value;
 #pragma unroll
     for (int t = 0; t < DT; ++t) o[t] = z16;
-    m = mr = -__builtin_inff();
+    m = b = -__builtin_inff();
     lsum = 0.f;
     for (int c0 = 0; c0 < mine; c0 += 32) {
       if (INF_V || c0) table = entries(c0);
@@ -487,14 +485,14 @@ __global__ __launch_bounds__(64 * W, 2) void pattn_split(const ktir_pattn_t d, i
     if (__any(nan)) pages(std::true_type{});
   }
   if (bad) *err = 1;
-  // bring l and O from mr to m
-  if (mine > 0 && mr != m && m != -__builtin_inff()) {
-    const float fin = exp_f(__fsub_rn(mr, m));
+  // bring l and O from 2^b to e^m, and O from P's scale
+  if (mine > 0 && m != -__builtin_inff()) {
+    const float fin = exp2_f(__builtin_fmaf(-m, LOG2E, b)), f = __fmul_rn(fin, 1.f / P_SCALE<BF16>);
     lsum = __fmul_rn(lsum, fin);
 #pragma unroll
     for (int t = 0; t < DT; ++t)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) o[t][i] = __fmul_rn(o[t][i], fin);
+      for (int i = 0; i < 16; ++i) o[t][i] = __fmul_rn(o[t][i], f);
   }
   // the wavefront's state into its LDS: 4-column groups of a row, rows side by side
   __builtin_amdgcn_s_waitcnt(0);

@@ -7,6 +7,7 @@ import pytest
 from ktir_cpu_amd import configs
 from ktir_cpu_amd import runtime as rt
 from oracle.interp import bf16_bits, bf16_from_bits
+from tests.test_oracle_example_pins import PA_FN
 
 pytestmark = pytest.mark.gpu
 
@@ -156,3 +157,86 @@ def test_tiles_row_sum_of_far_scores(M, N, D):
     s = (_f64(q)[0, 0] @ _f64(k)[0, 0].T)[0]
     np.testing.assert_array_equal(_device(d.m_out, S), np.full(S, s.max()))
     np.testing.assert_allclose(_device(d.l_out, S), np.full(S, np.exp(s - s.max()).sum()), rtol=4e-6)
+
+
+# ---- paged ---------------------------------------------------------------------
+
+def _paged(dt, tokens, block_q, head, q, k, v, context, scale):
+    """One KV head: q [tokens, 4, head], k and v [keys, head] in order of position."""
+    n = k.shape[0] // 16
+    gen = dict(tokens=tokens, block_q=block_q, head=head, q_heads=4, kv_heads=1, blocks=n, max_pages=n)
+    order = np.random.default_rng(2).permutation(n)
+    pages = lambda x: _bits(x, dt).reshape(n, 16, 1, head)[np.argsort(order)]
+    kw = dict(output_ptr=_bits(np.zeros(q.shape), dt), query_ptr=_bits(q, dt), key_cache_ptr=pages(k),
+              value_cache_ptr=pages(v), block_tables_ptr=order.astype(np.int32)[None], cur_batch_start_index=0,
+              block_table_offset=0, num_tiles=n, context_len=context, scale=scale)
+    prep, d = _prepare(configs.paged_attention(dt=dt, **gen), PA_FN, kw)
+    assert d.n_items > 0
+    return prep, d
+
+
+def _paged_want(q, k, v, context, scale, dt):
+    q, k, v = (_f64(_bits(x, dt)) for x in (q, k, v))
+    s = np.einsum("thd,jd->thj", q, k) * scale
+    late = np.arange(k.shape[0])[None, None] > context + np.arange(q.shape[0])[:, None, None]
+    s = np.where(late, -np.inf, s)
+    m = s.max(-1, keepdims=True)
+    p = np.exp(s - m)
+    l = p.sum(-1, keepdims=True)
+    return p @ v / l, p @ np.abs(v) / l, m[..., 0], l[..., 0]
+
+
+# half a unit of what P is rounded to: a lane of at most 16 rows carries one
+# f16 term or two bf16 ones
+P_ERR = {(8, "f16"): 2.0 ** -12, (8, "bf16"): 2.0 ** -17, (32, "f16"): 0.0, (32, "bf16"): 0.0}
+ROWS = {8: dict(tokens=8, block_q=2), 32: dict(tokens=16, block_q=8)}
+
+
+@pytest.mark.parametrize("splits", [1, 3])
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("head", [64, 128])
+@pytest.mark.parametrize("rows", list(ROWS))
+def test_paged_within_its_roundings(rows, head, dt, splits, monkeypatch):
+    from ktir_cpu_amd import fusion
+    monkeypatch.setattr(fusion, "_pattn_splits", lambda *a: splits)
+    rng = np.random.default_rng(rows + head)
+    t, S = ROWS[rows]["tokens"], 336
+    q, k, v = (rng.standard_normal(x) for x in ((t, 4, head), (S, head), (S, head)))
+    args = (q, k, v, S - t, head ** -0.5)
+    prep, d = _paged(dt, t, ROWS[rows]["block_q"], head, *args)
+    want, spread, _, _ = _paged_want(*args, dt)
+    _near(_f64(prep.outputs()["output_ptr"]), want, dt, spread, P_ERR[rows, dt] + 2.0 ** -21)
+
+
+@pytest.mark.parametrize("splits", [1, 3])
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("gap", [9.0, 14.0, 16.5, 24.0])
+@pytest.mark.parametrize("at", [3, 300])
+@pytest.mark.parametrize("rows", list(ROWS))
+def test_paged_heavy_key_without_value(rows, at, gap, dt, splits, monkeypatch):
+    from ktir_cpu_amd import fusion
+    monkeypatch.setattr(fusion, "_pattn_splits", lambda *a: splits)
+    t, S, head = ROWS[rows]["tokens"], 512, 128
+    if rows == 8 and dt == "f16":
+        gap = min(gap, 17.0)                     # below, one f16 term is subnormal
+    q, k, v = _sink(S, head, at, gap, 250.0)
+    args = (np.broadcast_to(q[0], (t, 4, head)), k, v, S - t, 1.0)
+    prep, d = _paged(dt, t, ROWS[rows]["block_q"], head, *args)
+    want, spread, _, _ = _paged_want(*args, dt)
+    _near(_f64(prep.outputs()["output_ptr"]), want, dt, spread, P_ERR[rows, dt] + _exp_err(gap))
+
+
+@pytest.mark.parametrize("splits", [1, 3])
+@pytest.mark.parametrize("rows", list(ROWS))
+def test_paged_row_sum_of_far_scores(rows, splits, monkeypatch):
+    """As for the dense tiles, across wavefronts and workgroups whose keys
+    have other maxima."""
+    from ktir_cpu_amd import fusion
+    monkeypatch.setattr(fusion, "_pattn_splits", lambda *a: splits)
+    t, S, head = ROWS[rows]["tokens"], 512, 128
+    q, k = _far_scores(S, head, 32)
+    args = (np.broadcast_to(q[0], (t, 4, head)), k, np.random.default_rng(1).standard_normal((S, head)), S - t, 1.0)
+    prep, d = _paged("f16", t, ROWS[rows]["block_q"], head, *args)
+    _, _, m, l = _paged_want(*args, "f16")
+    np.testing.assert_array_equal(_device(d.m_out, 4 * t), m.reshape(-1))
+    np.testing.assert_allclose(_device(d.l_out, 4 * t), l.reshape(-1), rtol=4e-6)
