@@ -27,6 +27,10 @@ static int g_device = -1;
 // The pinned ring.  A part is handed out again only after the stream has
 // drained, under the mutex that also covers what is queued from it.
 constexpr uint64_t RING = 1 << 20, SMALL_COPY = 64 << 10, SMALL_LIST = 256 << 10;
+// Coherent, whatever the runtime's default: the host writes a part again that an
+// earlier kernel has read, and the next kernel must not find the old bytes in
+// the device's cache; the same goes for the error word.
+constexpr unsigned PINNED = hipHostMallocPortable | hipHostMallocCoherent;
 static std::mutex g_ring_mutex;
 static uint8_t* g_ring = nullptr;
 static uint64_t g_ring_head = 0;
@@ -76,7 +80,7 @@ extern "C" int ktir_init(int device) {
   KTIR_HIP_CHECK(hipSetDevice(device));
   KTIR_HIP_CHECK(hipStreamCreateWithFlags(&g_stream, hipStreamNonBlocking));
   if (!g_err_flag) {
-    KTIR_HIP_CHECK(hipHostMalloc((void**)&g_err_flag, sizeof(int), hipHostMallocPortable));
+    KTIR_HIP_CHECK(hipHostMalloc((void**)&g_err_flag, sizeof(int), PINNED));
     *g_err_flag = 0;
   }
   g_device = device;
@@ -129,7 +133,7 @@ extern "C" int ktir_free(uint64_t dptr) {
 // `bytes` of the ring, 256-byte aligned (the mutex held); null: no ring
 static uint8_t* ring_take(uint64_t bytes) {
   if (!g_ring) {
-    if (hipHostMalloc((void**)&g_ring, RING, hipHostMallocPortable) != hipSuccess) {
+    if (hipHostMalloc((void**)&g_ring, RING, PINNED) != hipSuccess) {
       (void)hipGetLastError();
       g_ring = nullptr;
       return nullptr;

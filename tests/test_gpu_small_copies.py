@@ -73,3 +73,18 @@ def test_ring_used_many_times_over(threads):
     for t in ts:
         t.join()
     assert not errors, errors[0]
+
+
+def test_ring_without_coherent_default():
+    """The same where the runtime's own default for pinned memory is not
+    coherent: the same parts of the ring, read by kernel after kernel, hold other
+    bytes each time."""
+    import os
+    import subprocess
+    import sys
+    code = ("from tests import test_gpu_small_copies as t\ne = []\nfor s in range(4): t._many(s, e)\n"
+            "assert not e, e[0]\nprint('whole')")
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    r = subprocess.run([sys.executable, "-c", code], cwd=root, env=dict(os.environ, HIP_HOST_COHERENT="0"),
+                       capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0 and "whole" in r.stdout, r.stdout + r.stderr
