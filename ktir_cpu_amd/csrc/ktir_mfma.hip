@@ -547,10 +547,22 @@ using namespace ktir;
 // 16-byte aligned rows, M and N multiples of 128, K a multiple of 64.  The
 // caller (the lockstep executor) has already checked that every lane's
 // operand range lies inside its allocation.
-// the fewest 256 x 256 blocks (one workgroup per CU) that beat smaller blocks
-// over the plane (ktir_mmplane.hip): 192 blocks (4096 x 3072 x 1024) 35 against
-// 39 us, 128 blocks (2048 x 4096 x 4096) 96 against 77 us
+// The fewest 256 x 256 blocks (one workgroup per CU) that beat smaller ones:
+// 192 blocks (3072 x 4096 x 1024) 35 us against 47 and 43, 128 blocks
+// (4096 x 2048 x 4096) 97 us against 77 and 83.
 constexpr int64_t Q_MIN = 160;
+
+// Where blocks of the plane (ktir_mmplane.hip: 128 x 128, smaller ones for few
+// lanes) beat the lanes' own tiles (mm_mfma_dma, `blocks` of 128 x 128): where
+// these leave CUs idle, up to one per CU over a longer K.  f16, us, own tiles / plane:
+//   64 blocks (1024^2): K = 64 5.6 / 4.9, 4096 50 / 20
+//   128 blocks (1024 x 2048): K = 64 5.8 / 6.3, 256 7.3 / 7.4, 1024 17 / 11, 4096 51 / 28
+//   256 blocks (2048^2): K = 256 8.1 / 10.5, 1024 18.3 / 17.4, 4096 54 / 45
+//   384 blocks (2048 x 3072): K = 64 7.6 / 9.5, 1024 21 / 24, 4096 62 / 67
+//   1024 blocks (4096^2): K = 512 28 / 34, 4096 141 / 149
+static bool plane_wins(int64_t blocks, int64_t k) {
+  return blocks <= 64 || (blocks <= 256 && k > (blocks <= 128 ? 192 : 512));
+}
 
 static int64_t kt_steps(const ktir_mm_t* d) { return d->K / BK; }
 
@@ -599,8 +611,9 @@ int ktir_launch_matmul_mfma(const ktir_mm_t* d, bool* handled) {
                     (d->c.dtype == KTIR_F32 || d->c.dtype == KTIR_F16 || d->c.dtype == KTIR_BF16) &&
                     d->round_dt == KTIR_F32 && d->accumulate != 1 && d->c.strides[1] == 1 &&
                     (127 * d->a.strides[0] + (d->ksteps - 1) * d->a_kstep + d->K) * 2 < (int64_t)0x7fffffff;
-  if ((!q256 || d->n_quads < Q_MIN) && launch_mm_plane(d)) {
-  } else if (q256) {
+  const bool large = q256 && d->n_quads >= Q_MIN;
+  if (!large && (!dma || plane_wins(blocks, d->ksteps * d->K)) && launch_mm_plane(d)) {
+  } else if (large) {
     if (f16)
       hipLaunchKernelGGL((mm_mfma_256<false>), dim3((unsigned)d->n_quads), dim3(256), 0, stream(), *d);
     else

@@ -12,11 +12,13 @@
 // tiles.  K advances 64 at a time through NS (two or four) LDS stages filled by
 // buffer_load ... lds (no registers) with one barrier a step; a step's
 // 256 to 512 MFMA cycles are far less than a load's latency, so where one
-// workgroup has a CU to itself three stages stay in flight (512 x 4096 x 4096,
-// f16: 49 us with two stages, 29 with four).  Then the LDS reads bound it: a
-// 64 x 64 quarter reads 16 KB for 16 MFMAs.
-// 512 x 4096 x 4096 in 64 x 64 tiles: 1009 us (mm_generic, f32 FMA) -> 26 us
-// (660 TFLOP/s); 2048^3 in 128 x 128 tiles: 47 us (mm_mfma_256) -> 26 us.
+// workgroup has a CU to itself three stages stay in flight (launches of
+// 512 x 4096 x 4096, f16, one after another: 49 us with two stages, 29 with four).
+// Then the LDS reads bound it: a 64 x 64 quarter reads 16 KB for 16 MFMAs.
+// 512 x 4096 x 4096 in 64 x 64 tiles, as a pass between others: 1009 us
+// (mm_generic, f32 FMA) -> 26 us (660 TFLOP/s); 2048^3 in 128 x 128 tiles: 30 us
+// (mm_mfma_dma) -> 26 us.  Where those tiles fill the chip they stay the better
+// blocks (plane_wins in ktir_mfma.hip).
 // Layouts: A as 128-byte rows (16-byte chunk c of row
 // r at slot c ^ swz_a(r), read by ds_read_b128), B row-major as in HBM (chunk c
 // at c ^ mp_swz(r), read by ds_read_b64_tr_b16); both layouts are free of bank

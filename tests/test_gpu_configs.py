@@ -407,6 +407,23 @@ def test_gemm_plane_blocks(shape, dt):
                                rtol=2.0 ** (-10 if dt == "f16" else -7), atol=shape[2] * 2.0 ** -24)
 
 
+# tiles of 128 as blocks of the plane (144 blocks over a long K; 64 and 120
+# blocks) and each in its own block (272 and, in groups of four, 288 blocks; a
+# short K)
+_TILE128_SHAPES = [(1536, 1536, 640, 128, 128, 64, 4, 4), (1024, 1024, 192, 128, 128, 64, 1, 1), (1280, 1536, 256, 128, 128, 64, 2, 2),
+                   (2176, 2048, 64, 128, 128, 64, 1, 1), (2304, 2048, 128, 128, 128, 64, 2, 2), (1536, 1536, 128, 128, 128, 64, 4, 4)]
+
+
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("shape", _TILE128_SHAPES)
+def test_gemm_128_tiles_either_blocks(shape, dt):
+    """As the plane's blocks: K 2^-24 of the sum of magnitudes, one rounding."""
+    ref, out, g = _run(_cases.gemm(*shape) if dt == "f16" else _cases.gemm_bf16(*shape))
+    assert set(g.last_plan.counts()) == {"mm"}
+    np.testing.assert_allclose(_half_f32(out["c_ptr"], dt), _half_f32(ref["c_ptr"], dt),
+                               rtol=2.0 ** (-10 if dt == "f16" else -7), atol=shape[2] * 2.0 ** -24)
+
+
 def test_gemm_plane_f32_result_and_separate_lanes():
     """f32 results of 64 x 64 tiles; then the same launch without its plane
     (lanes that share nothing): one plane per lane."""
