@@ -471,7 +471,7 @@ typedef struct ktir_pattn {
    * rows together.  With pages of 16 keys, one 16-bit operand type and 64 or
    * 128 columns, `splits` workgroups of `waves` (4 or 8) wavefronts share an
    * item's keys; for splits > 1 ws holds n_items * splits * (64 + 32 * D)
-   * floats.  Other launches ignore the items. */
+   * floats.  Other launches (`waves` 1 among them) ignore the items. */
   uint64_t items, item_lanes, ws;
   int64_t n_items;
   int32_t splits, waves;

@@ -19,6 +19,7 @@
 // (q . k), m' = max(m, max_c s), p = exp(s - m'), alpha = exp(m - m'),
 // acc' = acc * alpha + p . v, l' = l * alpha + sum_c p.
 #include <climits>
+#include <type_traits>
 #include "ktir_common.h"
 
 namespace ktir {
@@ -589,13 +590,18 @@ __device__ __forceinline__ int64_t pa_readlane(int64_t v, int src) {
 // e^x as 2^(x log2 e) on the hardware exp2 (v_exp_f32)
 __device__ __forceinline__ float pa_exp(float x) { return __builtin_amdgcn_exp2f(__fmul_rn(x, 1.44269504088896341f)); }
 
+// a packed pair of bf16 values with 0 in the place of infinities and NaN
+__device__ __forceinline__ uint32_t pa_finite(uint32_t w) {
+  return ((w & 0x7f80u) == 0x7f80u ? 0u : w & 0xffffu) | ((w & 0x7f800000u) == 0x7f800000u ? 0u : w & 0xffff0000u);
+}
+
 // Pages move in groups of G: the next group's loads are issued, the current
 // group's G pages are computed (one online-softmax step each, in order),
 // then one wait for the next group.  A page that is not wholly inside its
 // window or not 16-byte aligned ends the grouped loop; the lane's
 // remaining pages then run one at a time with element loads.
 template <bool BF16, int DT, int G>
-__global__ __launch_bounds__(64) void pattn_mfma(const ktir_pattn_t d, int vec, int* err) {
+__global__ __launch_bounds__(64, DT == 1 ? 6 : (DT == 2 ? 4 : (DT == 4 ? 3 : 1))) void pattn_mfma(const ktir_pattn_t d, int vec, int* err) {
   constexpr int D = 32 * DT, NT = 2 * DT;   // NT tiles of 16 columns
   const int l = threadIdx.x, n = l & 15, g = l >> 4;
   const int M = (int)d.M;
@@ -663,12 +669,19 @@ __global__ __launch_bounds__(64) void pattn_mfma(const ktir_pattn_t d, int vec, 
   // relative to mr <= m, moved up to m only when m passes mr by more than 8
   // (so P <= e^8) and once after the loop: the same quantities as the
   // loop body's per-page rescale by alpha = exp(m - m'), up to rounding.
-  float m = d.m0, mr = d.m0, lsum = d.l0;
+  float m, mr, lsum;
   pa_f4 o[NT];
+  auto start = [&]() {
+    m = mr = d.m0;
+    lsum = d.l0;
 #pragma unroll
-  for (int t = 0; t < NT; ++t) o[t] = pa_f4{0.f, 0.f, 0.f, 0.f};
+    for (int t = 0; t < NT; ++t) o[t] = pa_f4{0.f, 0.f, 0.f, 0.f};
+  };
+  start();
 
-  auto step = [&](int j, const PaOps<DT>& cur) {
+  // INF_V: the second term of P (0, or of the other sign) meets no infinity of V
+  auto step = [&](auto inf_v, int j, const PaOps<DT>& cur) {
+    constexpr bool INF_V = decltype(inf_v)::value;
     pa_f4 st = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int t = 0; t < DT; ++t)
@@ -727,7 +740,8 @@ __global__ __launch_bounds__(64) void pattn_mfma(const ktir_pattn_t d, int vec, 
       const uint32_t a1 = __builtin_amdgcn_perm(pa_vword<DT>(cur, 3, w), pa_vword<DT>(cur, 2, w), sel);
       const uint2 va = make_uint2(a0, a1);
       o[t] = mfma_k16<BF16>(va, ph, o[t]);
-      if constexpr (BF16) o[t] = mfma_k16<BF16>(va, pl, o[t]);
+      if constexpr (BF16) o[t] = mfma_k16<BF16>(INF_V ? make_uint2(pa_finite(a0), pa_finite(a1)) : va, pl, o[t]);
+      if constexpr (INF_V) __builtin_amdgcn_sched_barrier(0);   // rare: must not set the register count
     }
   };
 
@@ -769,14 +783,14 @@ __global__ __launch_bounds__(64) void pattn_mfma(const ktir_pattn_t d, int vec, 
       okB = issue(j + G, B);
 #pragma unroll
       for (int u = 0; u < G; ++u)
-        if (j + u < trips) step(j + u, A[u]);
+        if (j + u < trips) step(std::false_type{}, j + u, A[u]);
       j += G;
       __builtin_amdgcn_s_waitcnt(0);
       if (j >= trips || !okB) break;
       okA = issue(j + G, A);
 #pragma unroll
       for (int u = 0; u < G; ++u)
-        if (j + u < trips) step(j + u, B[u]);
+        if (j + u < trips) step(std::false_type{}, j + u, B[u]);
       j += G;
       __builtin_amdgcn_s_waitcnt(0);
       if (j >= trips) break;
@@ -785,13 +799,30 @@ __global__ __launch_bounds__(64) void pattn_mfma(const ktir_pattn_t d, int vec, 
   // page by page from page j (the whole loop when the pages are not
   // aligned, else from the first page that leaves its window), element
   // loads where a piece leaves the window
-  for (; j < trips; ++j) {
-    const int64_t page = uni(pa_fix(pa_entry_raw(d, tp, j, trips), bad));
-    const int64_t k0 = kb + page * d.k_page, v0 = vb + page * d.v_page;
-    PaOps<DT> one;
-    if (vec && pa_fast<DT>(d, k0, v0)) pa_load_fast<DT>(d, k0, v0, lo, one);
-    else pa_load_any<DT>(d, k0, v0, lo, one);
-    step(j, one);
+  auto rest = [&](auto inf_v) {
+    for (; j < trips; ++j) {
+      const int64_t page = uni(pa_fix(pa_entry_raw(d, tp, j, trips), bad));
+      const int64_t k0 = kb + page * d.k_page, v0 = vb + page * d.v_page;
+      PaOps<DT> one;
+      if (vec && pa_fast<DT>(d, k0, v0)) pa_load_fast<DT>(d, k0, v0, lo, one);
+      else pa_load_any<DT>(d, k0, v0, lo, one);
+      step(inf_v, j, one);
+    }
+  };
+  rest(std::false_type{});
+  // two terms of P: a NaN anywhere in the result may be an infinity of P V, so
+  // the pages run again
+  if constexpr (BF16) {
+    bool nan = false;
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) nan |= o[t][i] != o[t][i];
+    if (__builtin_amdgcn_ballot_w64(nan)) {
+      start();
+      j = 0;
+      rest(std::true_type{});
+    }
   }
   if (bad) *err = 1;
   // bring P, l and O from mr to m (m > mr only where the loop ran and m

@@ -1041,7 +1041,7 @@ def _paged_attention(ex, trips, tm1, q, probes, peeled, l0, slots, mask, names):
         lanes, items = _pattn_items(trips, k[1], v[1], k[5], ck0.astype(np.int64), M)
         d.item_lanes, d.items, d.n_items = up(lanes), up(items), len(items)
         d.splits = _pattn_splits(len(items), int(trips.max()))
-        d.waves = _pattn_waves(len(items), d.splits, int(trips.max()))
+        d.waves = _pattn_waves(len(items), d.splits, int(trips.max()), L if M <= 16 else 0, D)
         if d.splits > 1:
             ws = ex.pool.temp(len(items) * d.splits * (64 + 32 * D) * 4)
             keep.append(ws)
@@ -1097,11 +1097,33 @@ def _pattn_splits(n_items, trips, cus=256):
     return s if trips / 16 - trips / (8 * s) >= 2.5 else 1
 
 
-def _pattn_waves(n_items, splits, trips, cus=256):
+def _pattn_one_us(lanes, n_items, trips, head):
+    """Time of the launch with one wavefront per lane, in us: the first page,
+    the lanes' start, then page after page, in step or bound by what all lanes
+    read.  Measured within 20 % for 32 to 16384 lanes of 128 columns, 1 to 80 pages
+    (1024 lanes, 10 pages each of its own: 17.0, of 256 sequences: 13)."""
+    l, i, w = lanes / 1000, n_items / 1000, head / 128
+    return 6.3 + 1.2 * l + trips * max(0.5 + (0.15 * l + 0.4 * i) * w, (0.55 * l + 0.4 * i) * w)
+
+
+def _pattn_four_us(lanes, n_items, trips, head):
+    """The same with a workgroup of four wavefronts per item: the wavefronts'
+    states are merged once per workgroup, and two workgroups share a CU (1024
+    items, 10 pages each of its own: 29.8; 256 items of four lanes: 10)."""
+    i, w = n_items / 1000, head / 128
+    return max(8.5 + 1.2 * n_items / lanes, 2 + 17.1 * i * w) + trips * max(0.2, 0.9 * i * w)
+
+
+def _pattn_waves(n_items, splits, trips, lanes=0, head=128, cus=256):
     """Wavefronts of a workgroup: eight where the only workgroup of a CU has
     enough pages for them (256 tokens after 1024: 25.2 us, with four 27.2; after
     8191: 72 us, with four 97), four where it has few (one token after 500: 13.4
-    us, with eight 13.8), shares an item with others or shares its CU."""
+    us, with eight 13.8), shares an item with others or shares its CU.  One, a
+    lane each, for few pages and for many sequences (`lanes`: those of at most 16
+    rows, which that kernel takes): 2048 lanes of 5 pages of their own 19 us,
+    with four 42."""
+    if lanes and splits == 1 and _pattn_one_us(lanes, n_items, trips, head) < _pattn_four_us(lanes, n_items, trips, head):
+        return 1
     return 8 if splits == 1 and n_items <= cus and trips >= 48 else 4
 
 

@@ -1,6 +1,6 @@
 """Paged attention on values that its matrix-core kernels could lose: NaN and
 infinities in Q, K and V, for lanes whose P is one or several terms of the
-operand type."""
+operand type; and lanes that are sequences of their own, which share no pages."""
 import numpy as np
 import pytest
 
@@ -37,15 +37,16 @@ def _run(src, kw, oracle=True):
     return got["output_ptr"], None if ref is None else ref["output_ptr"]
 
 
-@pytest.mark.parametrize("splits", [1, 2])
+@pytest.mark.parametrize("splits,waves", [(1, 4), (2, 4), (1, 8), (1, 1)])
 @pytest.mark.parametrize("dt", ["f16", "bf16"])
 @pytest.mark.parametrize("head", [64, 128])
 @pytest.mark.parametrize("rows", list(ROWS))
-def test_non_finite_inputs(rows, head, dt, splits, monkeypatch):
+def test_non_finite_inputs(rows, head, dt, splits, waves, monkeypatch):
     """NaN in a query row, an infinity in a key, infinities of both signs and
     a NaN in V: NaN and infinities exactly where the oracle has them."""
     from ktir_cpu_amd import fusion
     monkeypatch.setattr(fusion, "_pattn_splits", lambda *a: splits)
+    monkeypatch.setattr(fusion, "_pattn_waves", lambda *a: waves)
     gen = dict(ROWS[rows], head=head)
     kw = paged_inputs(tokens=gen["tokens"], head=head, seed=11)
     pages = kw["block_tables_ptr"][0]
@@ -64,3 +65,37 @@ def test_non_finite_inputs(rows, head, dt, splits, monkeypatch):
     assert np.isnan(ref).any() and np.isposinf(ref).any() and np.isneginf(ref).any()
     ok = ~np.isnan(ref)
     np.testing.assert_allclose(got[ok], ref[ok], rtol=1e-2, atol=1e-3)
+
+
+def _sequences(n, pages, dt, head=64):
+    """n tokens of 4 query heads, each a sequence with its own `pages` pages."""
+    rng = np.random.default_rng(n + pages)
+    gen = dict(tokens=n, block_q=1, q_heads=8, kv_heads=2, head=head, blocks=96, max_pages=n * pages)
+    src = configs.paged_attention(dt=dt, **gen)
+    old = "%bt_col = arith.addi %block_table_offset, %j : index"
+    assert old in src
+    src = src.replace(old, "%bt_col = arith.addi %own, %j : index")
+    one = "    %c1 = arith.constant 1 : index\n"
+    src = src.replace(one, one + f"    %per = arith.constant {pages} : index\n    %own = arith.muli %p0, %per : index\n", 1)
+    kw = paged_inputs(tokens=n, q_heads=8, kv_heads=2, head=head, blocks=96, max_pages=n * pages, seed=n)
+    kw = {k: (v if k == "block_tables_ptr" else _bits(v, dt)) for k, v in kw.items()}
+    return src, dict(kw, **dict(PA_ARGS, num_tiles=pages, context_len=16 * pages - n // 2))
+
+
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("n,pages,waves", [(40, 3, 1), (40, 24, 4)])
+def test_sequences_of_their_own(n, pages, waves, dt):
+    """Few pages each: one wavefront per lane; more: four per item of one lane."""
+    from ktir_cpu_amd.interpreter import KTIRInterpreter
+    src, kw = _sequences(n, pages, dt)
+    o = OracleInterpreter()
+    o.load(src)
+    ref = o.execute_function(PA_FN, **{k: (v.copy() if isinstance(v, np.ndarray) else v) for k, v in kw.items()})
+    g = KTIRInterpreter()
+    g.load(src)
+    got = g.execute_function(PA_FN, **kw)
+    d = g.last_plan.launches[-1][1]
+    assert (d.lanes, d.n_items, d.splits, d.waves) == (2 * n, 2 * n, 1, waves)
+    # P in one f16 term or two bf16 terms, one rounding of the result
+    np.testing.assert_allclose(_f32(got["output_ptr"], dt), _f32(ref["output_ptr"], dt),
+                               rtol=2.0 ** (-7 if dt == "bf16" else -10), atol=2.0 ** -10 if dt == "f16" else 2.0 ** -14)

@@ -301,3 +301,16 @@ def test_collapse_dims_keeps_every_element_offset():
     d3 = LeafSpec(0, "f32", LaneOff(0, 720), _cstrides((2, 3, 4, 5, 6)), 0, 1 << 20)
     e4, _ = _collapse_dims(e3, d3, 4)
     assert e4.shape == (2, 3, 20, 6)          # merges only until the rank fits
+
+
+def test_paged_wavefronts_per_item():
+    """One wavefront per lane where lanes have few pages or share none and are
+    many; workgroups where a lane alone would take too long."""
+    from ktir_cpu_amd.fusion import _pattn_waves
+    assert _pattn_waves(2048, 1, 10, 2048, 128) == 1          # 2048 sequences
+    assert _pattn_waves(32, 1, 2, 32, 128) == 1               # two pages
+    assert _pattn_waves(64, 1, 40, 64, 128) == 4              # few sequences, many pages
+    assert _pattn_waves(2048, 1, 40, 16384, 128) == 4         # eight lanes share their pages
+    assert _pattn_waves(256, 1, 80, 1024, 128) == 8           # 256 tokens after 1024
+    assert _pattn_waves(2048, 1, 10, 0, 128) == 4             # more than 16 rows per lane
+    assert _pattn_waves(8, 60, 512, 8, 128) == 4              # keys over several workgroups
