@@ -8,7 +8,7 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
-SIZES = [0, 1, 15, 16, 17, 255, 257, 4095, 4096, 4097, 65535, 65536, 65537, 300001]
+SIZES = [0, 1, 15, 16, 17, 255, 257, 4095, 4096, 4097, 16383, 16384, 16385, 40000, 65535, 65536, 65537, 300001]
 
 
 def _bytes(n, seed):
