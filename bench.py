@@ -184,8 +184,6 @@ def _rope():
               out_ptr=np.zeros_like(x))
     return dict(src=configs.rope(H, S, D, 4, 2, 256), fn="rope_fwd_kernel", kw=kw, cores=8,
                 bytes=2 * H * S * D * 2 + 2 * S * (D // 2) * 2, flops=6 * H * S * D // 2, bound="hbm",
-                # two launches, one per half of the rotated rows: each does half of the work
-                dominant_share=0.5,
                 dtype="f16 (products, sum and difference each rounded to f16)",
                 workload=f"rope H={H} S={S} D={D} f16 grid=4x2 seq tile 256 (the reference's "
                          f"latency/rope_fwd_4x2 form)")
@@ -222,8 +220,8 @@ CONFIGS = {"vector_add": _vector_add, "vector_add_4096": _vector_add_4096, "copy
 
 
 # kernels that make up each kind of launch (the HIP kernel names)
-_LAUNCH_KERNELS = {"mm": ("mm_mfma", "mm_generic"), "attn": ("attn_kernel", "attn_pp", "attn_v16"), "rmw": ("rmw_",),
-                   "prog": ("prog_",), "pattn": ("pattn_kernel",)}
+_LAUNCH_KERNELS = {"mm": ("mm_mfma", "mm_plane", "mm_generic"), "attn": ("attn_kernel", "attn_pp", "attn_tile", "attn_v16"),
+                   "rmw": ("rmw_",), "prog": ("prog_",), "pattn": ("pattn_",)}
 
 
 def _traffic(config, kind):
@@ -419,13 +417,13 @@ def measure(name, steps, warmup, with_cpu):
     dom_ms = float(durs[dom]) if n and durs.any() else ms
     kind = plan.launches[dom][0] if n else None
     # the dominant launch processes all of the workload's algorithmic units
-    # (all bytes moved / all flops), or the share the config states
+    # (all bytes moved / all flops)
     if cfg["bound"] == "hbm":
         units, unit, peak, scale = cfg["bytes"], "GB/s", HBM_PEAK_GBS, 1e9
     else:
         units, unit, peak, scale = cfg["flops"], "TFLOP/s", MFMA_F16_TFLOPS, 1e12
     value = units / (ms * 1e-3) / scale
-    achieved = units * cfg.get("dominant_share", 1.0) / (dom_ms * 1e-3) / scale
+    achieved = units / (dom_ms * 1e-3) / scale
     # host <-> device copies of all array arguments, and one whole call
     t0 = time.perf_counter()
     prep.reset_inputs()
@@ -610,8 +608,8 @@ def collect_traffic(root):
                         vals.setdefault(name, []).append(float(row["Counter_Value"]))
         return {k: float(np.median(v)) for k, v in vals.items()}, {k: len(v) for k, v in vals.items()}
 
-    (cf, _), (cw, _) = per_kernel("copy", "FETCH_SIZE"), per_kernel("copy", "WRITE_SIZE")
-    ck = max(cf, key=cf.get)
+    (cf, nc), (cw, _) = per_kernel("copy", "FETCH_SIZE"), per_kernel("copy", "WRITE_SIZE")
+    ck = max(cf, key=lambda k: (nc[k], cf[k]))      # not the row sum that empties the caches between cold replays
     each = 256 * 1024 * 1024
     fscale, wscale = each / (cf[ck] * 1024), each / (cw[ck] * 1024)
     out = {"calibration": {"kernel": ck, "bytes_each_way": each, "fetch_kib": cf[ck], "write_kib": cw[ck],
