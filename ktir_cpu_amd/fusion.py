@@ -851,7 +851,7 @@ def _attention_loop(ex, op, lb, st, trips, inits):
         lo = rel + np.minimum(0, tm1 * step)
         hi = rel + np.maximum(0, tm1 * step) + (N - 1) * row + D - 1
         if np.any(run & ((lo < 0) | (hi >= alloc.n_elems) | (rel % 8 != 0))) or row % 8 or step % 8 or row < D \
-                or row >= 1 << 23:
+                or row >= (1 << 25 if M == N == D == 128 else 1 << 23):       # 32-bit byte offsets in a wavefront's rows
             return None
         tiles[key] = (alloc, rel, row, step)
     q_off = q_leaf.lane.values(L)

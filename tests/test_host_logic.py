@@ -314,3 +314,24 @@ def test_paged_wavefronts_per_item():
     assert _pattn_waves(256, 1, 80, 1024, 128) == 8           # 256 tokens after 1024
     assert _pattn_waves(2048, 1, 10, 0, 128) == 4             # more than 16 rows per lane
     assert _pattn_waves(8, 60, 512, 8, 128) == 4              # keys over several workgroups
+
+
+@pytest.mark.parametrize("tile,row,fused", [(128, 1 << 23, True), (128, 1 << 25, False), (64, 1 << 22, True), (64, 1 << 23, False)])
+def test_attention_rows_far_apart(tile, row, fused, monkeypatch):
+    """K rows up to the distance whose 32-bit byte offsets the kernel of the
+    tile's shape holds run in one launch (32 rows of a wavefront for 128^3)."""
+    from ktir_cpu_amd import runtime as rt
+    from ktir_cpu_amd.interpreter import KTIRInterpreter
+    from tests import _cases
+    from tests.test_attention_output_reuse import _NoDevice
+    lib = _NoDevice()
+    monkeypatch.setattr(rt, "lib", lambda: lib)
+    src, fn, kw = _cases.flash_attention(B=1, H=1, S=128, D=tile, blk=tile, dt="f16", causal=False)
+    i = src.index("%k_view =")
+    old = f"strides: [{128 * tile}, {128 * tile}, {tile}, 1]"
+    assert old in src[i:]
+    src = src[:i] + src[i:].replace(old, f"strides: [{128 * row}, {128 * row}, {row}, 1]", 1)
+    kw["k_ptr"] = np.zeros((1, 1, 128, row), np.float16)       # never touched
+    it = KTIRInterpreter()
+    it.load(src)
+    assert ("attn" in it.prepare(fn, **kw).plan.counts()) == fused
