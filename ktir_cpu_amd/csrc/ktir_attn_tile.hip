@@ -26,10 +26,9 @@
 // instructions bound it (the split of P takes as many as the exponentials, the
 // test for small P 3 to 4 % of the time).  Where no CU has a second workgroup,
 // the key tiles go to two groups of four wavefronts, whose states meet in LDS at
-// the end.  Full attention
-// of 2048 x 64, f16, 64 x 64 tiles: 16 heads 33.9 us (510 TFLOP/s), 40 with one
-// group, and 43.4 ms for the loop's about 450 launches; 32 heads (two workgroups
-// per CU) 68.7 us.
+// the end.  Full attention of 2048 x 64, f16, 64 x 64 tiles: 16 heads 37 us
+// (465 TFLOP/s; 34 us, and 40 with one group, while f16 lost small P), and 43.4 ms
+// for the loop's about 450 launches; 32 heads (two workgroups per CU) 68 us.
 #include <type_traits>
 
 #include "ktir_attn_common.h"
