@@ -64,17 +64,15 @@ __device__ __forceinline__ uint32_t finite2(uint32_t w) {
 // loop holds P in f32; here it enters as terms of a 16-bit type whose products
 // are exact and are summed in f32.
 //   bf16: the terms have f32's exponents; three of them hold P's 24 bits.
-//   f16: P lies in (0, 2^P_LAG], relative to a base that the row max passes by
-//   at most P_LAG.  Times P_SCALE = 2^13 (2^2.9 2^13 < 65504; O carries the
+//   f16: P lies in (0, e^P_LAG], relative to a base that the row max passes by
+//   at most P_LAG.  Times P_SCALE = 2^13 (e^2 2^13 < 65504; O carries the
 //   factor to the end) two f16 terms hold 23 bits of a P from P_SMALL on.  Below
 //   that the second term is subnormal, so a step with a smaller P, other than
 //   0, also adds what the two terms leave of each P, as three bf16 terms, times
 //   V as two (exact: f16 has 11 bits, bf16 8).  Without it a key of weight
 //   e^-16 counts nothing where the heaviest one has V = 0.
-// The base is a power of two, 2^b: P = 2^(S log2 e - b) rounds once, scores far
-// from 0 included, and a move of the base is 2^(b - b').
 template <bool BF16>
-constexpr float P_LAG = BF16 ? 11.5f : 2.9f;
+constexpr float P_LAG = BF16 ? 8.f : 2.f;
 template <bool BF16>
 constexpr float P_SCALE = BF16 ? 1.f : 8192.f;
 constexpr float P_SMALL = 0x1p-15f;
@@ -214,9 +212,6 @@ __device__ __forceinline__ float mask_ninf(float x, bool kill) { return kill ? -
 
 // e^x as 2^(x log2 e) on the hardware exp2 (v_exp_f32)
 __device__ __forceinline__ float exp_f(float x) { return __builtin_amdgcn_exp2f(__fmul_rn(x, LOG2E)); }
-
-// 2^x on the hardware (v_exp_f32)
-__device__ __forceinline__ float exp2_f(float x) { return __builtin_amdgcn_exp2f(x); }
 
 // ds_read_b64_tr_b16: in each 16-lane group, member t receives element t % 4
 // of the 4-element chunks addressed by members 4s + t / 4, s = 0..3

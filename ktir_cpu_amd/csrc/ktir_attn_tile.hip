@@ -10,13 +10,19 @@
 //   S^T = K Q^T     A = K rows from LDS, B = Q^T in registers, so a query row's
 //                   scores lie in lanes l and l ^ 32;
 //   softmax         row max and sum in the lane and one exchange, P, l and O kept
-//                   relative to a base 2^b that moves when e^m passes it by P_LAG;
+//                   relative to a base 2^b that moves when e^m passes it by e^P_LAG;
 //   O^T += V^T P^T  V^T by transposing LDS reads, the keys in the order in which
 //                   a lane's own scores are its P fragment.
 // P, f32 in the op-by-op loop, enters P V as three bf16 terms (24 bits) or, in
 // f16, as two terms (23 bits) and, in a step with a P below 2^-15, the rest
 // of them too (ktir_attn_common.h): results from float64 by no more than one
 // rounding of their type and f32's of the exponentials, as the loop's are.
+// P = 2^(S log2 e - b) rounds once, for scores far from 0 too, as 2^b is the base
+// itself.  Beyond 2^19 the rounding of b would pass 1, so b ends at -2^20 below (the
+// P of a row that a mask of -1e9 or of the type's lowest value has filled so far are
+// 0, as any later score makes them), and a workgroup with a row that ends up out there,
+// or with a NaN in its result, runs its loop again in the general form: e^(S - mr)
+// with a base mr, and V's infinities kept from the later terms of P.
 //
 // K and V tiles are double-buffered in LDS: tile j + 1 streams in (buffer_load
 // ... lds, no registers) while tile j is computed, one barrier per tile.  A
@@ -51,6 +57,10 @@ __device__ __forceinline__ void att_stage(const uint16_t* src, int64_t row_strid
                                              16, (int)((r * row_stride + 8 * x) * 2), (int)(i * RB * row_stride * 2), 0, 0);
   }
 }
+
+// the lowest b, and whether a final row maximum asks for the general form
+constexpr float AT_LOW = -0x1p20f;
+__device__ __forceinline__ bool at_far(float m) { return fabsf(m) > 0x1p19f && fabsf(m) < __builtin_inff(); }
 
 // The position mask keeps score (row, key) iff ((lo <= kpos - qpos <= hi) != inv).
 // G groups of four wavefronts take every G-th key tile of the same lanes, each
@@ -96,7 +106,7 @@ __global__ __launch_bounds__(256 * G, G == 1 && N * D == 64 * 64 ? 3 : 2) void a
   const float c1 = __fmul_rn(d.scale, LOG2E);
   const f32x16_t z16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   f32x16_t o[DT];                                   // O^T tiles: d = 32 dt + 8 g + 4 h + t, row r32
-  float m, b, lsum;                                 // b: the base 2^b of P, l and O (at most 2^P_LAG below e^m)
+  float m, b, lsum;                                 // b: the base's exponent (general form: mr)
   const int k_off = r32 * D, k_x = kv_swz<D>(r32 & 15);
   // V^T fragment: member tj of 16-lane group tg addresses key 4 (tg / 2) + tj / 4
   // (+ 8) of the 16-key step, columns 16 (tg % 2) + 4 (tj % 4) of a 32-column tile
@@ -105,9 +115,10 @@ __global__ __launch_bounds__(256 * G, G == 1 && N * D == 64 * 64 ? 3 : 2) void a
   const int v_c = 2 * (tg & 1) + ((tj >> 1) & 1), v_in = 4 * (tj & 1);
   const int v_b0 = v_row0 * D + v_in, v_x0 = v_c ^ kv_swz<D>(v_row0), v_x1 = v_c ^ kv_swz<D>(v_row0 + 8);
 
-  auto step = [&](auto inf_v, int j, const uint16_t* Kc, const uint16_t* Vc, uint16_t* Kn,
+  // GEN: the general form
+  auto step = [&](auto gen, int j, const uint16_t* Kc, const uint16_t* Vc, uint16_t* Kn,
                   uint16_t* Vn) __attribute__((always_inline)) {
-    constexpr bool INF_V = decltype(inf_v)::value;
+    constexpr bool GEN = decltype(gen)::value;
     if (j + G < Tmax) {
       att_stage<N, D>(K + (int64_t)(j + G) * d.k_step, d.k_row, Kn, w, l);
       att_stage<N, D>(V + (int64_t)(j + G) * d.v_step, d.v_row, Vn, w, l);
@@ -155,10 +166,11 @@ __global__ __launch_bounds__(256 * G, G == 1 && N * D == 64 * 64 ? 3 : 2) void a
       for (int kt = 1; kt < KT; ++kt) xm = fmax_nan(xm, x[kt]);
       xm = pair_max(xm);
       const float mn = fmax_nan(m, fast ? __fmul_rn(d.scale, xm) : xm);
-      const float bn = __fmul_rn(mn, LOG2E);
-      const bool up = bn > __fadd_rn(b, P_LAG<BF16>);
+      // -inf (tile 0 masked whole) stays: P is then the loop's NaN
+      const float bn = GEN ? mn : fmax_nan(__fmul_rn(mn, LOG2E), mn == -__builtin_inff() ? mn : AT_LOW);
+      const bool up = bn > __fadd_rn(b, GEN ? P_LAG<BF16> : P_LAG<BF16> * LOG2E);
       if (__any(up)) {
-        const float al = up ? exp2_f(__fsub_rn(b, bn)) : 1.f;
+        const float db = __fsub_rn(b, bn), al = up ? (GEN ? exp_f(db) : __builtin_amdgcn_exp2f(db)) : 1.f;
 #pragma unroll
         for (int t = 0; t < DT; ++t)
 #pragma unroll
@@ -169,20 +181,22 @@ __global__ __launch_bounds__(256 * G, G == 1 && N * D == 64 * 64 ? 3 : 2) void a
       // a group without tile 0 whose scores have all been -inf: P is 0 against
       // any base (with tile 0 it is the loop's exp(-inf - (-inf)), NaN)
       const float pb = G > 1 && grp && mn == -__builtin_inff() ? 0.f : b;
-      if (fast) {
+      if constexpr (GEN) {
+        const float to_s = fast ? d.scale : 1.f;
 #pragma unroll
         for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
-          for (int i = 0; i < 16; ++i) sc[kt][i] = exp2_f(__builtin_fmaf(sc[kt][i], c1, -pb));
+          for (int i = 0; i < 16; ++i) sc[kt][i] = exp_f(__builtin_fmaf(sc[kt][i], to_s, -pb));
       } else {
+        const float to_2 = fast ? c1 : LOG2E;
 #pragma unroll
         for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
-          for (int i = 0; i < 16; ++i) sc[kt][i] = exp2_f(__builtin_fmaf(sc[kt][i], LOG2E, -pb));
+          for (int i = 0; i < 16; ++i) sc[kt][i] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[kt][i], to_2, -pb));
       }
       // whether a P of this tile is too small for two f16 terms
       bool small = false;
-      if constexpr (!BF16 && !INF_V) {
+      if constexpr (!BF16 && !GEN) {
         float least = 1.f;
         if (fast) {
 #pragma unroll
@@ -214,7 +228,7 @@ __global__ __launch_bounds__(256 * G, G == 1 && N * D == 64 * 64 ? 3 : 2) void a
       lsum = __fadd_rn(lsum, pair_sum(__fadd_rn(__fadd_rn(a0, a1), __fadd_rn(a2, a3))));
       m = mn;
       // P V: by the terms of the operand type, by the rest they leave (f16) or by
-      // bf16 terms of the whole P (f16, infinities in V)
+      // bf16 terms of the whole P (f16, general form)
       enum { TERMS, REST, WHOLE };
       auto pv = [&](auto how) __attribute__((always_inline)) {
         constexpr int HOW = decltype(how)::value;
@@ -242,15 +256,15 @@ __global__ __launch_bounds__(256 * G, G == 1 && N * D == 64 * 64 ? 3 : 2) void a
             const uint2 hi = ds_tr16(vt + v_b0 + 8 * D + 8 * ((4 * dt) ^ v_x1));
             const uint4 a = make_uint4(lo.x, lo.y, hi.x, hi.y);
             if constexpr (HOW == TERMS) {
-              o[dt] = pv_mfma<BF16, PARTS, INF_V>(a, t0, t1, o[dt]);
+              o[dt] = pv_mfma<BF16, PARTS, GEN>(a, t0, t1, o[dt]);
             } else {
-              o[dt] = pv_mfma_bf<INF_V>(a, tb, o[dt]);
+              o[dt] = pv_mfma_bf<GEN>(a, tb, o[dt]);
               __builtin_amdgcn_sched_barrier(0);   // rare: must not set the register count
             }
           }
         }
       };
-      if constexpr (!BF16 && INF_V) {
+      if constexpr (!BF16 && GEN) {
         pv(std::integral_constant<int, WHOLE>{});
       } else {
         pv(std::integral_constant<int, TERMS>{});
@@ -260,7 +274,7 @@ __global__ __launch_bounds__(256 * G, G == 1 && N * D == 64 * 64 ? 3 : 2) void a
     __builtin_amdgcn_s_waitcnt(0);                  // this wavefront's part of the next tile has landed
     __syncthreads();                                // every wavefront: done with tile j, the next one whole
   };
-  auto loop = [&](auto inf_v) __attribute__((always_inline)) {
+  auto loop = [&](auto gen) __attribute__((always_inline)) {
 #pragma unroll
     for (int t = 0; t < DT; ++t) o[t] = z16;
     m = b = -__builtin_inff();
@@ -273,20 +287,23 @@ __global__ __launch_bounds__(256 * G, G == 1 && N * D == 64 * 64 ? 3 : 2) void a
     __syncthreads();
     // as many steps in every group (one past the end computes nothing)
     for (int j = 0; j < Tmax; j += 2 * G) {
-      step(inf_v, j + grp, K0s, V0s, K1s, V1s);
-      if (j + G < Tmax) step(inf_v, j + G + grp, K1s, V1s, K0s, V0s);
+      step(gen, j + grp, K0s, V0s, K1s, V1s);
+      if (j + G < Tmax) step(gen, j + G + grp, K1s, V1s, K0s, V0s);
     }
   };
   loop(std::false_type{});
   // An infinite V times the terms of P after the first (0, or of the other
-  // sign) is NaN where P V is infinite.  So a NaN anywhere in the workgroup's
-  // result runs the loop again with only the first term meeting such values.
-  bool nan = false;
+  // sign) is NaN where P V is infinite, so a NaN anywhere in the workgroup's
+  // result asks for the general form too.
+  bool again = at_far(m);
 #pragma unroll
   for (int t = 0; t < DT; ++t)
 #pragma unroll
-    for (int i = 0; i < 16; ++i) nan |= o[t][i] != o[t][i];
-  if (__syncthreads_or(nan)) loop(std::true_type{});
+    for (int i = 0; i < 16; ++i) again |= o[t][i] != o[t][i];
+  const bool gen = __syncthreads_or(again);
+  if (gen) loop(std::true_type{});
+  // what brings l and O to e^m
+  float fin = gen ? exp_f(__fsub_rn(b, m)) : __builtin_amdgcn_exp2f(__builtin_fmaf(-m, LOG2E, b));
   if constexpr (G == 2) {
     // group 1's state, through the tiles (read by now: the barrier above), to
     // the thread of group 0 with the same row and columns
@@ -301,14 +318,15 @@ __global__ __launch_bounds__(256 * G, G == 1 && N * D == 64 * 64 ? 3 : 2) void a
         for (int g = 0; g < 4; ++g)
           *ex(4 * t + g) = make_float4(o[t][4 * g], o[t][4 * g + 1], o[t][4 * g + 2], o[t][4 * g + 3]);
       exs[0] = m;
-      exs[256] = b;
+      exs[256] = fin;
       exs[512] = lsum;
     }
     __syncthreads();
     if (grp == 1) return;
     if (T > 0) {
-      const float m1 = exs[0], mm = fmax_nan(m, m1), bm = __fmul_rn(mm, LOG2E);
-      const float w0 = exp2_f(__fsub_rn(b, bm)), w1 = m1 == -__builtin_inff() ? 0.f : exp2_f(__fsub_rn(exs[256], bm));
+      const float m1 = exs[0], mm = fmax_nan(m, m1);
+      const float w0 = __fmul_rn(fin, exp_f(__fsub_rn(m, mm)));
+      const float w1 = m1 == -__builtin_inff() ? 0.f : __fmul_rn(exs[256], exp_f(__fsub_rn(m1, mm)));
 #pragma unroll
       for (int t = 0; t < DT; ++t)
 #pragma unroll
@@ -321,13 +339,12 @@ __global__ __launch_bounds__(256 * G, G == 1 && N * D == 64 * 64 ? 3 : 2) void a
         }
       lsum = __fadd_rn(__fmul_rn(lsum, w0), __fmul_rn(exs[512], w1));
       m = mm;
-      b = bm;
+      fin = 1.f;
     }
   }
   if (lane < 0) return;
   if (T > 0) {
-    // bring l and O from 2^b to e^m, and O from P's scale
-    const float fin = exp2_f(__builtin_fmaf(-m, LOG2E, b));
+    // l and O to e^m, and O from P's scale
     if (!BF16 || !__all(fin == 1.f)) {
       const float f = __fmul_rn(fin, 1.f / P_SCALE<BF16>);
 #pragma unroll

@@ -12,7 +12,7 @@
 // nothing until the end, run without barriers, and a single query row of a
 // decode step keeps the whole chip busy.  Per pair, as in ktir_attn_tile.hip:
 //   S^T = K Q^T (32 x 32 x 16 MFMA), masked and scaled in f32,
-//   m, l and O of the wavefront's keys (online softmax, O relative to a base 2^b),
+//   m, l and O of the wavefront's keys (online softmax, O relative to mr <= m),
 //   O^T += V^T P^T.
 // P enters P V as PARTS terms of the operand type: one f16 / two bf16 terms for
 // lanes of at most 16 rows (as the one-wavefront kernel), one more for others,
@@ -290,7 +290,7 @@ __global__ __launch_bounds__(64 * W, 2) void pattn_split(const ktir_pattn_t d, i
   };
   const f32x16_t z16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   f32x16_t o[DT];                              // O^T tiles: column 32 dt + 8 g + 4 h + t of row r32
-  float m, b, lsum;                            // b: the base 2^b of P, l and O (at most 2^P_LAG below e^m)
+  float m, mr, lsum;
   const int k_off = r32 * D, k_x = kv_swz<D>(r32 & 15);
   const int tg = l >> 4, tj = l & 15;
   const int v_row0 = 4 * (tg >> 1) + (tj >> 2);
@@ -345,22 +345,24 @@ __global__ __launch_bounds__(64 * W, 2) void pattn_split(const ktir_pattn_t d, i
     bool poison = false;
     if (j0 == 0) poison = pair_max(x0) == -__builtin_inff();
     const float mn = fmax_nan(m, pair_max(fmax_nan(x0, x1)));
-    const float bn = __fmul_rn(mn, LOG2E);
-    const bool up = bn > __fadd_rn(b, P_LAG<BF16>);
+    const bool up = mn > __fadd_rn(mr, P_LAG<BF16>);
     if (__any(up)) {
-      const float al = up ? exp2_f(__fsub_rn(b, bn)) : 1.f;
+      const float al = up ? exp_f(__fsub_rn(mr, mn)) : 1.f;
 #pragma unroll
       for (int t = 0; t < DT; ++t)
 #pragma unroll
         for (int i = 0; i < 16; ++i) o[t][i] = __fmul_rn(o[t][i], al);
       lsum = __fmul_rn(lsum, al);
-      b = up ? bn : b;
+      mr = up ? mn : mr;
     }
     m = mn;
-    // all keys so far masked: P = 0 against any base
-    const float pb = mn == -__builtin_inff() ? 0.f : (mn != mn ? mn : b);
+    // all keys so far masked: P = 0 against any base.  The exponent is (S - mr)
+    // log2 e, not S log2 e - mr log2 e: the rounding of the second product would
+    // stand between wavefronts of other bases, and passes 1 where a mask's fill
+    // (-1e9, the type's lowest value) is the maximum so far.
+    const float mb = mn == -__builtin_inff() ? 0.f : (mn != mn ? mn : mr);
 #pragma unroll
-    for (int i = 0; i < 16; ++i) x[i] = exp2_f(__builtin_fmaf(x[i], LOG2E, -pb));
+    for (int i = 0; i < 16; ++i) x[i] = exp_f(__fsub_rn(x[i], mb));
     // whether a P is too small for two f16 terms
     bool small = false;
     if constexpr (!BF16 && PARTS == 2 && !INF_V) small = __any(least_positive<16>(x) < P_SMALL);
@@ -444,7 +446,7 @@ __global__ __launch_bounds__(64 * W, 2) void pattn_split(const ktir_pattn_t d, i
     constexpr bool INF_V = decltype(inf_v)::value;
 #pragma unroll
     for (int t = 0; t < DT; ++t) o[t] = z16;
-    m = b = -__builtin_inff();
+    m = mr = -__builtin_inff();
     lsum = 0.f;
     for (int c0 = 0; c0 < mine; c0 += 32) {
       if (INF_V || c0) table = entries(c0);
@@ -485,9 +487,9 @@ __global__ __launch_bounds__(64 * W, 2) void pattn_split(const ktir_pattn_t d, i
     if (__any(nan)) pages(std::true_type{});
   }
   if (bad) *err = 1;
-  // bring l and O from 2^b to e^m, and O from P's scale
+  // bring l and O from mr to m, and O from P's scale
   if (mine > 0 && m != -__builtin_inff()) {
-    const float fin = exp2_f(__builtin_fmaf(-m, LOG2E, b)), f = __fmul_rn(fin, 1.f / P_SCALE<BF16>);
+    const float fin = exp_f(__fsub_rn(mr, m)), f = __fmul_rn(fin, 1.f / P_SCALE<BF16>);
     lsum = __fmul_rn(lsum, fin);
 #pragma unroll
     for (int t = 0; t < DT; ++t)

@@ -134,6 +134,50 @@ def test_tiles_heavy_key_without_value(M, N, D, at, gap, dt, out_dt):
     _near(_f64(prep.outputs()["o_ptr"]), want, dt if out_dt == "own" else "f32", spread, _exp_err(gap))
 
 
+# finite fills of a mask: the score of a masked key, and the running maximum of a
+# row while all its keys are masked
+FILLS = {"-1.0e4": -1e4, "-1.0e6": -1e6, "-1.0e7": -1e7, "-1.0e9": -1e9, "0xFF7FFFFF": float(np.finfo(np.float32).min)}
+
+
+def _filled(src, fill):
+    """`src` with `fill` for masked scores, and keys kept from beyond the row's
+    position on: rows whose first tiles are masked whole, and a last row that
+    is masked throughout (whose weights are then all equal)."""
+    name = "%mv" if "%mv = arith.select" in src else "%r"
+    old = f"{name} = arith.select %keep, %sv, %neg_inf : f32"
+    head = "    %c1 = arith.constant 1 : index\n"
+    assert src.count(old) == src.count(head) == 1 and "arith.cmpi ule" in src
+    return src.replace(old, old.replace("%neg_inf", "%fill")).replace("arith.cmpi ule", "arith.cmpi ugt") \
+        .replace(head, head + f"    %fill = arith.constant {fill} : f32\n")
+
+
+def _filled_want(s, keep, v, fill):
+    s = np.where(keep, s, FILLS[fill])
+    p = np.exp(s - s.max(-1, keepdims=True))
+    p /= p.sum(-1, keepdims=True)
+    return p @ v, p @ np.abs(v)
+
+
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("fill", list(FILLS))
+@pytest.mark.parametrize("M,N,D", [(64, 64, 64), (128, 64, 128), (128, 128, 64)])
+@pytest.mark.parametrize("H", [2, 140])
+def test_tiles_of_finite_fills(M, N, D, fill, dt, H):
+    S = 256
+    rng = np.random.default_rng(M + N)
+    q, k, v = (_bits(rng.standard_normal((1, H, S, D)), dt) for _ in range(3))
+    src = _filled(configs.flash_attention(1, H, S, D, M, dt, True, N), fill)
+    old = f"arith.divui %q_end, %KBLK : index" if M != N else "%n_kv = arith.addi %qb, %c1 : index"
+    assert src.count(old) == 1
+    src = src.replace(old, old[:old.index("arith")] + f"arith.constant {S // N} : index")
+    prep, d = _prepare(src, "flash_attention", dict(q_ptr=q, k_ptr=k, v_ptr=v, o_ptr=np.zeros_like(q), scale=D ** -0.5))
+    assert (d.M, d.N, d.D) == (M, N, D)
+    s = np.einsum("bhid,bhjd->bhij", _f64(q), _f64(k)) * D ** -0.5
+    pos = np.arange(S)
+    want, spread = _filled_want(s, pos[None, :] > pos[:, None], _f64(v), fill)
+    _near(_f64(prep.outputs()["o_ptr"]), want, dt, spread)
+
+
 def _far_scores(S, D, steps):
     """q and k of exact scores near 7600 that rise by 3/4 from step to step of `steps` keys."""
     q, k = np.zeros((S, D)), np.zeros((S, D))
@@ -240,3 +284,27 @@ def test_paged_row_sum_of_far_scores(rows, splits, monkeypatch):
     _, _, m, l = _paged_want(*args, "f16")
     np.testing.assert_array_equal(_device(d.m_out, 4 * t), m.reshape(-1))
     np.testing.assert_allclose(_device(d.l_out, 4 * t), l.reshape(-1), rtol=4e-6)
+
+
+@pytest.mark.parametrize("splits,waves", [(1, 4), (3, 4), (1, 1)])
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("fill", list(FILLS))
+@pytest.mark.parametrize("rows", list(ROWS))
+def test_paged_finite_fills(rows, fill, dt, splits, waves, monkeypatch):
+    """Tokens near the end of the keys: most pages of a row masked whole, the
+    last token's all."""
+    from ktir_cpu_amd import fusion
+    monkeypatch.setattr(fusion, "_pattn_splits", lambda *a: splits)
+    monkeypatch.setattr(fusion, "_pattn_waves", lambda *a: waves)
+    real = configs.paged_attention
+    monkeypatch.setattr(configs, "paged_attention", lambda **k: _filled(real(**k), fill))
+    t, S, head = ROWS[rows]["tokens"], 256, 64
+    rng = np.random.default_rng(rows)
+    q, k, v = (rng.standard_normal(x) for x in ((t, 4, head), (S, head), (S, head)))
+    prep, d = _paged(dt, t, ROWS[rows]["block_q"], head, q, k, v, S - t, head ** -0.5)
+    q, k, v = (_f64(_bits(x, dt)) for x in (q, k, v))
+    s = np.einsum("thd,jd->thj", q, k) * head ** -0.5
+    keep = np.arange(S)[None, None] > S - t + np.arange(t)[:, None, None]
+    want, spread = _filled_want(s, keep, v, fill)
+    # (f16 on one wavefront: P relative to a base that lags by up to 8)
+    _near(_f64(prep.outputs()["output_ptr"]), want, dt, spread, P_ERR[rows, dt] + 2.0 ** -21)
