@@ -64,9 +64,12 @@ __device__ __forceinline__ bool at_far(float m) { return fabsf(m) > 0x1p19f && f
 
 // The position mask keeps score (row, key) iff ((lo <= kpos - qpos <= hi) != inv).
 // G groups of four wavefronts take every G-th key tile of the same lanes, each
-// with tile buffers of its own.
+// with tile buffers of its own.  Two wavefronts per SIMD, also where 256
+// registers spill up to 17: one, with 512, takes 156 us for 122 (32 heads of 2048
+// x 128, tiles of 64) and 55 for 43 (64 heads of 1024 x 64, tiles of 128); three,
+// in 64 x 64 x 64 tiles, as long as two (77 us, 32 heads of 2048 x 64).
 template <bool BF16, int M, int N, int D, int G>
-__global__ __launch_bounds__(256 * G, G == 1 && N * D == 64 * 64 ? 3 : 2) void attn_tile(const ktir_attn_t d, int mlo, int mhi, int minv) {
+__global__ __launch_bounds__(256 * G, 2) void attn_tile(const ktir_attn_t d, int mlo, int mhi, int minv) {
   constexpr int KT = N / 32, DS = D / 16, DT = D / 32, PARTS = BF16 ? 3 : 2;
   __shared__ __align__(16) uint16_t K0a[G][N * D];  // K tiles of a group's even / odd steps
   __shared__ __align__(16) uint16_t K1a[G][N * D];
